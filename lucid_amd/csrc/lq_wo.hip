@@ -38,14 +38,10 @@
 #include <type_traits>
 
 #include "lq_internal.h"
+#include "lq_wo.h"
 
 namespace lq {
 namespace {
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 
 constexpr int WO_MAX_WAVES = 16;
 constexpr int WO_RING = 4;  // k-blocks in flight per wave
@@ -54,65 +50,6 @@ constexpr int WO_RING = 4;  // k-blocks in flight per wave
 // does not fit the 128 registers per lane of a 16-wave workgroup.
 constexpr int wo_max_waves(int S, bool xf32, bool grouped) {
     return (grouped && S * (xf32 ? 2 : 1) >= 4) ? 8 : WO_MAX_WAVES;
-}
-
-__device__ __forceinline__ h2 bits_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
-
-// k offset of half h within a lane's 8-element step for a code width.
-template <int BITS>
-__device__ __forceinline__ int korder(int h) {
-    return BITS == 4 ? ((h & 1) * 4 + (h >> 1)) : h;
-}
-
-// Four bytes -> four halves (byte - off) in byte order.
-__device__ __forceinline__ void bytes_to_h2(uint32_t w, _Float16 off, h2& a, h2& b) {
-    const uint32_t p0 = __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u);
-    const uint32_t p1 = __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u);
-    const h2 o = {off, off};
-    a = bits_h2(p0) - o;
-    b = bits_h2(p1) - o;
-}
-
-// One MFMA step's 8 codes as fp16: 8-bit from two words (signed codes are xor'ed with
-// 0x80 so the byte is c + 128), 4-bit from one word.
-template <int BITS, bool SIGNED>
-__device__ __forceinline__ h8 unpack_step(const uint32_t* w) {
-    if constexpr (BITS == 8) {
-        const uint32_t x0 = SIGNED ? (w[0] ^ 0x80808080u) : w[0];
-        const uint32_t x1 = SIGNED ? (w[1] ^ 0x80808080u) : w[1];
-        const _Float16 off = SIGNED ? (_Float16)1152.0f : (_Float16)1024.0f;
-        h2 a, b, c, d;
-        bytes_to_h2(x0, off, a, b);
-        bytes_to_h2(x1, off, c, d);
-        return h8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-    } else {
-        const h2 o = {(_Float16)1024.0f, (_Float16)1024.0f};
-        h2 r[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) r[s] = bits_h2(((w[0] >> (4 * s)) & 0x000F000Fu) | 0x64006400u) - o;
-        return h8{r[0].x, r[0].y, r[1].x, r[1].y, r[2].x, r[2].y, r[3].x, r[3].y};
-    }
-}
-
-__device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-// Epilogue of one output: the float32 product rounded to the activation's type (hmode, a
-// LQ_ROUND_* value), the layer bias rounded to that type and added there, then ReLU --
-// Lucid's quantized_matmul returning x's dtype and QuantizedLinearMLX's y + bias.to(y.dtype),
-// relu (lucid/nn/quantized/mlx_linear.py:215-222).  A half or bfloat16 sum of two such values
-// is exact in float32 before its rounding (24 >= 2 p + 2 bits), so the float32 add then round
-// equals the narrow add.  hmode 0 leaves the float32 result as it is.
-__device__ __forceinline__ float wo_finish(float v, bool has_bias, float b, int relu, int hmode) {
-    if (hmode == LQ_ROUND_NONE) {
-        if (has_bias) v = v + b;
-    } else {
-        v = round_result_to(v, hmode);
-        if (has_bias) v = round_result_to(v + round_to(b, hmode), hmode);
-    }
-    if (relu && v <= 0.0f) v = 0.0f;
-    return v;
 }
 
 // ------------------------------------------------------------------ kernel
@@ -1407,6 +1344,12 @@ bool launch_wv(WvArgs a, bool xf32, hipStream_t st) {
     return xf32 ? by_j(T2{}, F32{}) : by_j(T2{}, F16{});
 }
 
+// The same call for the tiled kernel (gs 0: per-channel).
+WoTileCall tile_call(const WoArgs& a, bool xf32, int bits, int gs) {
+    return WoTileCall{a.x, a.ldx, xf32, a.w, a.ldw_bytes, a.w_scale, a.w_zp, a.g_bias, a.bias, a.y, a.ldy,
+                      a.relu, a.hmode, a.M, a.N, a.K, bits, gs};
+}
+
 constexpr int64_t WO_MAX_DIM = (int64_t)1 << 30;
 constexpr size_t WO_MAX_LDS = 64 * 1024;
 
@@ -1421,7 +1364,7 @@ size_t lq_gemv_w8_workspace_size(int64_t M, int64_t N, int64_t K) {
     if (M <= 2 || K <= 0 || M >= WO_MAX_DIM || K >= WO_MAX_DIM || N >= WO_MAX_DIM) return 0;  // VALU path
     const size_t prep = wo_prep_bytes(M, wo_plan(K, 2, false, wo_max_waves(2, true, false)), 2);
     if (M <= SK_MAX_M) return std::max(prep, sk_ws_bytes(sk_plan(std::max<int64_t>(N, 1), K)));
-    return prep;
+    return std::max(prep, wo_tile_ws_bytes(M, N, K, 0));
 }
 
 int lq_gemv_w8(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d_W, int64_t ldw,
@@ -1463,6 +1406,13 @@ int lq_gemv_w8(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d_W, int
     if (sk_preferred(a) && sk_fits(a, xf32, 2, d_workspace, workspace_bytes)) {
         const int rc = launch_sk<8, true, 2, false>(a, xf32, st, d_workspace);
         return rc ? rc : launch_status("lq_gemv_w8");
+    }
+    if (M > SK_MAX_M) {
+        const WoTileCall t = tile_call(a, xf32, 8, 0);
+        if (wo_tile_takes(t)) {
+            wo_tile_launch(t, d_workspace, workspace_bytes, st);
+            return launch_status("lq_gemv_w8");
+        }
     }
     const bool vec = aligned16(d_W) && ldw % 16 == 0 && K % 16 == 0 && K >= 16 && aligned16(d_x) &&
                      ldx % (xf32 ? 4 : 8) == 0;
@@ -1519,7 +1469,7 @@ size_t lq_group_matmul_workspace_size(int64_t M, int64_t N, int64_t K, int group
     const int S = group_size / 32;
     const size_t prep = wo_prep_bytes(M, wo_plan(K, S, true, wo_max_waves(S, true, true)), S);
     if (M <= SK_MAX_M) return std::max(prep, sk_ws_bytes(sk_plan(std::max<int64_t>(N, 1), K)));
-    return prep;
+    return std::max(prep, wo_tile_ws_bytes(M, N, K, group_size));
 }
 
 int lq_group_matmul(const void* d_x, int x_dtype, int64_t ldx, const uint32_t* d_packed,
@@ -1604,6 +1554,13 @@ int lq_group_matmul(const void* d_x, int x_dtype, int64_t ldx, const uint32_t* d
                   : S == 2 ? launch_sk<4, false, 2, true>(a, xf32, st, d_workspace)
                            : launch_sk<4, false, 4, true>(a, xf32, st, d_workspace);
         return rc ? rc : launch_status("lq_group_matmul");
+    }
+    if (M > SK_MAX_M) {
+        const WoTileCall t = tile_call(a, xf32, bits, group_size);
+        if (wo_tile_takes(t)) {
+            wo_tile_launch(t, d_workspace, workspace_bytes, st);
+            return launch_status("lq_group_matmul");
+        }
     }
     const bool vec = aligned16(d_x) && ldx % (xf32 ? 4 : 8) == 0;
 #define LQ_GM(B, SS)                                                          \

@@ -1,0 +1,766 @@
+// lq_wo_tile.hip -- weight-only product y = x . w^T for many activation rows (prompts, batches):
+// a tiled GEMM on v_mfma_f32_16x16x32_f16 over the operands of lq_wo.hip.
+//
+// The GEMV kernels give a workgroup 16 weight rows and 16 activation rows and stream the weight
+// again for every 16 rows; the product ran at 60-70 TFLOP/s whatever its size.  Here a workgroup of
+// eight waves owns BM x 128 outputs (BM 128 in waves of 64 x 32, or 64 / 32 for few rows) and walks
+// K in stages of 64 through two LDS slots:
+//  * the activations are prepared once per call (wo_tile_prep_kernel): float32 values split into
+//    fp16 hi + lo terms after an exact power-of-two pre-scale, half values as they are, both in
+//    the order in which a stage's 16-byte pieces are read; with each block's sum.
+//  * the weight codes go to LDS as stored; each wave unpacks its fragments to fp16.
+//  * the group scales and biases, transposed by the same prepare launch, and the block sums ride
+//    along.  LDS holds everything in MFMA fragment order: reads and writes without bank conflicts.
+// Measured (float32 x, 8 bits, groups of 64, N = K = 4096; the GEMV kernels before): M = 64 34.5 ->
+// 23 us, M = 256 132 -> 40, M = 1024 504 -> 104 us = 330 TFLOP/s (two fp16 products each), M = 2048
+// 992 -> 205; half x, 4 bits, M = 1024 456 -> 88.  What bounds it now is the issue of instructions:
+// per wave and stage 32 MFMA (16 cycles each), 64 FMA of scales, 32 for unpacking, 26 LDS reads;
+// the matrix cores are busy about a third of the time.
+// Arithmetic per 64-wide block (32 for groups of 32): blk = sum c (hi + lo) in fp32, then
+// acc += s blk + b bsum.  A row's values are scaled by one 2^e for the whole row (its largest
+// value in [2^14, 2^15)); a block whose own maximum lies below 2^-3 of that scale gets an
+// exponent of its own and its sum is multiplied back (factor f, else 1), so every block keeps
+// ~22 significant bits of its own largest value.  2^-e is applied to the finished sum.
+// Few tiles: K is split into ranges over workgroups, their sums added in range order by
+// wo_tile_reduce_kernel.  Without a workspace the same sums are made by workgroups that split
+// the activations themselves and walk the ranges in order: the same bits, slower.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "lq_dma.h"
+#include "lq_internal.h"
+#include "lq_wo.h"
+
+namespace lq {
+namespace {
+
+struct WtArgs {
+    WoTileCall c;
+    int G;             // groups per weight row
+    int KB;            // stages of 64 k
+    int Mp;            // rows padded to 16
+    int tiles_m, tiles_n;
+    int rs;            // stages per K range
+    int ranges;        // K ranges
+    const char* xp;    // split activations: [Mp][KB][2 steps][T][4 quarters] of 8 halves
+    const float2* xm;  // [KB][NG][Mp]: block sum (scaled by 2^e), factor f
+    const vf4* xr;     // [Mp]: {2^-e, row sum (scaled), 1 if a block has its own exponent, 0}
+    const float2* sb;  // [G][Np]: group scale, group bias
+    int Np;            // columns padded to 128
+    float* part;       // range sums [ranges][tile][frag][thread] f4, or null
+};
+
+constexpr int WT_FLUSH = 8;  // stages per first-level sum
+
+// Blocks per stage: groups of 32 make two blocks of 32 k, everything else one of 64.
+template <int S>
+constexpr int wt_blocks() { return S == 2 ? 1 : 2; }
+
+// MFMA fragment position of the stage's octet o (8 consecutive k) of a row: step and lane quarter.
+template <int S>
+__device__ __forceinline__ void octet_pos(int o, int& step, int& q) {
+    if (S == 2) { step = o & 1; q = o >> 1; }   // a lane quarter holds 16 consecutive k
+    else { step = o >> 2; q = o & 3; }          // one block of 32 per step
+}
+
+__device__ __forceinline__ float row_exp2(float amax, int* e_out) {
+    int e = 0;
+    if (amax > 0.0f && amax <= 3.0e38f) e = min(max(14 - ilogbf(amax), -120), 120);
+    *e_out = e;
+    return ldexpf(1.0f, e);
+}
+
+// The 8 values of octet o of one row (0 past K or for rows past M).
+template <bool XF32>
+__device__ __forceinline__ void load_octet(const WoTileCall& c, int m, int k, bool vec, float (&v)[8]) {
+    const bool in = m < c.M;
+    if (vec && in && k + 8 <= c.K) {
+        if constexpr (XF32) {
+            const vf4* p = reinterpret_cast<const vf4*>(static_cast<const float*>(c.x) + (int64_t)m * c.ldx + k);
+            const vf4 a = p[0], b = p[1];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = a[i], v[4 + i] = b[i];
+        } else {
+            const h8 a = *reinterpret_cast<const h8*>(static_cast<const _Float16*>(c.x) + (int64_t)m * c.ldx + k);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = (float)a[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[i] = 0.0f;
+            if (in && k + i < c.K) {
+                if constexpr (XF32) v[i] = static_cast<const float*>(c.x)[(int64_t)m * c.ldx + k + i];
+                else v[i] = (float)static_cast<const _Float16*>(c.x)[(int64_t)m * c.ldx + k + i];
+            }
+        }
+    }
+}
+
+template <bool XF32>
+__device__ __forceinline__ bool x_vec(const WoTileCall& c) {
+    return (reinterpret_cast<uintptr_t>(c.x) & 15) == 0 && c.ldx % (XF32 ? 4 : 8) == 0;
+}
+
+__device__ __forceinline__ float octet_sum(const float (&v)[8]) {
+    float s = v[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) s += v[i];
+    return s;
+}
+
+__device__ __forceinline__ float octet_amax(const float (&v)[8]) {
+    float a = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a = fmaxf(a, fabsf(v[i]));
+    return a;
+}
+
+// hi / lo terms, block sum and factor of one octet; the 4 S lanes of a block's octets are
+// consecutive lanes of one wave.  up = 2^e of the row.
+template <int BITS, int S, int T>
+__device__ __forceinline__ void split_octet(const float (&v)[8], float up, int e, h8& hi, h8& lo, float& bsum, float& f) {
+    float bs = octet_sum(v), am = octet_amax(v);
+#pragma unroll
+    for (int off = 1; off < 4 * S; off <<= 1) {
+        bs += __shfl_xor(bs, off, 64);
+        am = fmaxf(am, __shfl_xor(am, off, 64));
+    }
+    f = 1.0f;
+    float u = up;
+    if (T == 2 && am > 0.0f && am * up < 0.125f) {
+        int e2;
+        u = row_exp2(am, &e2);
+        f = ldexpf(1.0f, e - e2);
+    }
+    bsum = T == 2 ? bs * up : bs;
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+        const float x = T == 2 ? v[korder<BITS>(h)] * u : v[korder<BITS>(h)];
+        hi[h] = (_Float16)x;
+        lo[h] = T == 2 ? (_Float16)(x - (float)hi[h]) : (_Float16)0.0f;
+    }
+}
+
+// Quarter w of one row's largest |x| and sum, by one wave: lane l owns octets 64 w + l, + 256, ...
+// The row's sum is its four quarters' sums added in order.
+template <bool XF32>
+__device__ __forceinline__ void row_scan(const WoTileCall& c, int m, int w, int lane, bool vec, float& amax, float& sum) {
+    amax = 0.0f;
+    sum = 0.0f;
+    const int no = (c.K + 7) / 8;
+    for (int o0 = 64 * w; o0 < no; o0 += 512) {  // two octets in flight
+        float v[2][8];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) load_octet<XF32>(c, m, (o0 + lane + 256 * u) * 8, vec, v[u]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            amax = fmaxf(amax, octet_amax(v[u]));
+            sum += octet_sum(v[u]);
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+        sum += __shfl_xor(sum, off, 64);
+    }
+}
+
+// The operands the tiled kernel wants contiguous.  The first Mp workgroups: one activation row
+// each, as [stage][step][term][lane quarter] 16-byte pieces, with its block sums and factors and
+// its scale.  The others (group-wise): 32 x 32 pieces of the group scales and biases transposed to
+// [group][column] pairs, rounded to the activation's type (a missing bias is 0).
+template <int BITS, int S, int T, bool GROUPED, int HM>
+__global__ __launch_bounds__(256) void wo_tile_prep_kernel(WtArgs a, char* xp, float2* xm, vf4* xr, float2* sb) {
+    constexpr int NG = wt_blocks<S>();
+    constexpr bool XF32 = T == 2;
+    __shared__ float2 sh[32][33];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (GROUPED && (int)blockIdx.x >= a.Mp) {
+        const int id = blockIdx.x - a.Mp, gt = (a.G + 31) / 32;
+        const int g0 = id % gt * 32, n0 = id / gt * 32, x = tid & 31, y = tid >> 5;
+#pragma unroll
+        for (int r = y; r < 32; r += 8) {
+            const int n = n0 + r, g = g0 + x;
+            const bool in = n < a.c.N && g < a.G;
+            const int64_t at = (int64_t)n * a.G + g;
+            sh[r][x] = make_float2(in ? round_to(a.c.w_scale[at], HM) : 0.0f,
+                                   in && a.c.g_bias ? round_to(a.c.g_bias[at], HM) : 0.0f);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = y; r < 32; r += 8)
+            if (g0 + r < a.G) sb[(int64_t)(g0 + r) * a.Np + n0 + x] = sh[x][r];
+        return;
+    }
+    const int m = blockIdx.x;
+    const bool vec = x_vec<XF32>(a.c);
+    float amax, sum, up = 1.0f;
+    int e = 0;
+    row_scan<XF32>(a.c, m, wave, lane, vec, amax, sum);
+    if (lane == 0) sh[0][wave] = make_float2(amax, sum);
+    __syncthreads();
+    amax = fmaxf(fmaxf(sh[0][0].x, sh[0][1].x), fmaxf(sh[0][2].x, sh[0][3].x));
+    sum = ((sh[0][0].y + sh[0][1].y) + sh[0][2].y) + sh[0][3].y;
+    if (T == 2) up = row_exp2(amax, &e);
+    bool own = false;
+    for (int og = tid; og < a.KB * 8; og += 256) {
+        const int kb = og >> 3, o = og & 7;
+        float v[8];
+        load_octet<XF32>(a.c, m, og * 8, vec, v);
+        h8 hi, lo;
+        float bsum, f;
+        split_octet<BITS, S, T>(v, up, e, hi, lo, bsum, f);
+        int step, q;
+        octet_pos<S>(o, step, q);
+        h8* dst = reinterpret_cast<h8*>(xp) + ((int64_t)m * a.KB + kb) * 8 * T + step * T * 4 + q;
+        dst[0] = hi;
+        if (T == 2) dst[4] = lo;
+        if ((o & (4 * S - 1)) == 0) xm[((int64_t)kb * NG + o / (4 * S)) * a.Mp + m] = make_float2(bsum, f);
+        own |= f != 1.0f;
+    }
+    own = __syncthreads_or(own);
+    if (tid == 0) xr[m] = vf4{T == 2 ? ldexpf(1.0f, -e) : 1.0f, T == 2 ? sum * up : sum, own ? 1.0f : 0.0f, 0.0f};
+}
+
+// Tile of a workgroup: consecutive tiles (groups of eight tile rows, column by column) on one
+// XCD, so the 32 workgroups of an XCD share activation and weight panels in its L2.
+__device__ __forceinline__ void wt_tile_of(int id, int tm, int tn, int& m, int& n) {
+    const int total = tm * tn, q = total / 8, r = total % 8, x = id % 8;
+    const int p = x * q + min(x, r) + id / 8;
+    const int band = p / (8 * tn), m0 = band * 8, h = min(8, tm - m0), in = p - m0 * tn;
+    m = m0 + in % h;
+    n = in / h;
+}
+
+// The finished value of four consecutive columns of one row.
+template <bool GROUPED, bool XF32>
+__device__ __forceinline__ void wt_store(const WoTileCall& c, int m, int n, f4 v, float down, float sum) {
+    if (m >= c.M || n >= c.N) return;
+    const bool xf = XF32;
+    f4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int nn = min(n + i, c.N - 1);
+        float t = v[i];
+        if constexpr (!GROUPED) {
+            if (c.w_zp) t = t - c.w_zp[nn] * sum;
+            t = c.w_scale[nn] * (t * down);
+        } else {
+            t = t * down;
+        }
+        out[i] = wo_finish(t, c.bias != nullptr, c.bias ? c.bias[nn] : 0.0f, c.relu, c.hmode);
+    }
+    const int64_t at = (int64_t)m * c.ldy + n;
+    const bool whole = n + 4 <= c.N && (c.ldy & 3) == 0;
+    if (xf) {
+        float* y = static_cast<float*>(c.y) + at;
+        if (whole && (reinterpret_cast<uintptr_t>(c.y) & 15) == 0) {
+            *reinterpret_cast<f4*>(y) = out;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i < c.N) y[i] = out[i];
+        }
+    } else {
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        _Float16* y = static_cast<_Float16*>(c.y) + at;
+        const h4 o = {(_Float16)out[0], (_Float16)out[1], (_Float16)out[2], (_Float16)out[3]};
+        if (whole && (reinterpret_cast<uintptr_t>(c.y) & 7) == 0) {
+            *reinterpret_cast<h4*>(y) = o;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i < c.N) y[i] = o[i];
+        }
+    }
+}
+
+// HM: the group scales' rounding (LQ_ROUND_*), a constant so that none costs nothing.
+template <int BITS, int S, int T, bool GROUPED, int HM, int WM, int WN, int FM, int FN, bool INLINE>
+__global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
+    constexpr int W = WM * WN, BM = 16 * WM * FM, BN = 16 * WN * FN, NG = wt_blocks<S>();
+    constexpr int A_BYTES = BM * 128 * T, B_BYTES = BN * 8 * BITS;
+    constexpr int SB_BYTES = GROUPED ? NG * 2 * BN * 4 : 0, XF_BYTES = NG * 2 * BM * 4;
+    constexpr int STAGE = A_BYTES + B_BYTES + SB_BYTES + XF_BYTES;
+    constexpr int NST = INLINE ? 1 : 2, NT = 64 * W;
+    // 16-byte pieces per thread and stage, then pairs (scale, bias; block sum, factor)
+    constexpr int A_I = (A_BYTES + 16 * NT - 1) / (16 * NT), B_I = (B_BYTES + 16 * NT - 1) / (16 * NT);
+    constexpr int F_N = (SB_BYTES + XF_BYTES) / 8, F_I = (F_N + NT - 1) / NT;
+    constexpr int TOT_BYTES = BM * BN * 4;
+    static_assert(NST * STAGE + TOT_BYTES + (INLINE ? 12 * BM : 0) <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE + TOT_BYTES];
+    __shared__ float2 row_xr[INLINE ? BM : 1];
+    __shared__ int row_e[INLINE ? BM : 1];
+    const WoTileCall& c = a.c;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    int tm, tn;
+    wt_tile_of(blockIdx.x, a.tiles_m, a.tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
+
+    // ---- one stage: global memory -> registers -> LDS (LDS-DMA copies, with the scales gathered
+    // from their rows, took 178 us where this form took 157, at M = 1024, four waves)
+    struct Stage {
+        vu4 x[INLINE ? 1 : A_I];
+        vu4 w[B_I];
+        float2 f[F_I];
+    };
+    const int row_bytes = c.K * BITS / 8;
+    const uint8_t* b_row[B_I];
+    int b_chunk[B_I];
+#pragma unroll
+    for (int u = 0; u < B_I; ++u) {
+        // 8 bits: 1 KB is one 16-row tile of four 16-byte chunks; 4 bits: two tiles of two chunks
+        const int i = (tid + u * NT) % (B_BYTES / 16), l = i & 63;
+        const int r = BITS == 8 ? (i >> 6) * 16 + (l & 15) : (i >> 5) * 16 + (l & 15);
+        b_row[u] = c.w + (int64_t)min(n0 + r, c.N - 1) * c.ldw_bytes;
+        b_chunk[u] = (BITS == 8 ? l >> 4 : (l >> 4) & 1) * 16;
+    }
+    const char* a_ptr[INLINE ? 1 : A_I];
+    if constexpr (!INLINE) {
+#pragma unroll
+        for (int u = 0; u < A_I; ++u) {
+            // the piece's place in LDS (fragment order) -> its place in its row
+            const int i = (tid + u * NT) % (A_BYTES / 16), fr = i >> 6, l = i & 63;
+            const int m = min(m0 + fr / (2 * T) * 16 + (l & 15), a.Mp - 1);
+            a_ptr[u] = a.xp + (int64_t)m * a.KB * 128 * T + (fr % (2 * T) * 4 + (l >> 4)) * 16;
+        }
+    }
+    const float2* f_ptr[F_I];  // the first stage's pair and the stages' distance
+    int64_t f_step[F_I];
+    auto pair = [&](int u) __attribute__((always_inline)) { return min(tid + u * NT, F_N - 1); };
+#pragma unroll
+    for (int u = 0; u < F_I; ++u) {
+        const int i = pair(u);
+        if (i < SB_BYTES / 8) {  // [block][BN]
+            f_ptr[u] = a.sb + (int64_t)(i / BN) * a.Np + n0 + i % BN;
+            f_step[u] = 0;
+        } else {                 // [block][BM]
+            const int j = i - SB_BYTES / 8;
+            f_ptr[u] = a.xm + (int64_t)(j / BM) * a.Mp + min(m0 + j % BM, a.Mp - 1);
+            f_step[u] = (int64_t)NG * a.Mp;
+        }
+    }
+    auto load = [&](Stage& s, int kb) __attribute__((always_inline)) {
+        if constexpr (!INLINE) {
+#pragma unroll
+            for (int u = 0; u < A_I; ++u) s.x[u] = *reinterpret_cast<const vu4*>(a_ptr[u] + (int64_t)kb * 128 * T);
+        }
+#pragma unroll
+        for (int u = 0; u < B_I; ++u)
+            s.w[u] = *reinterpret_cast<const vu4*>(b_row[u] + min(kb * 8 * BITS + b_chunk[u], row_bytes - 16));
+#pragma unroll
+        for (int u = 0; u < F_I; ++u) {
+            const int i = pair(u);
+            if (GROUPED && i < SB_BYTES / 8) {
+                const int blk = i / BN, g = min((kb * 64 + blk * 32) / c.gs, a.G - 1);
+                if constexpr (INLINE) {
+                    const int64_t at = (int64_t)min(n0 + i % BN, c.N - 1) * a.G + g;
+                    s.f[u] = make_float2(round_to(c.w_scale[at], HM), c.g_bias ? round_to(c.g_bias[at], HM) : 0.0f);
+                } else {
+                    s.f[u] = f_ptr[u][(int64_t)(g - blk) * a.Np];
+                }
+            } else if constexpr (!INLINE) {
+                s.f[u] = f_ptr[u][kb * f_step[u]];
+            }
+        }
+    };
+    auto store = [&](const Stage& s, int slot) __attribute__((always_inline)) {
+        char* base = lds + slot * STAGE;
+        if constexpr (!INLINE) {
+#pragma unroll
+            for (int u = 0; u < A_I; ++u) *reinterpret_cast<vu4*>(base + (tid + u * NT) % (A_BYTES / 16) * 16) = s.x[u];
+        }
+#pragma unroll
+        for (int u = 0; u < B_I; ++u) *reinterpret_cast<vu4*>(base + A_BYTES + (tid + u * NT) % (B_BYTES / 16) * 16) = s.w[u];
+#pragma unroll
+        for (int u = 0; u < F_I; ++u) {
+            const int i = pair(u);
+            if (!INLINE || i < SB_BYTES / 8) reinterpret_cast<float2*>(base + A_BYTES + B_BYTES)[i] = s.f[u];
+        }
+    };
+
+    // ---- the activation rows' scales, where no prepared copy holds them
+    constexpr bool XF32 = T == 2;
+    const bool vec = INLINE && x_vec<XF32>(c);
+    if constexpr (INLINE) {
+        for (int r = wave; r < BM; r += W) {
+            float amax = 0.0f, sum = 0.0f, up = 1.0f;
+            int e = 0;
+            for (int w = 0; w < 4; ++w) {
+                float am, sm;
+                row_scan<XF32>(c, m0 + r, w, lane, vec, am, sm);
+                amax = fmaxf(amax, am);
+                sum = w ? sum + sm : sm;
+            }
+            if (T == 2) up = row_exp2(amax, &e);
+            if (lane == 0) {
+                row_xr[r] = make_float2(T == 2 ? ldexpf(1.0f, -e) : 1.0f, T == 2 ? sum * up : sum);
+                row_e[r] = e;
+            }
+        }
+        __syncthreads();
+    }
+    auto stage_inline = [&](int kb) __attribute__((always_inline)) {
+        char* base = lds;
+        for (int i = tid; i < BM * 8; i += 64 * W) {
+            const int r = i >> 3, o = i & 7;
+            float v[8];
+            load_octet<XF32>(c, m0 + r, kb * 64 + o * 8, vec, v);
+            h8 hi, lo;
+            float bsum, f;
+            split_octet<BITS, S, T>(v, T == 2 ? ldexpf(1.0f, row_e[r]) : 1.0f, row_e[r], hi, lo, bsum, f);
+            int step, qq;
+            octet_pos<S>(o, step, qq);
+            h8* dst = reinterpret_cast<h8*>(base) + ((r >> 4) * 2 + step) * T * 64 + qq * 16 + (r & 15);
+            dst[0] = hi;
+            if (T == 2) dst[64] = lo;
+            if ((o & (4 * S - 1)) == 0) {
+                reinterpret_cast<float2*>(base + A_BYTES + B_BYTES + SB_BYTES)[o / (4 * S) * BM + r] = make_float2(bsum, f);
+            }
+        }
+    };
+
+    // ---- one stage's products
+    // two levels of sums: acc over WT_FLUSH stages, tot over those, in LDS (a chain of all K / 64
+    // additions would lose about a bit against the GEMV kernels' sums per wave)
+    f4 acc[FM][FN];
+    f4* const tot = reinterpret_cast<f4*>(lds + NST * STAGE) + tid;  // [fragment][thread]
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < FM; ++m)
+#pragma unroll
+            for (int n = 0; n < FN; ++n) acc[m][n] = f4{0.f, 0.f, 0.f, 0.f};
+    };
+    // acc (stages t0 .. t) joins the range's sum; each thread touches its own slots only
+    auto flush = [&](bool first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < FM; ++m)
+#pragma unroll
+            for (int n = 0; n < FN; ++n) {
+                f4* p = tot + (m * FN + n) * NT;
+                *p = first ? acc[m][n] : *p + acc[m][n];
+            }
+        clear();
+    };
+    // a wave's operands of one block, as they lie in LDS
+    struct Frags {
+        vu4 x[FM][S][T];
+        uint32_t w[FN][S * BITS / 4];
+        f4 sb[GROUPED ? FN : 1][2];  // scale, bias of four columns, interleaved
+        float2 xf[FM];               // block sum, factor
+    };
+    auto read = [&](Frags& r, const char* base, int b) __attribute__((always_inline)) {
+        const vu4* A = reinterpret_cast<const vu4*>(base) + lane;
+        const char* B = base + A_BYTES;
+        const float2* sb = reinterpret_cast<const float2*>(base + A_BYTES + B_BYTES) + b * BN + 4 * q;
+        const float2* xf = reinterpret_cast<const float2*>(base + A_BYTES + B_BYTES + SB_BYTES) + b * BM + wm * FM * 16 + l16;
+#pragma unroll
+        for (int m = 0; m < FM; ++m) r.xf[m] = xf[m * 16];
+#pragma unroll
+        for (int n = 0; n < FN; ++n) {
+            const int nt = wn * FN + n;
+            uint32_t* w = r.w[n];
+            if constexpr (BITS == 8 && S == 2) {
+                const vu4 v = *reinterpret_cast<const vu4*>(B + nt * 1024 + lane * 16);
+                w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+            } else if constexpr (BITS == 8) {
+                const u2v v = *reinterpret_cast<const u2v*>(B + nt * 1024 + ((b * 2 + (q >> 1)) * 16 + l16) * 16 + (q & 1) * 8);
+                w[0] = v.x; w[1] = v.y;
+            } else if constexpr (S == 2) {
+                const u2v v = *reinterpret_cast<const u2v*>(B + nt * 512 + ((q >> 1) * 16 + l16) * 16 + (q & 1) * 8);
+                w[0] = v.x; w[1] = v.y;
+            } else {
+                w[0] = *reinterpret_cast<const uint32_t*>(B + nt * 512 + (b * 16 + l16) * 16 + q * 4);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < S; ++j)
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int m = 0; m < FM; ++m) r.x[m][j][t] = A[(((wm * FM + m) * 2 + (S == 2 ? j : b)) * T + t) * 64];
+        if constexpr (GROUPED) {
+#pragma unroll
+            for (int n = 0; n < FN; ++n) {
+                const f4* p = reinterpret_cast<const f4*>(sb + (wn * FN + n) * 16);
+                r.sb[n][0] = p[0];
+                r.sb[n][1] = p[1];
+            }
+        }
+    };
+    auto products = [&](const Frags& r, auto own) __attribute__((always_inline)) {
+        constexpr bool OWN = decltype(own)::value;  // some row's block has its own exponent
+#pragma unroll
+        for (int n = 0; n < FN; ++n) {
+            h8 wa[S];
+#pragma unroll
+            for (int j = 0; j < S; ++j) wa[j] = unpack_step<BITS, !GROUPED>(&r.w[n][j * BITS / 4]);
+            f4 blk[FM];
+#pragma unroll
+            for (int m = 0; m < FM; ++m) blk[m] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < S; ++j)
+#pragma unroll
+                for (int t = 0; t < T; ++t)
+#pragma unroll
+                    for (int m = 0; m < FM; ++m) blk[m] = mfma16(wa[j], __builtin_bit_cast(h8, r.x[m][j][t]), blk[m]);
+#pragma unroll
+            for (int m = 0; m < FM; ++m) {
+                if constexpr (OWN) blk[m] *= r.xf[m].y;
+                if constexpr (GROUPED) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[m][n][i] = __builtin_fmaf(r.sb[n][i / 2][i % 2 * 2 + 1], r.xf[m].x,
+                                                      __builtin_fmaf(r.sb[n][i / 2][i % 2 * 2], blk[m][i], acc[m][n][i]));
+                } else {
+                    acc[m][n] += blk[m];
+                }
+            }
+        }
+    };
+    auto finish = [&](int m, int n, f4 v) __attribute__((always_inline)) {
+        const int row = m0 + (wm * FM + m) * 16 + l16, col = n0 + (wn * FN + n) * 16 + 4 * q;
+        float down, sum;
+        if constexpr (INLINE) {
+            const float2 r = row_xr[(wm * FM + m) * 16 + l16];
+            down = r.x;
+            sum = r.y;
+        } else {
+            const vf4 r = a.xr[min(row, a.Mp - 1)];
+            down = r.x;
+            sum = r.y;
+        }
+        wt_store<GROUPED, XF32>(c, row, col, v, down, sum);
+    };
+
+    if constexpr (INLINE) {
+        f4 sum[FM][FN];
+        for (int r = 0; r < a.ranges; ++r) {
+            clear();
+            const int k0 = r * a.rs, n = min(a.rs, a.KB - k0);
+            for (int t = 0; t < n; ++t) {
+                __syncthreads();
+                Stage st;
+                load(st, k0 + t);
+                stage_inline(k0 + t);
+                store(st, 0);
+                __syncthreads();
+#pragma unroll
+                for (int b = 0; b < NG; ++b) {
+                    Frags r;
+                    read(r, lds, b);
+                    products(r, std::integral_constant<bool, T == 2>{});  // factors of 1 change nothing
+                }
+                if (t % WT_FLUSH == WT_FLUSH - 1 || t == n - 1) flush(t < WT_FLUSH);
+            }
+#pragma unroll
+            for (int m = 0; m < FM; ++m)
+#pragma unroll
+                for (int nn = 0; nn < FN; ++nn) {
+                    const f4 v = tot[(m * FN + nn) * NT];
+                    sum[m][nn] = r ? sum[m][nn] + v : v;
+                }
+        }
+#pragma unroll
+        for (int m = 0; m < FM; ++m)
+#pragma unroll
+            for (int nn = 0; nn < FN; ++nn) finish(m, nn, sum[m][nn]);
+    } else {
+        const int k0 = blockIdx.y * a.rs, n = min(a.rs, a.KB - k0);
+        clear();
+        // stage t + 1 goes from registers to LDS and stage t + 2 from memory to registers while
+        // stage t is computed (the last stages repeat the range's last one: no branch in the loop)
+        Stage st;
+        load(st, k0);
+        store(st, 0);
+        load(st, k0 + min(1, n - 1));
+        auto walk = [&](auto own) __attribute__((always_inline)) {
+            for (int t = 0; t < n; ++t) {
+                block_barrier();  // stage t is in LDS; the other slot has been read
+                store(st, (t + 1) & 1);
+                load(st, k0 + min(t + 2, n - 1));
+#pragma unroll
+                for (int b = 0; b < NG; ++b) {
+                    Frags r;
+                    read(r, lds + (t & 1) * STAGE, b);
+                    products(r, own);
+                }
+                if (t % WT_FLUSH == WT_FLUSH - 1 || t == n - 1) flush(t < WT_FLUSH);
+            }
+        };
+        // one test per workgroup: a test per block would wait for the factors before every product
+        // (141 against 109 us at M = 1024, N = K = 4096, 8 bits)
+        bool own = false;
+        if (T == 2) own = __syncthreads_or(tid < BM && a.xr[min(m0 + tid, a.Mp - 1)].z != 0.0f);
+        if (own) walk(std::integral_constant<bool, T == 2>{});
+        else walk(std::false_type{});
+        if (a.part) {
+            f4* dst = reinterpret_cast<f4*>(a.part) + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * FM * FN * 64 * W + tid;
+#pragma unroll
+            for (int m = 0; m < FM; ++m)
+#pragma unroll
+                for (int nn = 0; nn < FN; ++nn) dst[(m * FN + nn) * NT] = tot[(m * FN + nn) * NT];
+        } else {
+#pragma unroll
+            for (int m = 0; m < FM; ++m)
+#pragma unroll
+                for (int nn = 0; nn < FN; ++nn) finish(m, nn, tot[(m * FN + nn) * NT]);
+        }
+    }
+}
+
+// Adds the K ranges' sums in range order and finishes the outputs: blockIdx.x the tile,
+// blockIdx.y the fragment, a thread the four outputs of its lane.
+template <bool GROUPED, bool XF32, int WM, int WN, int FM, int FN>
+__global__ __launch_bounds__(64 * WM * WN) void wo_tile_reduce_kernel(WtArgs a) {
+    constexpr int W = WM * WN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, l16 = lane & 15;
+    const int m = blockIdx.y / FN, n = blockIdx.y % FN;
+    int tm, tn;
+    wt_tile_of(blockIdx.x, a.tiles_m, a.tiles_n, tm, tn);
+    const int row = tm * 16 * WM * FM + (wave / WN * FM + m) * 16 + l16;
+    const int col = tn * 16 * WN * FN + (wave % WN * FN + n) * 16 + 4 * q;
+    const f4* src = reinterpret_cast<const f4*>(a.part) + ((int64_t)blockIdx.x * FM * FN + blockIdx.y) * 64 * W + tid;
+    const int64_t stride = (int64_t)gridDim.x * FM * FN * 64 * W;
+    const vf4 xr = a.xr[min(row, a.Mp - 1)];
+    f4 v = src[0];
+    int r = 1;
+    for (; r + 3 < a.ranges; r += 4) {
+        const f4 p0 = src[r * stride], p1 = src[(r + 1) * stride], p2 = src[(r + 2) * stride], p3 = src[(r + 3) * stride];
+        v += p0; v += p1; v += p2; v += p3;
+    }
+    for (; r < a.ranges; ++r) v += src[r * stride];
+    wt_store<GROUPED, XF32>(a.c, row, col, v, xr.x, xr.y);
+}
+
+// ------------------------------------------------------------------ host side
+
+enum { WT_128 = 0, WT_64 = 1, WT_32 = 2 };
+
+struct WtPlan {
+    int cfg, BM, BN;
+    int64_t tiles_m, tiles_n;
+    int KB, rs, ranges;
+    size_t xp, xm, xr, sb, part;  // byte sizes
+};
+
+WtPlan wt_plan(int64_t M, int64_t N, int64_t K, bool xf32, int gs) {
+    WtPlan p{};
+    p.cfg = M <= 32 ? WT_32 : M <= 64 ? WT_64 : WT_128;
+    p.BM = p.cfg == WT_128 ? 128 : p.cfg == WT_64 ? 64 : 32;
+    p.BN = 128;
+    p.tiles_m = (M + p.BM - 1) / p.BM;
+    p.tiles_n = (N + p.BN - 1) / p.BN;
+    p.KB = (int)((K + 63) / 64);
+    const int64_t t = p.tiles_m * p.tiles_n;
+    // fewer tiles than CUs: K ranges of at least four stages, about one workgroup per CU
+    const int64_t want = t > 128 ? 1 : std::min<int64_t>({16, 256 / t, std::max(1, p.KB / 4)});
+    p.rs = (int)((p.KB + want - 1) / want);
+    p.ranges = (p.KB + p.rs - 1) / p.rs;
+    const int NG = gs == 32 ? 2 : 1, T = xf32 ? 2 : 1;
+    const int64_t Mp = (M + 15) / 16 * 16;
+    auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    p.xp = up((size_t)Mp * p.KB * 128 * T);
+    p.xm = up((size_t)p.KB * NG * 2 * Mp * 4);
+    p.xr = up((size_t)Mp * 16);
+    p.sb = gs ? up((size_t)(K / gs) * 8 * (size_t)(p.tiles_n * p.BN)) : 0;
+    p.part = p.ranges > 1 ? up((size_t)p.ranges * t * p.BM * p.BN * 4) : 0;
+    return p;
+}
+
+template <int BITS, int S, int T, bool GROUPED, int HM, int WM, int WN, int FM, int FN>
+void wt_go(const WtPlan& p, WtArgs& a, hipStream_t st) {
+    const unsigned t = (unsigned)(p.tiles_m * p.tiles_n);
+    const unsigned scale_blocks = GROUPED ? (unsigned)((a.G + 31) / 32) * (unsigned)(a.Np / 32) : 0;
+    hipLaunchKernelGGL((wo_tile_prep_kernel<BITS, S, T, GROUPED, HM>), dim3((unsigned)a.Mp + scale_blocks), dim3(256), 0, st, a,
+                       const_cast<char*>(a.xp), const_cast<float2*>(a.xm), const_cast<vf4*>(a.xr),
+                       const_cast<float2*>(a.sb));
+    hipLaunchKernelGGL((wo_tile_kernel<BITS, S, T, GROUPED, HM, WM, WN, FM, FN, false>), dim3(t, (unsigned)p.ranges),
+                       dim3(64 * WM * WN), 0, st, a);
+    if (p.ranges > 1)
+        hipLaunchKernelGGL((wo_tile_reduce_kernel<GROUPED, T == 2, WM, WN, FM, FN>), dim3(t, FM * FN), dim3(64 * WM * WN), 0, st, a);
+}
+
+template <int BITS, int S, bool GROUPED>
+void wt_config(const WtPlan& p, WtArgs& a, bool inl, hipStream_t st) {
+    auto go = [&](auto t, auto h) {
+        constexpr int T = decltype(t)::value, HM = decltype(h)::value;
+        if (inl) {  // one tile size: an output's sums do not depend on it
+            a.tiles_m = (a.c.M + 31) / 32;
+            hipLaunchKernelGGL((wo_tile_kernel<BITS, S, T, GROUPED, HM, 1, 4, 2, 2, true>),
+                               dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(256), 0, st, a);
+        } else if (p.cfg == WT_128) wt_go<BITS, S, T, GROUPED, HM, 2, 4, 4, 2>(p, a, st);
+        else if (p.cfg == WT_64) wt_go<BITS, S, T, GROUPED, HM, 2, 4, 2, 2>(p, a, st);
+        else wt_go<BITS, S, T, GROUPED, HM, 2, 4, 1, 2>(p, a, st);
+    };
+    using T1 = std::integral_constant<int, 1>;
+    using T2 = std::integral_constant<int, 2>;
+    using None = std::integral_constant<int, LQ_ROUND_NONE>;
+    if constexpr (!GROUPED) {
+        a.c.xf32 ? go(T2{}, None{}) : go(T1{}, None{});
+    } else {  // scales rounded to the activation's type: half always, bfloat16 on request
+        if (!a.c.xf32) go(T1{}, std::integral_constant<int, LQ_ROUND_F16>{});
+        else if (a.c.hmode == LQ_ROUND_BF16) go(T2{}, std::integral_constant<int, LQ_ROUND_BF16>{});
+        else go(T2{}, None{});
+    }
+}
+
+}  // namespace
+
+bool wo_tile_takes(const WoTileCall& c) {
+    // Three launches and their latencies (17 us at M = 32, N = K = 4096) against a GEMV kernel whose
+    // time grows with the 16-row blocks times the weight: measured equal near 2^25 (M = 32: 19.4
+    // against 16.9 us in float32, 16.7 against 17.3 in half; M = 33: 27.2 against 20.7; M = 600,
+    // N = 512, K = 1024, 2^24.2: 15.2 against 21.2 us).
+    if (c.M <= 16 || c.K < 64 || (int64_t)((c.M + 15) / 16) * c.N * c.K <= ((int64_t)1 << 25)) return false;
+    const int64_t row_bytes = (int64_t)c.K * c.bits / 8;
+    if (!aligned16(c.w) || c.ldw_bytes % 16 || row_bytes % 16) return false;
+    // 32-bit offsets inside a workgroup's weight rows and scales; grid and tile counts
+    if (128 * c.ldw_bytes >= ((int64_t)1 << 31)) return false;
+    const WtPlan p = wt_plan(c.M, c.N, c.K, c.xf32, c.gs);
+    return p.tiles_m * p.tiles_n < ((int64_t)1 << 24) && (c.gs == 0 || (int64_t)128 * (c.K / c.gs) < ((int64_t)1 << 28)) &&
+           (int64_t)4 * c.M < ((int64_t)1 << 28);
+}
+
+size_t wo_tile_ws_bytes(int64_t M, int64_t N, int64_t K, int gs) {
+    size_t need = 0;
+    for (int xf32 = 0; xf32 < 2; ++xf32) {
+        const WtPlan p = wt_plan(M, std::max<int64_t>(N, 1), K, xf32 != 0, gs);
+        need = std::max(need, p.xp + p.xm + p.xr + p.sb + p.part);
+    }
+    return need;
+}
+
+int wo_tile_launch(const WoTileCall& c, void* ws, size_t ws_bytes, hipStream_t st) {
+    const WtPlan p = wt_plan(c.M, c.N, c.K, c.xf32, c.gs);
+    WtArgs a{};
+    a.c = c;
+    a.G = c.gs ? c.K / c.gs : 1;
+    a.KB = p.KB;
+    a.Mp = (c.M + 15) / 16 * 16;
+    a.Np = (int)(p.tiles_n * p.BN);
+    a.tiles_m = (int)p.tiles_m;
+    a.tiles_n = (int)p.tiles_n;
+    a.rs = p.rs;
+    a.ranges = p.ranges;
+    const bool inl = !ws || !aligned16(ws) || ws_bytes < p.xp + p.xm + p.xr + p.sb + p.part;
+    if (!inl) {
+        char* b = static_cast<char*>(ws);
+        a.xp = b;
+        a.xm = reinterpret_cast<const float2*>(b + p.xp);
+        a.xr = reinterpret_cast<const vf4*>(b + p.xp + p.xm);
+        a.sb = reinterpret_cast<const float2*>(b + p.xp + p.xm + p.xr);
+        a.part = p.part ? reinterpret_cast<float*>(b + p.xp + p.xm + p.xr + p.sb) : nullptr;
+    }
+    if (c.gs == 0) wt_config<8, 2, false>(p, a, inl, st);
+    else if (c.bits == 8) c.gs == 32 ? wt_config<8, 1, true>(p, a, inl, st) : wt_config<8, 2, true>(p, a, inl, st);
+    else c.gs == 32 ? wt_config<4, 1, true>(p, a, inl, st) : wt_config<4, 2, true>(p, a, inl, st);
+    note_path(inl ? "wo tiles inline" : p.ranges > 1 ? "wo tiles split" : "wo tiles");
+    return LQ_OK;
+}
+
+}  // namespace lq

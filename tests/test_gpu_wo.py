@@ -361,6 +361,78 @@ def test_group_matmul_presplit_matches_inline(gpu, bits, gs):
     np.testing.assert_array_equal(outs[0], outs[1])
 
 
+# (bits, group size (0: per-channel int8), M, N, K): the 32 / 64 / 128-row tiles, ragged last tiles
+# and stages, K ranges and none
+WO_TILE_CASES = [(8, 0, 20, 4608, 4096), (8, 0, 64, 4099, 4096), (8, 0, 600, 1000, 1040), (8, 0, 1031, 515, 1040),
+                 (8, 0, 2049, 2100, 272), (8, 64, 33, 4096, 4096), (8, 64, 1025, 2050, 512), (8, 128, 129, 2048, 2176),
+                 (8, 32, 300, 1900, 1056), (4, 32, 30, 4200, 4128), (4, 64, 700, 640, 2048), (4, 128, 2200, 2180, 384)]
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("bits,gs,M,N,K", WO_TILE_CASES)
+def test_wo_tiles(gpu, bits, gs, M, N, K, half):
+    """The tiled kernel for many rows: against float64 within the fp32 / fp16 tolerance, the same
+    bits with and without a workspace; rows of very different magnitude, and a row whose later
+    blocks are far smaller than its first (blocks with their own exponent) under weights that are
+    zero in that first block, so its result is the small blocks' alone."""
+    from lucid_amd import _C
+    from lucid_amd.quantization import _qgemm
+
+    rng = np.random.default_rng(M + K + bits + gs)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    if not half:
+        x[0] *= 1e-20
+        x[-1] *= 1e15
+        x[1, 64:] *= 1e-9
+    x[2] = 0.0
+    if half:
+        x = x.astype(np.float16)
+    b = rng.standard_normal(N).astype(np.float32)
+    xd, bd = _t(gpu, x), _t(gpu, b)
+    code = _C.F16 if half else _C.F32
+    if gs == 0:
+        W = rng.integers(-128, 128, (N, K)).astype(np.int8)
+        W[0, :64] = 0
+        s = rng.uniform(1e-3, 1e-1, N).astype(np.float32)
+        z = rng.integers(-3, 4, N).astype(np.float32)
+        z[0] = 0.0
+        dW, ds, dz = _t(gpu, W), _t(gpu, s), _t(gpu, z)
+        wd = (W.astype(np.float64) - z[:, None]) * s[:, None]
+        nbytes = _C.lib().lq_gemv_w8_workspace_size(M, N, K)
+        call = lambda y, ws, n: _C.call(  # noqa: E731
+            "lq_gemv_w8", xd.data_ptr(), code, K, dW.data_ptr(), K, ds.data_ptr(), dz.data_ptr(), bd.data_ptr(),
+            y.data_ptr(), N, M, N, K, _C.EPI_RELU, ws, n, None)
+    else:
+        w = rng.standard_normal((N, K)).astype(np.float32)
+        w[0, :64] = 0.0
+        packed, scales, biases = _qgemm.quantize(_t(gpu, w), group_size=gs, bits=bits)
+        sc, bi = scales.numpy(), biases.numpy()
+        if half:  # scales and group biases in x's type
+            sc, bi = sc.astype(np.float16).astype(np.float32), bi.astype(np.float16).astype(np.float32)
+        wd = O.group_dequantize(packed.numpy().view(np.uint32), sc, bi, gs, bits).astype(np.float64)
+        nbytes = _C.lib().lq_group_matmul_workspace_size(M, N, K, gs)
+        call = lambda y, ws, n: _C.call(  # noqa: E731
+            "lq_group_matmul", xd.data_ptr(), code, K, packed.data_ptr(), scales.data_ptr(), biases.data_ptr(),
+            bd.data_ptr(), y.data_ptr(), N, M, N, K, gs, bits, 1, _C.EPI_RELU, ws, n, None)
+    outs = []
+    for n, path in ((nbytes, "wo tiles"), (0, "wo tiles inline")):
+        ws = gpu.empty((max(n, 16),), np.uint8, "gpu")
+        y = gpu.empty((M, N), x.dtype, "gpu")
+        call(y, ws.data_ptr() if n else None, n)
+        assert _C.last_path().startswith(path)
+        outs.append(y.numpy())
+    np.testing.assert_array_equal(outs[0], outs[1])
+    # row by row: the scale of a comparison is the row's own largest result without the bias
+    prod = x.astype(np.float64) @ wd.T
+    ref = np.maximum(prod + (b.astype(np.float16) if half and gs else b), 0.0)
+    rtol = 1e-3 if half else 1e-5
+    atol = rtol * (np.abs(prod).max(1, keepdims=True) + np.abs(b))
+    assert np.all(np.abs(outs[0] - ref) <= atol + rtol * np.abs(ref))
+    if not half:  # the small blocks' result, without the large block's products
+        want = max(prod[1, 0] + b[0], 0.0)
+        assert abs(outs[0][1, 0] - want) <= 1e-5 * (abs(prod[1, 0]) + abs(b[0]))
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("M,N,K", [(16, 4096, 4096), (5, 4608, 4096), (12, 1000, 2048)])
