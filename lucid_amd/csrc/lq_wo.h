@@ -102,4 +102,23 @@ size_t wo_tile_ws_bytes(int64_t M, int64_t N, int64_t K, int gs);
 // every workgroup, with the same results.
 int wo_tile_launch(const WoTileCall& c, void* ws, size_t ws_bytes, hipStream_t st);
 
+// ---------------------------------------------- x . w_hat (lq_wo_nt.hip)
+
+// y[M, K] = x[M, N] w_hat[N, K] (+ bias, ReLU) of group-wise packed rows.
+struct WoNtCall {
+    const void* x;
+    int64_t ldx;
+    bool xf32;
+    const uint8_t* w;
+    const float* scales;   // [N][K / gs]
+    const float* biases;   // [N][K / gs] or null
+    const float* bias;     // layer bias [K] or null
+    void* y;
+    int64_t ldy;
+    int relu, hmode;
+    int M, N, K, bits, gs;
+};
+
+void group_matmul_nt_launch(const WoNtCall& c, hipStream_t st);
+
 }  // namespace lq

@@ -9,8 +9,8 @@
 //    y = sum_g (s[n,g] sum_{k in g} c[n,k] x[m,k] + b[n,g] sum_{k in g} x[m,k]) + bias[n]
 //    -- quantized_matmul with transpose=true (lucid/_C/ops/quantized/QuantizedMatmul.cpp:143-163,
 //    formula lucid/quantization/_qgemm.py:167-170).
-// The transpose=false product x . w_hat (also the QLoRA input gradient) is a separate float32
-// tiled kernel, group_matmul_nt_kernel, below.
+// The transpose=false product x . w_hat (also the QLoRA input gradient) is in lq_wo_nt.hip, the
+// product of many activation rows in lq_wo_tile.hip.
 //
 // Operands.  The codes enter the MFMA as exact fp16 values: a code c of 8 or fewer bits is
 // placed under the exponent of 1024 (fp16 1024 + c, by v_perm byte placement or nibble
@@ -1021,130 +1021,6 @@ __global__ __launch_bounds__(256) void group_dequantize_kernel(const uint32_t* _
         *reinterpret_cast<vf4*>(w + id * PER + e) = vf4{out[e], out[e + 1], out[e + 2], out[e + 3]};
 }
 
-// ------------------------------------------- x . w_hat (quantized_matmul, transpose = false)
-//
-// y[m, k] = sum_n x[m, n] w_hat[n, k] for the packed w_hat[N, K] (groups along k): the product
-// of quantized_matmul with transpose=false, and the input gradient of the transpose=true
-// product, dX = dY dequant(W) (QuantizedMatmulBackward::apply, QuantizedMatmul.cpp:73-90).
-// The group scale / bias change along the summed axis n, so there is no factoring of the
-// sums as in the transpose=true kernel: each weight tile is dequantized into LDS exactly as
-// group_dequantize_kernel writes it, fl32(fl32(c s) + b), and the kernel is a float32 tiled
-// GEMM over it (128 x 128 outputs per 256-thread workgroup, 8 x 8 per thread, n in steps of
-// 16, fused multiply-adds in n order).
-constexpr int NT_T = 128, NT_K = 16, NT_R = NT_T / 16;
-
-template <int BITS, bool XF32>
-__global__ __launch_bounds__(256) void group_matmul_nt_kernel(const void* __restrict__ xv, int64_t ldx,
-                                                              const uint32_t* __restrict__ packed,
-                                                              const float* __restrict__ scales,
-                                                              const float* __restrict__ biases,
-                                                              const float* __restrict__ bias, void* __restrict__ yv,
-                                                              int64_t ldy, int64_t M, int64_t N, int64_t K, int gs,
-                                                              int relu, int hmode) {
-    constexpr int PER = 32 / BITS;
-    constexpr uint32_t L = (1u << BITS) - 1u;
-    constexpr int WPR = NT_T / PER;  // packed words per tile row
-    __shared__ __attribute__((aligned(16))) float xs[NT_K][NT_T + 4];  // row stride 16-byte aligned
-    __shared__ __attribute__((aligned(16))) float ws[NT_K][NT_T];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int64_t G = K / gs, words_per_row = K / PER;
-    const int64_t KT = (K + NT_T - 1) / NT_T, MT = (M + NT_T - 1) / NT_T;
-    for (int64_t tile = blockIdx.x; tile < KT * MT; tile += gridDim.x) {
-        const int64_t k0 = (tile % KT) * NT_T, m0 = (tile / KT) * NT_T;
-        float acc[NT_R][NT_R] = {};
-        // The next n-tile's activations and packed words (with their group scale / bias) are
-        // loaded into registers while this tile's FMAs run, then dequantized into LDS.
-        constexpr int XPT = NT_T * NT_K / 256, WPT = (NT_K * WPR + 255) / 256;
-        float xq[XPT];
-        uint32_t wq[WPT];
-        float sq[WPT], bq[WPT];
-        auto fetch = [&](int64_t n0) __attribute__((always_inline)) {
-#pragma unroll
-            for (int u = 0; u < XPT; ++u) {
-                const int e = threadIdx.x + 256 * u;
-                const int r = e / NT_K, kk = e % NT_K;
-                const int64_t gm = m0 + r, gn = n0 + kk;
-                float v = 0.0f;
-                if (gm < M && gn < N) {
-                    if constexpr (XF32) v = static_cast<const float*>(xv)[gm * ldx + gn];
-                    else v = (float)static_cast<const _Float16*>(xv)[gm * ldx + gn];
-                }
-                xq[u] = v;
-            }
-#pragma unroll
-            for (int u = 0; u < WPT; ++u) {
-                const int e = threadIdx.x + 256 * u;
-                const int r = e / WPR, wc = e % WPR;
-                const int64_t gn = n0 + r, gk = k0 + (int64_t)wc * PER;
-                wq[u] = 0u;
-                sq[u] = 0.0f;
-                bq[u] = 0.0f;
-                if (e < NT_K * WPR && gn < N && gk < K) {  // K is a multiple of the group size: whole words
-                    wq[u] = packed[gn * words_per_row + gk / PER];
-                    const int64_t gi = gn * G + gk / gs;
-                    sq[u] = round_to(scales[gi], hmode);
-                    bq[u] = biases ? round_to(biases[gi], hmode) : 0.0f;
-                }
-            }
-        };
-        fetch(0);
-        for (int64_t n0 = 0; n0 < N; n0 += NT_K) {
-#pragma unroll
-            for (int u = 0; u < XPT; ++u) {
-                const int e = threadIdx.x + 256 * u;
-                xs[e % NT_K][e / NT_K] = xq[u];
-            }
-#pragma unroll
-            for (int u = 0; u < WPT; ++u) {
-                const int e = threadIdx.x + 256 * u;
-                if (e < NT_K * WPR) {
-                    const int r = e / WPR, wc = e % WPR;
-#pragma unroll
-                    for (int q = 0; q < PER; ++q) {  // w_hat = fl32(fl32(c s) + b); 0 past N / K (s = 0)
-                        const float t = (float)((wq[u] >> (q * BITS)) & L) * sq[u];
-                        ws[r][wc * PER + q] = biases ? t + bq[u] : t;
-                    }
-                }
-            }
-            __syncthreads();
-            if (n0 + NT_K < N) fetch(n0 + NT_K);
-#pragma unroll
-            for (int kk = 0; kk < NT_K; ++kk) {
-                // this thread's NT_R consecutive rows and columns: 16-byte LDS reads
-                float xr[NT_R], wr[NT_R];
-#pragma unroll
-                for (int i = 0; i < NT_R; i += 4) {
-                    const vf4 v = *reinterpret_cast<const vf4*>(&xs[kk][ty * NT_R + i]);
-                    xr[i] = v[0]; xr[i + 1] = v[1]; xr[i + 2] = v[2]; xr[i + 3] = v[3];
-                }
-#pragma unroll
-                for (int j = 0; j < NT_R; j += 4) {
-                    const vf4 v = *reinterpret_cast<const vf4*>(&ws[kk][tx * NT_R + j]);
-                    wr[j] = v[0]; wr[j + 1] = v[1]; wr[j + 2] = v[2]; wr[j + 3] = v[3];
-                }
-#pragma unroll
-                for (int i = 0; i < NT_R; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT_R; ++j) acc[i][j] = fmaf(xr[i], wr[j], acc[i][j]);
-            }
-            __syncthreads();
-        }
-#pragma unroll
-        for (int i = 0; i < NT_R; ++i) {
-            const int64_t gm = m0 + ty * NT_R + i;
-            if (gm >= M) continue;
-#pragma unroll
-            for (int j = 0; j < NT_R; ++j) {
-                const int64_t gk = k0 + tx * NT_R + j;
-                if (gk >= K) continue;
-                const float v = wo_finish(acc[i][j], bias != nullptr, bias ? bias[gk] : 0.0f, relu, hmode);
-                if constexpr (XF32) static_cast<float*>(yv)[gm * ldy + gk] = v;
-                else static_cast<_Float16*>(yv)[gm * ldy + gk] = (_Float16)v;
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------ host side
 
 struct WoPlan {
@@ -1493,21 +1369,10 @@ int lq_group_matmul(const void* d_x, int x_dtype, int64_t ldx, const uint32_t* d
         if (M == 0) return LQ_OK;
         LQ_REQUIRE(d_x && d_y && (N == 0 || (d_packed && d_scales)), "lq_group_matmul: NULL pointer");
         LQ_REQUIRE(ldx >= N && ldy >= K, "lq_group_matmul: leading dimension too small");
-        const int64_t tiles = ((M + NT_T - 1) / NT_T) * ((K + NT_T - 1) / NT_T);
-        const dim3 grid((unsigned)std::min<int64_t>(tiles, 1 << 20));
-        const uint32_t* pk = N ? d_packed : nullptr;
-        const float* gb = N ? d_biases : nullptr;
-        const int relu = (flags & LQ_EPI_RELU) ? 1 : 0;
-        hipStream_t st = as_stream(stream);
-#define LQ_NT(B, XF)                                                                                           \
-    hipLaunchKernelGGL((group_matmul_nt_kernel<B, XF>), grid, dim3(256), 0, st, d_x, ldx, pk, d_scales, gb, d_bias, \
-                       d_y, ldy, M, N, K, group_size, relu, hmode)
-        if (bits == 8) {
-            if (x_dtype == LQ_F32) LQ_NT(8, true); else LQ_NT(8, false);
-        } else {
-            if (x_dtype == LQ_F32) LQ_NT(4, true); else LQ_NT(4, false);
-        }
-#undef LQ_NT
+        const WoNtCall c{d_x, ldx, x_dtype == LQ_F32, reinterpret_cast<const uint8_t*>(N ? d_packed : nullptr), d_scales,
+                         N ? d_biases : nullptr, d_bias, d_y, ldy, (flags & LQ_EPI_RELU) ? 1 : 0, hmode, (int)M, (int)N,
+                         (int)K, bits, group_size};
+        group_matmul_nt_launch(c, as_stream(stream));
         return launch_status("lq_group_matmul");
     }
     if (M == 0 || N == 0) return LQ_OK;

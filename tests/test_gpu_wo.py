@@ -699,6 +699,58 @@ def test_quantized_matmul_backward_is_the_adjoint(gpu, transpose, bits):
     assert abs(lhs - rhs) <= 1e-5 * mag
 
 
+# (M, N, K, bits, group size): the three tile sizes, ragged rows, summed lengths that are no
+# multiple of 32 or 8, last tiles of one group
+NT_CASES = [(33, 40, 64, 8, 64), (1, 8, 32, 4, 32), (70, 333, 288, 4, 32), (129, 1000, 640, 8, 128),
+            (700, 333, 2432, 8, 64), (2100, 520, 2432, 4, 128), (2049, 136, 2464, 8, 32)]
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N,K,bits,gs", NT_CASES)
+def test_quantized_matmul_no_transpose_tiles(gpu, M, N, K, bits, gs, half):
+    """Every tile size against float64, with rows whose magnitude grows, shrinks or starts at zero
+    along the summed axis (the running power of two of the fp16 split), a row whose large part
+    meets zero weights, and infinities and NaN where float64 has them."""
+    from lucid_amd.quantization import _qgemm
+
+    rng = np.random.default_rng(M + N + K + bits)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    zero = N // 64 * 32  # whole steps: the split keeps ~22 bits of a row's largest value in its step
+    w[:zero] = 0.0
+    x = rng.standard_normal((M, N)).astype(np.float32)
+    if M > 8:
+        if not half:
+            x[0] *= np.logspace(-12, 12, N).astype(np.float32)
+            x[1] *= np.logspace(12, -12, N).astype(np.float32)
+            x[2, :zero] *= 1e15
+            x[2, zero:] *= 1e-5
+        x[3, :zero] = 0.0
+        x[4] = 0.0
+    if half:
+        x = x.astype(np.float16)
+    packed, scales, biases = _qgemm.quantize(_t(gpu, w), group_size=gs, bits=bits)
+    sc, bi = scales.numpy(), biases.numpy()
+    if half:
+        sc, bi = sc.astype(np.float16).astype(np.float32), bi.astype(np.float16).astype(np.float32)
+    wd = O.group_dequantize(packed.numpy().view(np.uint32), sc, bi, gs, bits).astype(np.float64)
+    run = lambda v: _qgemm.quantized_matmul(_t(gpu, v), packed, scales, biases, transpose=False,  # noqa: E731
+                                            group_size=gs, bits=bits).numpy()
+    y = run(x)
+    ref = x.astype(np.float64) @ wd
+    rtol = 1e-3 if half else 1e-5
+    # a float32 sum's error scales with the sum of its terms' magnitudes
+    assert np.all(np.abs(y - ref) <= rtol * (np.abs(x.astype(np.float64)) @ np.abs(wd)) + (2.0 ** -24 if half else 0.0))
+    x[M // 2, N - 1] = np.inf
+    x[M // 2, 0] = np.inf
+    if M > 8:
+        x[5, N // 3] = np.nan
+    with np.errstate(invalid="ignore"):
+        ref = x.astype(np.float64) @ wd
+    y = run(x)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
+    np.testing.assert_array_equal(np.isinf(y), np.isinf(ref))
+
+
 def test_group_matmul_no_transpose_empty_reduction(gpu):
     """N = 0: x [M, 0] @ w_hat[0, K] is the bias alone."""
     from lucid_amd import _C
