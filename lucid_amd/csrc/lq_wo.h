@@ -121,4 +121,13 @@ struct WoNtCall {
 
 void group_matmul_nt_launch(const WoNtCall& c, hipStream_t st);
 
+// ---------------------------------------------- 1 to 16 rows over the packed weight (lq_wo_stream.hip)
+
+// Workspace of the K ranges' sums (0 up to K = 4096).
+size_t wo_stream_ws_bytes(int64_t N, int64_t K);
+// Whether it is the faster form for the shape.
+bool wo_stream_preferred(int64_t M, int64_t N, int64_t K, bool xf32);
+// c.w is lq_pack_weights_i8's form; M <= 16, K a multiple of 16, 16-byte aligned x rows and weight.
+void wo_stream_launch(const WoTileCall& c, void* ws, hipStream_t st);
+
 }  // namespace lq

@@ -1299,7 +1299,7 @@ int lq_gemv_w8(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d_W, int
 
 size_t lq_gemv_w8_packed_workspace_size(int64_t M, int64_t N, int64_t K) {
     if (M < 1 || M > SK_MAX_M || K <= 0 || K >= WO_MAX_DIM || N <= 0 || N >= WO_MAX_DIM) return 0;
-    return sk_ws_bytes(sk_plan(N, K));
+    return std::max(sk_ws_bytes(sk_plan(N, K)), wo_stream_ws_bytes(N, K));
 }
 
 int lq_gemv_w8_packed(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d_W_packed,
@@ -1318,7 +1318,7 @@ int lq_gemv_w8_packed(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d
     LQ_REQUIRE(K >= 16 && K % 16 == 0, "lq_gemv_w8_packed: K must be a positive multiple of 16");
     LQ_REQUIRE(aligned16(d_W_packed) && aligned16(d_x) && (ldx * eb) % 16 == 0,
                "lq_gemv_w8_packed: the weight, x and its rows must be 16-byte aligned");
-    const size_t need = sk_ws_bytes(sk_plan(N, K));
+    const size_t need = std::max(sk_ws_bytes(sk_plan(N, K)), wo_stream_ws_bytes(N, K));
     LQ_REQUIRE(need == 0 || (d_workspace && aligned16(d_workspace) && workspace_bytes >= need),
                "lq_gemv_w8_packed: workspace smaller than lq_gemv_w8_packed_workspace_size");
     WoArgs a{};
@@ -1335,6 +1335,10 @@ int lq_gemv_w8_packed(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d
     a.M = (int)M;
     a.N = (int)N;
     a.K = (int)K;
+    if (wo_stream_preferred(M, N, K, xf32)) {
+        wo_stream_launch(tile_call(a, xf32, 8, 0), d_workspace, as_stream(stream));
+        return launch_status("lq_gemv_w8_packed");
+    }
     const int rc = launch_sk<8, true, 2, false, true>(a, xf32, as_stream(stream), d_workspace);
     return rc ? rc : launch_status("lq_gemv_w8_packed");
 }
