@@ -302,8 +302,9 @@ enum { LQ_EPI_RELU = 1, LQ_EPI_A_U8S8 = 2, LQ_EPI_ROUND_BF16 = 4 /* lq_group_mat
  * The zero points enter as sum_k A*B - za*bsum[n] - zb[n]*asum[m] + K*za*zb[n] with
  * bsum[n] = sum_k B[n,k] (d_b_sums, e.g. cached by the module from lq_row_sums_i8; NULL =
  * computed into the workspace) and asum[m] = sum_k A[m,k] (computed when zb is given).
- * Fast paths need 16-byte aligned A/B, lda/ldb/K multiples of 16; other shapes run a
- * generic kernel with the same results.
+ * Fast paths need 16-byte aligned A/B, lda/ldb/K multiples of 16; with the workspace, operands
+ * whose K is no multiple of 16 are copied into that form first; other shapes run a generic
+ * kernel with the same results.
  * Replaces the nnq.Linear / nnqd.Linear compute: dequantize(W) -> F.linear -> act ->
  * fake_quantize (lucid/nn/quantized/linear.py:206-215, dynamic/linear.py:85-92,
  * Linear.cpp:199 -> Matmul.cpp:80-122).  The workspace (lq_gemm_w8a8_workspace_size)
@@ -320,7 +321,8 @@ int lq_gemm_w8a8(const int8_t* d_A, int64_t lda, const int8_t* d_B, int64_t ldb,
 /* lq_gemm_w8a8 without a workspace argument, allocating nothing: the code sums, split-K
  * partials and tile counters live in a static 16 MiB device array the library holds on each
  * GPU it runs on (lq_gemm_w8a8_noalloc_scratch_bytes()).  Shapes whose workspace
- * (lq_gemm_w8a8_workspace_size) exceeds it fail with LQ_ERR_UNSUPPORTED.  Calls on one GPU
+ * (lq_gemm_w8a8_workspace_size, without the aligned copies it holds for a K that is no multiple
+ * of 16) exceeds it fail with LQ_ERR_UNSUPPORTED.  Calls on one GPU
  * share the array, so calls that overlap on one GPU (concurrent streams or threads) race;
  * serialize them.  Same results as lq_gemm_w8a8.  No counterpart in the reference: for
  * callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses

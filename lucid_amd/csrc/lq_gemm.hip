@@ -39,7 +39,8 @@ struct GemmArgs {
     const int8_t* B;
     void* C;
     int64_t lda, ldb, ldc;
-    int M, N, K;
+    int M, N, K;             // K: bytes of a row that are summed (zeros past k_true)
+    int k_true;              // the product's own K
     const float* a_scale;
     const float* b_scale;
     int a_stride, b_stride;
@@ -85,7 +86,7 @@ __device__ __forceinline__ int32_t corrected(int32_t raw, int m, int n, const Ge
     if (a.b_zp) {
         const uint32_t zb = (uint32_t)(int)a.b_zp[n];
         acc -= zb * (uint32_t)a.a_sums[m];
-        acc += (uint32_t)a.K * (uint32_t)p.za * zb;
+        acc += (uint32_t)a.k_true * (uint32_t)p.za * zb;
     }
     return (int32_t)acc;
 }
@@ -147,7 +148,7 @@ __device__ __forceinline__ void epilogue4c(const GemmArgs& a, const EpiParams& p
         if (p.has_za) acc -= (uint32_t)p.za * (uint32_t)c.bsum[r];
         if (a.b_zp) {
             acc -= (uint32_t)c.zb[r] * (uint32_t)row.asum;
-            acc += (uint32_t)a.K * (uint32_t)p.za * (uint32_t)c.zb[r];
+            acc += (uint32_t)a.k_true * (uint32_t)p.za * (uint32_t)c.zb[r];
         }
         out[r] = epi_one<KIND>((int32_t)acc, row.sa, c.sb[r], a.bias ? &c.bias[r] : nullptr, a.relu != 0, p,
                                a.gelu != 0);
@@ -422,7 +423,7 @@ __device__ __forceinline__ void pin_reads_mfmas() {
 // (int8) directly, with no LDS round trip.  The per-column epilogue inputs are loaded
 // after the main loop, so their registers do not compete with the fragment double buffer.
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int NBUF, int KIND>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NBUF, int KIND, bool RAGGED = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N)
 __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N >= 8 ? 2 : 1))) void gemm_i8_dma_kernel(GemmArgs a) {
     typedef DmaTile<BM, BN, WAVES_M, WAVES_N, NBUF> P;
@@ -443,7 +444,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N >= 8 ? 2 : 1))) void gemm_i
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const int nk = a.K / BK;
+    const int nk = (a.K + BK - 1) / BK;
     const EpiParams p = epi_params(a);
 
     // Epilogue inputs of a whole tile (both dimensions in range, unit-stride scales, 16-byte
@@ -487,11 +488,25 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N >= 8 ? 2 : 1))) void gemm_i
         }
     }
     const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>(lds);
+    // RAGGED: K, a multiple of 16, ends inside the last stage.  A's chunks at or past K have bit 31 of
+    // their offset set there, so they lie out of the buffer and read as 0 (B's bytes are multiplied by
+    // 0): one VALU operation per copy.  A variant of its own, because the 256x256 tiles have no register
+    // left: this mask cost whole-stage shapes up to 5%, a branch to it in the loop 20%.
+    uint32_t a_past[RAGGED ? A_I : 1];
+    if constexpr (RAGGED) {
+#pragma unroll
+        for (int j = 0; j < A_I; ++j)
+            a_past[j] = (nk - 1) * BK + (((lane & 7) ^ dma_swz((j * NW + wave) * RPI + (lane >> 3))) * 16) < a.K
+                            ? 0u
+                            : 0x80000000u;
+    }
     auto issue = [&](int buf, int kt) __attribute__((always_inline)) {
         const uint32_t k0 = (uint32_t)(min(kt, nk - 1) * BK);
         const uint32_t sb = lds_base + buf * SB;
+        const uint32_t past = kt >= nk - 1 ? 0x80000000u : 0u;
 #pragma unroll
-        for (int j = 0; j < A_I; ++j) lds_dma16(ra, a_off[j], k0, sb + (j * NW + wave) * RPI * BK);
+        for (int j = 0; j < A_I; ++j)
+            lds_dma16(ra, RAGGED ? a_off[j] | (a_past[RAGGED ? j : 0] & past) : a_off[j], k0, sb + (j * NW + wave) * RPI * BK);
 #pragma unroll
         for (int j = 0; j < B_I; ++j) lds_dma16(rb, b_off[j], k0, sb + BM * BK + (j * NW + wave) * RPI * BK);
     };
@@ -816,7 +831,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N >= 8 ? 2 : 1))) void gemm_i
                         const int nn = min(nc0 + q, a.N - 1);
                         const uint32_t zb = (uint32_t)(int)a.b_zp[nn];
                         accu -= zb * (uint32_t)asum;
-                        accu += (uint32_t)a.K * (uint32_t)p.za * zb;
+                        accu += (uint32_t)a.k_true * (uint32_t)p.za * zb;
                     }
                     if (INT_CODES) {
                         const float sc = rsa[j] * csb[q];
@@ -1458,6 +1473,31 @@ __global__ __launch_bounds__(256) void row_sums_i8_kernel(const int8_t* __restri
     if (lane == 0) sums[r] = s;
 }
 
+// ------------------------------------------------------------ aligned copies
+// Rows of K bytes at any alignment as rows of Kp bytes, a multiple of 16, the tail 0: the vector
+// kernels' form of operands they cannot read in place.  Blocks of a grid row handle A, then B.
+__global__ __launch_bounds__(256) void gemm_align_kernel(const int8_t* __restrict__ A, int64_t lda, int M,
+                                                         const int8_t* __restrict__ B, int64_t ldb, int64_t rows,
+                                                         int K, int Kp, int8_t* __restrict__ dst) {
+    const int per = Kp / 16;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= rows * per) return;
+    const int64_t r = i / per;
+    const int k = (int)(i - r * per) * 16;
+    const int8_t* src = (r < M ? A + r * lda : B + (r - M) * ldb) + k;
+    vu4 v = vu4{0, 0, 0, 0};
+    if (k + 16 <= K) {
+        __builtin_memcpy(&v, src, 16);
+    } else {
+        int8_t t[16] = {};
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            if (k + e < K) t[e] = src[e];  // none when the chunk lies past K
+        __builtin_memcpy(&v, t, 16);
+    }
+    *reinterpret_cast<vu4*>(dst + i * 16) = v;
+}
+
 // ------------------------------------------------------------------- dispatch
 
 // With a.extrema (float32 out): only the LDS-DMA kernels fold their output's extrema, into at
@@ -1472,7 +1512,7 @@ struct GemmLaunch {
         GemmArgs a = a0;
         const bool vec = aligned16(a.A) && aligned16(a.B) && (a.lda % 16 == 0) && (a.ldb % 16 == 0) &&
                          (a.K % 16 == 0);
-        const bool dma_ok = (a.K % 128 == 0) && ((int64_t)(a.M + 256) * a.lda < (int64_t)1 << 31) &&
+        const bool dma_ok = a.K > 0 && ((int64_t)(a.M + 256) * a.lda < (int64_t)1 << 31) &&
                             ((int64_t)(a.N + 256) * a.ldb < (int64_t)1 << 31);
         const int64_t tiles128 = ((int64_t)(a.M + 127) / 128) * ((a.N + 127) / 128);
         if (a.extrema) {
@@ -1512,12 +1552,29 @@ struct GemmLaunch {
             note_path("gemm skinny");
             return launch_status("lq_gemm_w8a8 (skinny)");
         }
-        // LDS-DMA path: whole 128-byte K stages, 32-bit buffer offsets (dma_ok above).
+        // LDS-DMA path: 32-bit buffer offsets (dma_ok above).
         const int64_t dma_tiles = ((int64_t)(a.M + 255) / 256) * ((a.N + 127) / 128);
         // 256x256 tiles (8 waves of 128x64: a third fewer LDS fragment bytes per MFMA) take
         // ~15% less time per op than 256x128 tiles (waves of 64x64) but come in half as many
         // workgroups: compare the two in rounds of 256 workgroups (one per CU).
         const int64_t t256 = ((int64_t)(a.M + 255) / 256) * ((a.N + 255) / 256);
+        // K not whole 128-byte stages: two of the tile shapes (the others gain too little over them to
+        // be compiled twice).  The register-staged 128x128 tiles below took 115 us at M = N = 4096, K = 4032
+        // and 98 us (split-K) at M = 512, N = 4096, K = 1040; these take 75.5 and 9.3 us.
+        if (dma_ok && a.K % 128 != 0 && dma_tiles >= 256) {
+            if (ext_parts) *ext_parts = (int)dma_tiles;
+            hipLaunchKernelGGL((gemm_i8_dma_kernel<256, 128, 4, 2, GEMM_NBUF, KIND, true>), dim3((unsigned)dma_tiles),
+                               dim3(512), 0, st, a);
+            note_path("gemm dma 256x128 ragged k");
+            return launch_status("lq_gemm_w8a8 (dma 256x128 ragged k)");
+        }
+        if (dma_ok && a.K % 128 != 0 && tiles128 >= 128) {
+            if (ext_parts) *ext_parts = (int)tiles128;
+            hipLaunchKernelGGL((gemm_i8_dma_kernel<128, 128, 4, 2, 3, KIND, true>), dim3((unsigned)tiles128),
+                               dim3(512), 0, st, a);
+            note_path("gemm dma 128x128 ragged k");
+            return launch_status("lq_gemm_w8a8 (dma 128x128 ragged k)");
+        }
         if (dma_ok && t256 >= 256 && ((t256 + 255) / 256) * 100 <= ((dma_tiles + 255) / 256) * 57) {
             if (ext_parts) *ext_parts = (int)t256;
             hipLaunchKernelGGL((gemm_i8_dma_kernel<256, 256, 2, 4, GEMM_NBUF, KIND>), dim3((unsigned)t256),
@@ -1583,10 +1640,14 @@ struct GemmLaunch {
 
 static bool valid_out_kind(int k) { return k >= LQ_OUT_I32 && k <= LQ_OUT_QU8S8; }
 
-// Workspace layout: [a_sums M][b_sums N][split partial M*N][tile counters], 256-byte aligned parts.
+// Workspace layout: [a_sums M][b_sums N][split partial M*N][tile counters][aligned copies of A and
+// B], 256-byte aligned parts; `total` is what a call may ask for, `copies` more only makes it faster.
 struct GemmWs {
-    size_t a_sums, b_sums, partial, counters, total;
+    size_t a_sums, b_sums, partial, counters, total, copies;
 };
+// Bytes of a copied row: whole 16-byte chunks, for the tiled kernels' row counts whole 128-byte stages
+// (the zeros cost less there than the masks of a partial stage).
+static int64_t copy_k(int64_t M, int64_t K) { return M > 128 ? (K + 127) / 128 * 128 : (K + 15) / 16 * 16; }
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 static GemmWs gemm_ws(int64_t M, int64_t N, int64_t K) {
     GemmWs w;
@@ -1601,6 +1662,8 @@ static GemmWs gemm_ws(int64_t M, int64_t N, int64_t K) {
     w.counters = w.partial + align256(part);
     const size_t tiles = (size_t)(((M + 127) / 128) * ((N + 127) / 128));
     w.total = w.counters + (may_split ? align256(sizeof(uint32_t) * tiles) : 0);
+    // (a call may still find its operands misaligned with K a multiple of 16: it has no copies then)
+    w.copies = K % 16 && K >= 16 ? align256((size_t)(M + N) * (size_t)copy_k(M, K)) : 0;
     return w;
 }
 
@@ -1641,7 +1704,8 @@ int lq_pack_weights_i8(const int8_t* d_B, int64_t ldb, int64_t N, int64_t K, int
 
 size_t lq_gemm_w8a8_workspace_size(int64_t M, int64_t N, int64_t K) {
     if (M < 0 || N < 0 || K < 0) return 0;
-    return gemm_ws(M, N, K).total;
+    const GemmWs w = gemm_ws(M, N, K);
+    return w.total + w.copies;
 }
 
 }  // extern "C"
@@ -1699,6 +1763,7 @@ static int gemm_entry(bool packed, const int8_t* d_A, int64_t lda, const int8_t*
     a.M = (int)M;
     a.N = (int)N;
     a.K = (int)K;
+    a.k_true = (int)K;
     a.a_scale = d_a_scale;
     a.b_scale = d_b_scale;
     a.a_stride = (int)a_scale_stride;
@@ -1747,6 +1812,21 @@ static int gemm_entry(bool packed, const int8_t* d_A, int64_t lda, const int8_t*
         default: return set_error(LQ_ERR_INVALID, "lq_gemm_w8a8: bad out_kind");
         }
     }
+    // Rows that the vector kernels cannot read (K no multiple of 16) are copied once, 16-byte aligned:
+    // one thread per output reads bytes otherwise.  M = 226, N = 2111, K = 620: 878 -> 30 us; M = 20,
+    // N = 1000, K = 2342: 280 -> 10.6 us; M = N = 4096, K = 4001: 218 ms -> 68 us.  Zero bytes past K add
+    // nothing.
+    if (ws.copies && d_workspace && aligned16(d_workspace) && workspace_bytes >= ws.total + ws.copies) {
+        const int Kp = (int)copy_k(M, K);
+        int8_t* copy = reinterpret_cast<int8_t*>(wsb + ws.total);
+        const int64_t chunks = (M + N) * (int64_t)(Kp / 16);
+        hipLaunchKernelGGL(gemm_align_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, d_A, lda, (int)M, d_B,
+                           ldb, M + N, (int)K, Kp, copy);
+        a.A = copy;
+        a.B = copy + M * Kp;
+        a.lda = a.ldb = a.K = Kp;
+        a.k_true = (int)K;
+    }
     int64_t split_bytes = 0;
     if (d_workspace && workspace_bytes >= ws.total && ws.total > ws.counters) {
         a.partial = (int32_t*)(wsb + ws.partial);
@@ -1783,11 +1863,14 @@ int lq_gemm_w8a8(const int8_t* d_A, int64_t lda, const int8_t* d_B, int64_t ldb,
                       stream);
 }
 
+static size_t dyn_quantize_tail(int64_t M, int64_t N) {
+    const size_t parts = sizeof(int2) * DYN_PARTS_MAX, dq = lq_dynamic_quantize_workspace_size(M * N);
+    return parts > dq ? parts : dq;
+}
+
 size_t lq_gemm_w8a8_dynamic_quantize_workspace_size(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K < 0) return 0;
-    const size_t g = (lq_gemm_w8a8_workspace_size(M, N, K) + 255) & ~(size_t)255;
-    const size_t parts = sizeof(int2) * DYN_PARTS_MAX, dq = lq_dynamic_quantize_workspace_size(M * N);
-    return g + (parts > dq ? parts : dq);
+    return align256(lq_gemm_w8a8_workspace_size(M, N, K)) + dyn_quantize_tail(M, N);
 }
 
 int lq_gemm_w8a8_dynamic_quantize(const int8_t* d_A, int64_t lda, const int8_t* d_B, int64_t ldb, float* d_y,
@@ -1798,9 +1881,10 @@ int lq_gemm_w8a8_dynamic_quantize(const int8_t* d_A, int64_t lda, const int8_t* 
                                   void* d_workspace, size_t workspace_bytes, void* stream) {
     const char* fn = "lq_gemm_w8a8_dynamic_quantize";
     LQ_REQUIRE(M > 0 && N > 0 && d_y && d_qparams && d_codes && qmax > qmin, std::string(fn) + ": bad arguments");
-    LQ_REQUIRE(d_workspace && workspace_bytes >= lq_gemm_w8a8_dynamic_quantize_workspace_size(M, N, K),
+    LQ_REQUIRE(d_workspace && workspace_bytes >= dyn_quantize_tail(M, N) + align256(gemm_ws(M, N, K).total),
                std::string(fn) + ": workspace too small");
-    const size_t g = (lq_gemm_w8a8_workspace_size(M, N, K) + 255) & ~(size_t)255;
+    size_t g = align256(lq_gemm_w8a8_workspace_size(M, N, K));
+    if (workspace_bytes < g + dyn_quantize_tail(M, N)) g = align256(gemm_ws(M, N, K).total);  // no copies
     void* tail = static_cast<char*>(d_workspace) + g;
     const size_t tail_bytes = workspace_bytes - g;
     int2* parts = static_cast<int2*>(tail);
@@ -1864,6 +1948,7 @@ int lq_dynamic_linear_packed_f32(const float* d_x, int64_t ldx, const float* d_r
     a.M = (int)M;
     a.N = (int)N;
     a.K = (int)K;
+    a.k_true = (int)K;
     a.b_scale = d_w_scale;
     a.b_stride = 1;
     a.b_sums = d_w_sums;
@@ -1969,7 +2054,7 @@ int lq_gemm_w8a8_noalloc(const int8_t* d_A, int64_t lda, const int8_t* d_B, int6
                          const int32_t* d_b_sums, const float* d_bias, const float* d_out_scale,
                          const float* d_out_zero_point, int out_qmin, int out_qmax, int out_kind,
                          int flags, void* stream) {
-    const size_t need = lq_gemm_w8a8_workspace_size(M, N, K);
+    const size_t need = M < 0 || N < 0 || K < 0 ? 0 : gemm_ws(M, N, K).total;  // copies: where they fit
     if (need > LQ_NOALLOC_SCRATCH_BYTES)
         return set_error(LQ_ERR_UNSUPPORTED,
                          "lq_gemm_w8a8_noalloc: this shape needs " + std::to_string(need) +

@@ -476,3 +476,36 @@ def test_gemm_dynamic_quantize_equals_calls(gpu, M, N, K, gelu, want):
     np.testing.assert_array_equal(p1.numpy().view(np.uint32), p2.numpy().view(np.uint32))
     yv = y2.numpy()
     np.testing.assert_array_equal(p2.numpy()[:2], np.array([yv.min(), yv.max()], np.float32))
+
+
+# K that is no multiple of 128 (a partial last stage of the LDS-DMA kernels, zeros past K) or of 16
+# (operands copied to aligned rows): each tile size, ragged M and N, one stage only
+@pytest.mark.parametrize("M,N,K,path", [(1000, 2100, 272, "gemm dma 128x128 ragged k"),
+                                        (512, 4096, 1040, "gemm dma 128x128 ragged k"),
+                                        (1500, 2900, 80, "gemm dma 128x128 ragged k"),
+                                        (2100, 4100, 368, "gemm dma 256x128 ragged k"),
+                                        (4000, 4050, 144, "gemm dma 256x128 ragged k"),
+                                        (300, 300, 1008, "gemm 128x128 split-k"),
+                                        (1000, 2100, 271, "gemm dma 128x128 3-stage"),
+                                        (4000, 4050, 127, "gemm dma 256x256"), (226, 2111, 620, "gemm 128x128"),
+                                        (7, 50, 381, "gemm skinny"), (129, 17, 17, "gemm 128x128")])
+def test_ragged_k(gpu, M, N, K, path):
+    """int32 sums and a requantized output with both zero points, bit for bit."""
+    from lucid_amd import _C
+
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    za, zb = 37.0, rng.integers(-3, 4, N).astype(np.float32)
+    acc = run_gemm(gpu, A, B, O.OUT_I32, za=za, zb=zb)
+    assert _C.last_path() == path
+    want = (A.astype(np.int64) - int(za)) @ (B.astype(np.int64) - zb.astype(np.int64)[:, None]).T
+    np.testing.assert_array_equal(acc, want.astype(np.int32))
+    np.testing.assert_array_equal(run_gemm(gpu, A, B, O.OUT_I32, za=za, zb=zb, b_sums=B.astype(np.int32).sum(1)), acc)
+    sa, sb = np.float32(0.01), rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    got = run_gemm(gpu, A, B, O.OUT_QU8S8, a_scale=sa, b_scale=sb, za=za, zb=zb, bias=bias, out_scale=0.05, out_zp=9.0,
+                   qmin=0, qmax=255, relu=True)
+    ref = O.gemm_w8a8(A, B, sa, sb, za=za, zb=zb, bias=bias, out_kind=O.OUT_QU8S8, out_scale=np.float32(0.05), out_zp=9.0,
+                      qmin=0, qmax=255, relu=True)
+    np.testing.assert_array_equal(got, ref)
