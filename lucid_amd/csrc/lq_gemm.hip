@@ -1558,6 +1558,13 @@ struct GemmLaunch {
         // ~15% less time per op than 256x128 tiles (waves of 64x64) but come in half as many
         // workgroups: compare the two in rounds of 256 workgroups (one per CU).
         const int64_t t256 = ((int64_t)(a.M + 255) / 256) * ((a.N + 255) / 256);
+        // Also with fewer tiles than CUs: a tile's chain of stages through LDS (14.6 us at K = 4096) is
+        // shorter than the split-K sums' fills, atomics and last-arriving epilogue: M = 256, N = K = 2048
+        // 62 -> 10.1 us, M = N = 1024, K = 4096 94 -> 14.6 us, M = 300, N = 300, K = 1008 45 -> 11.3 us, and
+        // of the unsplit 128x128 tiles, M = 700, N = 2048, K = 512 22 -> 7.1 us.  At most 16 tiles of a long K
+        // keep the split-K sums, the form that calls without allocation were checked with (M = 256,
+        // N = 1024, K = 4096: 62 us).
+        const bool dma_few = dma_ok && (tiles128 > 16 || a.K < 32 * 128);
         // K not whole 128-byte stages: two of the tile shapes (the others gain too little over them to
         // be compiled twice).  The register-staged 128x128 tiles below took 115 us at M = N = 4096, K = 4032
         // and 98 us (split-K) at M = 512, N = 4096, K = 1040; these take 75.5 and 9.3 us.
@@ -1568,7 +1575,7 @@ struct GemmLaunch {
             note_path("gemm dma 256x128 ragged k");
             return launch_status("lq_gemm_w8a8 (dma 256x128 ragged k)");
         }
-        if (dma_ok && a.K % 128 != 0 && tiles128 >= 128) {
+        if (dma_few && a.K % 128 != 0) {
             if (ext_parts) *ext_parts = (int)tiles128;
             hipLaunchKernelGGL((gemm_i8_dma_kernel<128, 128, 4, 2, 3, KIND, true>), dim3((unsigned)tiles128),
                                dim3(512), 0, st, a);
@@ -1590,7 +1597,7 @@ struct GemmLaunch {
             return launch_status("lq_gemm_w8a8 (dma 256x128)");
         }
         const int64_t dma_tiles_128 = ((int64_t)(a.M + 127) / 128) * ((a.N + 127) / 128);
-        if (dma_ok && dma_tiles_128 >= 128) {
+        if (dma_few) {
             if (ext_parts) *ext_parts = (int)dma_tiles_128;
             // One round of tiles (at most one per CU): the LDS a second workgroup per CU would
             // use goes to a third ring stage (M = 1024, N = K = 4096: 26.6 -> 20.8 us; a fourth

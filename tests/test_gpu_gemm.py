@@ -479,16 +479,19 @@ def test_gemm_dynamic_quantize_equals_calls(gpu, M, N, K, gelu, want):
 
 
 # K that is no multiple of 128 (a partial last stage of the LDS-DMA kernels, zeros past K) or of 16
-# (operands copied to aligned rows): each tile size, ragged M and N, one stage only
+# (operands copied to aligned rows): each tile size, ragged M and N, one stage
+# only, fewer tiles than one per CU
 @pytest.mark.parametrize("M,N,K,path", [(1000, 2100, 272, "gemm dma 128x128 ragged k"),
                                         (512, 4096, 1040, "gemm dma 128x128 ragged k"),
                                         (1500, 2900, 80, "gemm dma 128x128 ragged k"),
                                         (2100, 4100, 368, "gemm dma 256x128 ragged k"),
                                         (4000, 4050, 144, "gemm dma 256x128 ragged k"),
-                                        (300, 300, 1008, "gemm 128x128 split-k"),
+                                        (300, 300, 1008, "gemm dma 128x128 ragged k"),
                                         (1000, 2100, 271, "gemm dma 128x128 3-stage"),
-                                        (4000, 4050, 127, "gemm dma 256x256"), (226, 2111, 620, "gemm 128x128"),
-                                        (7, 50, 381, "gemm skinny"), (129, 17, 17, "gemm 128x128")])
+                                        (4000, 4050, 127, "gemm dma 256x256"), (226, 2111, 620, "gemm dma 128x64"),
+                                        (7, 50, 381, "gemm skinny"), (129, 17, 17, "gemm dma 128x64"),
+                                        (140, 96, 256, "gemm dma 128x64"), (256, 2048, 4096, "gemm dma 128x64"),
+                                        (200, 1000, 4112, "gemm 128x128 split-k")])
 def test_ragged_k(gpu, M, N, K, path):
     """int32 sums and a requantized output with both zero points, bit for bit."""
     from lucid_amd import _C
