@@ -701,6 +701,7 @@ struct WvArgs {
     int M, N, K;
     int G, gs;
     int NC;                  // 16-byte chunks per weight row
+    int nseg;                // segments of a row (group-wise)
     int Kpad;                // staged activation length (J * 64 chunks of codes)
     int xvec;                // activation rows allow 4-element vector loads
 };
@@ -726,42 +727,12 @@ __device__ __forceinline__ uint32_t opaque_and(uint32_t v, uint32_t m) {
     return r;
 }
 
-constexpr bool wv_persistent(bool grouped, int mx, int j) { return !grouped && mx == 1 && j <= 4; }
-
-template <int BITS, bool SIGNED, bool GROUPED, int MX, bool XF32, int J, int HM = LQ_ROUND_NONE>
-__global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
-    // HM: the group scales' rounding (a.hmode as a constant, so the default costs nothing)
-    constexpr int CK = 16 * 8 / BITS;  // codes per 16-byte chunk
-    extern __shared__ __attribute__((aligned(16))) float wv_lds[];
-    float* xs = wv_lds;                                   // [MX][Kpad], swizzled
-    float* gsum = xs + MX * a.Kpad;                       // [MX][G] (group-wise) or [MX] totals
-    constexpr bool PF = wv_persistent(GROUPED, MX, J);  // rows in a loop, the next one prefetched
+// The activations into LDS (xs) and their sums per group or per row (gsum).
+template <bool GROUPED, int MX, bool XF32>
+__device__ __forceinline__ void wv_stage(const WvArgs& a, float* xs, float* gsum) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int waves = blockDim.x >> 6;
-    const int gw = blockIdx.x * waves + wave;  // this wave's first row
-    const int wstride = gridDim.x * waves;
-
-    // every chunk load of a row at once (clamped to the row; chunks past the row meet zero x)
-    auto load_row = [&](int n, vu4* w, float* sgv, float* bgv) {
-        const uint8_t* row = a.w + (int64_t)n * a.ldw_bytes;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int c = min(lane + 64 * j, a.NC - 1);
-            w[j] = __builtin_nontemporal_load(reinterpret_cast<const vu4*>(row) + c);
-            if constexpr (GROUPED) {
-                const int64_t gi = (int64_t)n * a.G + min((lane + 64 * j) * CK / a.gs, a.G - 1);
-                sgv[j] = a.w_scale[gi];  // rounded to x's type where used: a rounding here would
-                bgv[j] = a.g_bias ? a.g_bias[gi] : 0.0f;  // wait for the prefetched row's loads
-            }
-        }
-    };
-    // the first row's loads go out before the activation staging so the two latencies overlap
-    vu4 wc[J];
-    float sg[GROUPED ? J : 1], bg[GROUPED ? J : 1];
-    load_row(min(gw, a.N - 1), wc, sg, bg);
-    __builtin_amdgcn_sched_barrier(0);
-
     // Activation staging in groups of four consecutive k (one 16-byte LDS slot; Kpad is a
     // multiple of 4), up to XU groups per thread with every load issued before any LDS store,
     // so the staging costs one L2 round trip per XU * blockDim.x groups instead of one per
@@ -800,19 +771,30 @@ __global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
 #pragma unroll
         for (int u = 0; u < XU; ++u) {
             const int i = base + u * (int)blockDim.x + tid;
+            if (i - lane >= nq) break;  // the whole wave is past the end
             if (i < nq) {
                 const int m = wv_row<MX>(4 * i, a.Kpad), k = (4 * i) - m * a.Kpad;
                 *reinterpret_cast<vf4*>(xs + m * a.Kpad + wv_slot(k)) = xv4[u];
             }
+            if constexpr (GROUPED) {
+                // the group's 8, 16 or 32 float4 partials are consecutive threads of one wave
+                const int per = a.gs / 4;
+                float v = (xv4[u][0] + xv4[u][1]) + (xv4[u][2] + xv4[u][3]);
+#pragma unroll
+                for (int off = 1; off < 32; off <<= 1)
+                    if (off < per) v += __shfl_xor(v, off, 64);
+                if (i < nq && (i & (per - 1)) == 0) {
+                    const int m = wv_row<MX>(4 * i, a.Kpad), k = (4 * i) - m * a.Kpad;
+                    if (k < a.K) gsum[m * a.G + k / a.gs] = v;  // Kpad is a multiple of gs
+                }
+            }
         }
     }
     __syncthreads();
-    // x sums: per group (group-wise) or per row (zero points), from float4 partials reduced
-    // across the lanes of a group by shuffles, then in fixed order across waves
-    if (GROUPED || a.w_zp) {
-        const int span = GROUPED ? a.gs : a.Kpad;  // elements summed into one value
-        const int per = span / 4;                  // float4 partials per value
-        float* wsum = gsum + (GROUPED ? MX * a.G : MX);  // [waves][MX] (zero-point totals)
+    // row sums (zero points), from float4 partials reduced across a wave by shuffles, then in fixed
+    // order across waves
+    if (!GROUPED && a.w_zp) {
+        float* wsum = gsum + MX;  // [waves][MX]
         for (int i0 = 0; i0 < MX * a.Kpad / 4; i0 += blockDim.x) {
             const int i = i0 + tid;
             float v = 0.0f;
@@ -821,48 +803,66 @@ __global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
                 const vf4 q = *reinterpret_cast<const vf4*>(xs + m * a.Kpad + wv_slot(k));
                 v = (q[0] + q[1]) + (q[2] + q[3]);
             }
-            if (GROUPED) {
-                // per <= 32 lanes of one group are consecutive threads of one wave
 #pragma unroll
-                for (int off = 1; off < 64; off <<= 1)
-                    if (off < per) v += __shfl_xor(v, off, 64);
-                if (i < MX * a.Kpad / 4 && (i % per) == 0) {
-                    const int m = wv_row<MX>(4 * i, a.Kpad), k = (4 * i) - m * a.Kpad;
-                    if (k < a.K) gsum[m * a.G + k / a.gs] = v;  // Kpad is a multiple of gs
-                }
-            } else {
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-                // a wave's 64 partials lie in one row (Kpad is a multiple of 256)
-                if (lane == 0 && i0 + wave * 64 < MX * a.Kpad / 4) {
-                    const int m = wv_row<MX>(4 * (i0 + wave * 64), a.Kpad);
-                    const int slot = (i0 / (int)blockDim.x) * waves + wave;
-                    wsum[slot * MX + m] = v;  // distinct slot per (pass, wave); zero for other rows below
-                }
-            }
-        }
-        if (!GROUPED) {
-            __syncthreads();
-            if (tid < MX) {
-                const int passes = (MX * a.Kpad / 4 + blockDim.x - 1) / blockDim.x;
-                float t = 0.0f;
-                for (int sidx = 0; sidx < passes * waves; ++sidx) {
-                    const int i = (sidx / waves) * blockDim.x + (sidx % waves) * 64;
-                    if (i < MX * a.Kpad / 4 && wv_row<MX>(4 * i, a.Kpad) == tid) t += wsum[sidx * MX + tid];
-                }
-                gsum[tid] = t;
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            // a wave's 64 partials lie in one row (Kpad is a multiple of 256)
+            if (lane == 0 && i0 + wave * 64 < MX * a.Kpad / 4) {
+                const int m = wv_row<MX>(4 * (i0 + wave * 64), a.Kpad);
+                const int slot = (i0 / (int)blockDim.x) * waves + wave;
+                wsum[slot * MX + m] = v;  // distinct slot per (pass, wave); zero for other rows below
             }
         }
         __syncthreads();
+        if (tid < MX) {
+            const int passes = (MX * a.Kpad / 4 + blockDim.x - 1) / blockDim.x;
+            float t = 0.0f;
+            for (int sidx = 0; sidx < passes * waves; ++sidx) {
+                const int i = (sidx / waves) * blockDim.x + (sidx % waves) * 64;
+                if (i < MX * a.Kpad / 4 && wv_row<MX>(4 * i, a.Kpad) == tid) t += wsum[sidx * MX + tid];
+            }
+            gsum[tid] = t;
+        }
+        __syncthreads();
     }
+}
+
+constexpr bool wv_persistent(int mx, int j) { return mx == 1 && j <= 4; }
+
+template <int MX, bool XF32, int J>
+__global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
+    constexpr int CK = 16;  // codes per 16-byte chunk
+    extern __shared__ __attribute__((aligned(16))) float wv_lds[];
+    float* xs = wv_lds;                                   // [MX][Kpad], swizzled
+    float* gsum = xs + MX * a.Kpad;                       // [MX] totals
+    constexpr bool PF = wv_persistent(MX, J);  // rows in a loop, the next one prefetched
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const int waves = blockDim.x >> 6;
+    const int gw = blockIdx.x * waves + wave;  // this wave's first row
+    const int wstride = gridDim.x * waves;
+
+    // every chunk load of a row at once (clamped to the row; chunks past the row meet zero x)
+    auto load_row = [&](int n, vu4* w) {
+        const uint8_t* row = a.w + (int64_t)n * a.ldw_bytes;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int c = min(lane + 64 * j, a.NC - 1);
+            w[j] = __builtin_nontemporal_load(reinterpret_cast<const vu4*>(row) + c);
+        }
+    };
+    // the first row's loads go out before the activation staging so the two latencies overlap
+    vu4 wc[J];
+    load_row(min(gw, a.N - 1), wc);
+    __builtin_amdgcn_sched_barrier(0);
+
+    wv_stage<false, MX, XF32>(a, xs, gsum);
     if (gw >= a.N) return;
 
     for (int n = gw; n < a.N; n += wstride) {
         const int nn = n + wstride;
         const bool more = PF && nn < a.N;  // wave-uniform
         vu4 wn[PF ? J : 1];
-        float sgn[PF && GROUPED ? J : 1], bgn[PF && GROUPED ? J : 1];
-        if (more) load_row(nn, wn, sgn, bgn);
+        if (more) load_row(nn, wn);
         float acc[MX];
 #pragma unroll
         for (int m = 0; m < MX; ++m) acc[m] = 0.0f;
@@ -876,43 +876,19 @@ __global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
 #pragma unroll
             for (int wi = 0; wi < 4; ++wi) {
                 const uint32_t wd = wc[j][wi];
-                float code[32 / BITS];
-                if constexpr (BITS == 8) {
+                float code[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        code[e] = SIGNED ? (float)(signed char)(wd >> (8 * e)) : (float)((wd >> (8 * e)) & 0xFFu);
-                } else {
-                    const uint32_t lo = opaque_and(wd, 0x0F0F0F0Fu);
-                    const uint32_t hi = opaque_and(wd >> 4, 0x0F0F0F0Fu);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        code[2 * e] = (float)((lo >> (8 * e)) & 0xFFu);
-                        code[2 * e + 1] = (float)((hi >> (8 * e)) & 0xFFu);
-                    }
-                }
-                const int kw = k0 + wi * (32 / BITS);
+                for (int e = 0; e < 4; ++e) code[e] = (float)(signed char)(wd >> (8 * e));
+                const int kw = k0 + wi * 4;
 #pragma unroll
                 for (int m = 0; m < MX; ++m) {
+                    const vf4 xv = *reinterpret_cast<const vf4*>(xs + m * a.Kpad + wv_slot(kw));
 #pragma unroll
-                    for (int f = 0; f < 32 / BITS; f += 4) {
-                        const vf4 xv = *reinterpret_cast<const vf4*>(xs + m * a.Kpad + wv_slot(kw + f));
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) p[m] = fmaf(code[f + e], xv[e], p[m]);
-                    }
+                    for (int e = 0; e < 4; ++e) p[m] = fmaf(code[e], xv[e], p[m]);
                 }
             }
-            if constexpr (GROUPED) {
-                const bool first = c < a.NC && (k0 % a.gs) == 0;
-                const int g = min(k0 / a.gs, a.G - 1);
 #pragma unroll
-                for (int m = 0; m < MX; ++m) {
-                    acc[m] = fmaf(round_to(sg[j], HM), p[m], acc[m]);
-                    if (first) acc[m] = fmaf(round_to(bg[j], HM), gsum[m * a.G + g], acc[m]);
-                }
-            } else {
-#pragma unroll
-                for (int m = 0; m < MX; ++m) acc[m] += p[m];
-            }
+            for (int m = 0; m < MX; ++m) acc[m] += p[m];
         }
 #pragma unroll
         for (int m = 0; m < MX; ++m) {
@@ -924,10 +900,8 @@ __global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
             for (int m = 0; m < MX; ++m) {
                 if (m >= a.M) break;
                 float v = acc[m];
-                if constexpr (!GROUPED) {
-                    if (a.w_zp) v = v - a.w_zp[n] * gsum[m];
-                    v = a.w_scale[n] * v;
-                }
+                if (a.w_zp) v = v - a.w_zp[n] * gsum[m];
+                v = a.w_scale[n] * v;
                 v = wo_finish(v, a.bias != nullptr, a.bias ? a.bias[n] : 0.0f, a.relu, a.hmode);
                 if constexpr (XF32)
                     reinterpret_cast<float*>(a.y)[(int64_t)m * a.ldy + n] = v;
@@ -940,10 +914,138 @@ __global__ __launch_bounds__(1024) void wo_gemv_valu_kernel(WvArgs a) {
 #pragma unroll
             for (int j = 0; j < J; ++j) {
                 wc[j] = wn[j];
-                if constexpr (GROUPED) sg[j] = sgn[j], bg[j] = bgn[j];
             }
         }
     }  // rows of this wave
+}
+
+// One or two rows against group-wise weights: the same chunks and sums, over a persistent grid.  A
+// wave's rows are cut into segments of 64 J chunks (J two at 4 bits, four at 8: 4096 codes; one for two rows at 4 bits), and the
+// loads of the next two segments -- of this row or of the wave's next one -- are in flight while one
+// is summed, scales and biases with them.  Nothing else is loaded in the loop and every load goes
+// out unconditionally (past the end: one line, unused), so that no wait reaches past the segment it
+// is for.  The lane's eight (8 bits: four) LDS addresses serve every chunk at a constant distance.
+// N = 11008, K = 4096, groups of 64: 15.0 -> 11.5 us at 4 bits (28 MB of weight), 22.3 -> 14.4 at 8; N = 4096,
+// K = 11008 at 4 bits 18.8 -> 11.8 (on the matrix cores before: its whole row did not fit the registers).
+// What is left is fixed: 5.4 us of a launch, staging and reduction at N = K = 512.
+template <int BITS, int MX, bool XF32, int J, int HM>
+__global__ __launch_bounds__(1024) void wo_gemv_group_kernel(WvArgs a) {
+    // HM: the group scales' rounding (a.hmode as a constant, so the default costs nothing)
+    constexpr int CK = 16 * 8 / BITS;  // codes per 16-byte chunk
+    constexpr int SL = CK / 4;         // LDS slots per chunk
+    extern __shared__ __attribute__((aligned(16))) float wv_lds[];
+    float* xs = wv_lds;              // [MX][Kpad], swizzled
+    float* gsum = xs + MX * a.Kpad;  // [MX][G]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const int gw = blockIdx.x * waves + wave;  // this wave's first row
+    const int wstride = gridDim.x * waves;
+    const int gsh = __builtin_ctz(a.gs);
+    int zero;  // 0 in a vector register: loads through it count with the weight loads, in order
+    __asm__("v_mov_b32 %0, 0" : "=v"(zero));
+    const float* g_bias = a.g_bias ? a.g_bias : a.w_scale;  // (any N G values: unused when null)
+    const float* bias = a.bias ? a.bias : a.w_scale;
+
+    struct Seg {
+        vu4 w[J];
+        float s[J], b[J], bias;
+    };
+    int ln = gw, ls = 0;  // the segment to load next
+    auto load = [&](Seg& t) __attribute__((always_inline)) {
+        const bool in = ln < a.N;
+        const int n = in ? ln : a.N - 1;
+        const vu4* row = reinterpret_cast<const vu4*>(a.w + (int64_t)n * a.ldw_bytes);
+        const float* srow = a.w_scale + (int64_t)n * a.G;
+        const float* brow = g_bias + (int64_t)n * a.G;
+        const int last = in ? a.NC - 1 : 0;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int c = min(lane + 64 * (ls * J + j), last);  // chunks past the row meet zero x
+            t.w[j] = __builtin_nontemporal_load(row + c);
+            const int g = (c * CK) >> gsh;
+            t.s[j] = srow[g];
+            t.b[j] = brow[g];
+        }
+        t.bias = bias[n + zero];
+        if (++ls == a.nseg) ls = 0, ln += wstride;
+    };
+    Seg A, B;
+    load(A);
+    load(B);
+    __builtin_amdgcn_sched_barrier(0);
+    wv_stage<true, MX, XF32>(a, xs, gsum);
+
+    uint32_t slot[SL];  // byte offsets of the lane's slots of chunk `lane`; chunk lane + 64 j: + 1024 SL j
+#pragma unroll
+    for (int i = 0; i < SL; ++i) slot[i] = 4 * wv_slot((lane * SL + i) * 4);
+    float acc[MX] = {};
+    int n = gw, sgm = 0;  // the segment to sum next
+    auto sum = [&](const Seg& t) __attribute__((always_inline)) {
+        const char* xseg = reinterpret_cast<const char*>(xs) + sgm * J * 1024 * SL;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            float p[MX] = {};
+#pragma unroll
+            for (int wi = 0; wi < 4; ++wi) {
+                const uint32_t wd = t.w[j][wi];
+                float code[32 / BITS];
+                if constexpr (BITS == 8) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) code[e] = (float)((wd >> (8 * e)) & 0xFFu);
+                } else {
+                    const uint32_t lo = opaque_and(wd, 0x0F0F0F0Fu);
+                    const uint32_t hi = opaque_and(wd >> 4, 0x0F0F0F0Fu);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        code[2 * e] = (float)((lo >> (8 * e)) & 0xFFu);
+                        code[2 * e + 1] = (float)((hi >> (8 * e)) & 0xFFu);
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < MX; ++m) {
+#pragma unroll
+                    for (int f = 0; f < 8 / BITS; ++f) {
+                        const vf4 xv = *reinterpret_cast<const vf4*>(xseg + (size_t)(4 * m) * a.Kpad +
+                                                                     slot[wi * (8 / BITS) + f] + j * 1024 * SL);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) p[m] = fmaf(code[4 * f + e], xv[e], p[m]);
+                    }
+                }
+            }
+            const int c = lane + 64 * (sgm * J + j), k0 = c * CK;
+            const bool first = c < a.NC && (k0 & (a.gs - 1)) == 0;
+            const int g = min(k0 >> gsh, a.G - 1);
+#pragma unroll
+            for (int m = 0; m < MX; ++m) {
+                acc[m] = fmaf(round_to(t.s[j], HM), p[m], acc[m]);
+                const float gb = a.g_bias ? round_to(t.b[j], HM) : 0.0f;
+                if (first) acc[m] = fmaf(gb, gsum[m * a.G + g], acc[m]);
+            }
+        }
+        if (++sgm != a.nseg) return;
+#pragma unroll
+        for (int m = 0; m < MX; ++m) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) acc[m] += __shfl_xor(acc[m], off, 64);
+            if (lane == 0 && m < a.M) {
+                const float v = wo_finish(acc[m], a.bias != nullptr, t.bias, a.relu, a.hmode);
+                if constexpr (XF32)
+                    reinterpret_cast<float*>(a.y)[(int64_t)m * a.ldy + n] = v;
+                else
+                    reinterpret_cast<_Float16*>(a.y)[(int64_t)m * a.ldy + n] = (_Float16)v;
+            }
+            acc[m] = 0.0f;
+        }
+        sgm = 0;
+        n += wstride;
+    };
+    while (n < a.N) {
+        sum(A);
+        if (n >= a.N) break;
+        load(A);
+        sum(B);
+        load(B);
+    }
 }
 
 // ------------------------------------------------- group-wise quantize / dequantize
@@ -1153,19 +1255,28 @@ int launch_wo(const WoPlan& p, WoArgs a, bool xf32, hipStream_t st, void* ws, si
     return LQ_OK;
 }
 
-// The VALU path: M <= 2, 16-byte aligned rows, at most 16 chunks per lane, staged rows fit
-// 64 KB of LDS.  Returns false when the shape does not qualify.
-template <int BITS, bool SIGNED, bool GROUPED>
-bool launch_wv(WvArgs a, bool xf32, hipStream_t st) {
-    constexpr int CK = 16 * 8 / BITS;
+// The VALU path: M <= 2, 16-byte aligned rows, per-channel at most 16 chunks per lane, staged rows
+// fit 64 KB of LDS.  Returns false when the shape does not qualify.
+bool launch_wv(WvArgs a, bool xf32, int bits, hipStream_t st) {
+    const bool grouped = a.gs != 0;
+    const int CK = 16 * 8 / bits;
     if (a.M > 2) return false;
-    const int64_t row_bytes = (int64_t)a.K * BITS / 8;
+    const int64_t row_bytes = (int64_t)a.K * bits / 8;
     if (row_bytes % 16) return false;
     a.NC = (int)(row_bytes / 16);
     const int Jn = (a.NC + 63) / 64;
-    const int J = Jn <= 1 ? 1 : Jn <= 2 ? 2 : Jn <= 4 ? 4 : Jn <= 8 ? 8 : Jn <= 12 ? 12 : Jn <= 16 ? 16 : 0;
+    int J = Jn <= 1 ? 1 : Jn <= 2 ? 2 : Jn <= 4 ? 4 : Jn <= 8 ? 8 : Jn <= 12 ? 12 : Jn <= 16 ? 16 : 0;
+    a.nseg = 1;
+    if (grouped) {
+        J = std::min(Jn <= 1 ? 1 : Jn <= 2 ? 2 : 4, bits == 8 ? 4 : a.M == 1 ? 2 : 1);  // what 128 registers hold
+        a.nseg = (Jn + J - 1) / J;
+    }
     if (J == 0) return false;
-    a.Kpad = J * 64 * CK;
+    if ((int64_t)a.nseg * J * 64 * CK > 16384) return false;  // 64 KB of one staged row
+    a.Kpad = a.nseg * J * 64 * CK;
+    // two long rows staged by the few waves of a small N: the matrix-core kernel is ahead (N = 1024,
+    // K = 5120 at 4 bits 12.6 us here, 11.0 there; N = 4096, K = 6144: 10.5 against 13.6)
+    if (grouped && a.M == 2 && a.N < 4096 && a.Kpad > 4096) return false;
     {
         const int eb = xf32 ? 4 : 2;  // element bytes; a 4-element load needs 4 * eb alignment
         a.xvec = (reinterpret_cast<uintptr_t>(a.x) % (4 * eb) == 0) && ((a.ldx * eb) % (4 * eb) == 0);
@@ -1174,50 +1285,54 @@ bool launch_wv(WvArgs a, bool xf32, hipStream_t st) {
     const int waves = a.N >= 4096 ? 16 : std::max(1, (a.N + 255) / 256);
     const size_t passes = ((size_t)MX * a.Kpad / 4 + 64 * waves - 1) / (64 * waves);
     const size_t lds = sizeof(float) * ((size_t)MX * a.Kpad +
-                                        (GROUPED ? (size_t)MX * a.G : (size_t)MX + passes * waves * MX));
+                                        (grouped ? (size_t)MX * a.G : (size_t)MX + passes * waves * MX));
     if (lds > 64 * 1024) return false;
     const int64_t row_groups = (a.N + waves - 1) / waves;
-    const bool persist = wv_persistent(GROUPED, MX, J);  // at most one workgroup per CU
+    const bool persist = grouped || wv_persistent(MX, J);  // at most one workgroup per CU
     const dim3 grid((unsigned)(persist ? std::min<int64_t>(row_groups, device_cu_count()) : row_groups));
     const dim3 block(64 * waves);
-    // (instantiated only for the chunk counts whose registers fit: group scales of 12+ chunks,
-    // or of 8 chunks at 4 bits and two rows, would spill)
-    auto go = [&](auto mx, auto xf, auto jv) {
-        constexpr int MXV = decltype(mx)::value, JV = decltype(jv)::value;
+    auto with = [&](auto mx, auto xf) {
+        constexpr int MXV = decltype(mx)::value;
         constexpr bool XV = decltype(xf)::value;
-        constexpr bool fits = !GROUPED || (JV <= 8 && !(BITS == 4 && MXV == 2 && JV > 4));
-        if constexpr (fits) {
-            // group scales rounded to x's type: half x always, bfloat16 on request
-            if constexpr (GROUPED && !XV)
-                hipLaunchKernelGGL((wo_gemv_valu_kernel<BITS, SIGNED, GROUPED, MXV, XV, JV, LQ_ROUND_F16>), grid,
-                                   block, lds, st, a);
-            else if (GROUPED && a.hmode == LQ_ROUND_BF16)
-                hipLaunchKernelGGL((wo_gemv_valu_kernel<BITS, SIGNED, GROUPED, MXV, XV, JV, LQ_ROUND_BF16>), grid,
-                                   block, lds, st, a);
-            else
-                hipLaunchKernelGGL((wo_gemv_valu_kernel<BITS, SIGNED, GROUPED, MXV, XV, JV>), grid, block, lds, st, a);
-            note_path("wo valu");
-            return true;
+        if (grouped) {
+            auto group = [&](auto bv, auto jv) {
+                constexpr int BV = decltype(bv)::value, JV = decltype(jv)::value;
+                // group scales rounded to x's type: half x always, bfloat16 on request
+                if constexpr (!XV)
+                    hipLaunchKernelGGL((wo_gemv_group_kernel<BV, MXV, XV, JV, LQ_ROUND_F16>), grid, block, lds, st, a);
+                else if (a.hmode == LQ_ROUND_BF16)
+                    hipLaunchKernelGGL((wo_gemv_group_kernel<BV, MXV, XV, JV, LQ_ROUND_BF16>), grid, block, lds, st, a);
+                else
+                    hipLaunchKernelGGL((wo_gemv_group_kernel<BV, MXV, XV, JV, LQ_ROUND_NONE>), grid, block, lds, st, a);
+            };
+            if (bits == 4) {
+                if (J == 1) group(std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{});
+                else if constexpr (MXV == 1) group(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+            } else {
+                if (J == 1) group(std::integral_constant<int, 8>{}, std::integral_constant<int, 1>{});
+                else if (J == 2) group(std::integral_constant<int, 8>{}, std::integral_constant<int, 2>{});
+                else group(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+            }
         } else {
-            return false;
+            auto go = [&](auto jv) {
+                hipLaunchKernelGGL((wo_gemv_valu_kernel<MXV, XV, decltype(jv)::value>), grid, block, lds, st, a);
+            };
+            switch (J) {
+                case 1: go(std::integral_constant<int, 1>{}); break;
+                case 2: go(std::integral_constant<int, 2>{}); break;
+                case 4: go(std::integral_constant<int, 4>{}); break;
+                case 8: go(std::integral_constant<int, 8>{}); break;
+                case 12: go(std::integral_constant<int, 12>{}); break;
+                default: go(std::integral_constant<int, 16>{});
+            }
         }
-    };
-    auto by_j = [&](auto mx, auto xf) {
-        switch (J) {
-            case 1: return go(mx, xf, std::integral_constant<int, 1>{});
-            case 2: return go(mx, xf, std::integral_constant<int, 2>{});
-            case 4: return go(mx, xf, std::integral_constant<int, 4>{});
-            case 8: return go(mx, xf, std::integral_constant<int, 8>{});
-            case 12: return go(mx, xf, std::integral_constant<int, 12>{});
-            default: return go(mx, xf, std::integral_constant<int, 16>{});
-        }
+        note_path("wo valu");
     };
     using T1 = std::integral_constant<int, 1>;
     using T2 = std::integral_constant<int, 2>;
-    using F32 = std::integral_constant<bool, true>;
-    using F16 = std::integral_constant<bool, false>;
-    if (MX == 1) return xf32 ? by_j(T1{}, F32{}) : by_j(T1{}, F16{});
-    return xf32 ? by_j(T2{}, F32{}) : by_j(T2{}, F16{});
+    if (MX == 1) xf32 ? with(T1{}, std::true_type{}) : with(T1{}, std::false_type{});
+    else xf32 ? with(T2{}, std::true_type{}) : with(T2{}, std::false_type{});
+    return true;
 }
 
 // The same call for the tiled kernel (gs 0: per-channel).
@@ -1277,7 +1392,7 @@ int lq_gemv_w8(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d_W, int
         v.x = d_x; v.ldx = ldx; v.w = a.w; v.ldw_bytes = ldw; v.w_scale = d_w_scale;
         v.w_zp = d_w_zero_point; v.bias = d_bias; v.y = d_y; v.ldy = ldy; v.relu = a.relu;
         v.M = (int)M; v.N = (int)N; v.K = (int)K;
-        if (launch_wv<8, true, false>(v, xf32, st)) return launch_status("lq_gemv_w8");
+        if (launch_wv(v, xf32, 8, st)) return launch_status("lq_gemv_w8");
     }
     if (sk_preferred(a) && sk_fits(a, xf32, 2, d_workspace, workspace_bytes)) {
         const int rc = launch_sk<8, true, 2, false>(a, xf32, st, d_workspace);
@@ -1411,8 +1526,7 @@ int lq_group_matmul(const void* d_x, int x_dtype, int64_t ldx, const uint32_t* d
         v.x = d_x; v.ldx = ldx; v.w = a.w; v.ldw_bytes = a.ldw_bytes; v.w_scale = d_scales;
         v.g_bias = d_biases; v.bias = d_bias; v.y = d_y; v.ldy = ldy; v.relu = a.relu; v.hmode = hmode;
         v.M = (int)M; v.N = (int)N; v.K = (int)K; v.G = a.G; v.gs = group_size;
-        const bool ok = bits == 8 ? launch_wv<8, false, true>(v, xf32, st) : launch_wv<4, false, true>(v, xf32, st);
-        if (ok) return launch_status("lq_group_matmul");
+        if (launch_wv(v, xf32, bits, st)) return launch_status("lq_group_matmul");
     }
     if (sk_preferred(a) && sk_fits(a, xf32, S, d_workspace, workspace_bytes)) {
         int rc;

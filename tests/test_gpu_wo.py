@@ -791,3 +791,53 @@ def test_quantized_linear_mlx_module_bf16(gpu):
     mag = np.maximum(np.maximum(np.abs(got), np.abs(want)), np.abs(pre))
     assert np.max(np.abs(got - want) / _ulp(mag, "bf16")) <= 1.0
 
+
+
+# (M, N, K, bits, group size): one, two and three segments of a row, partial last chunks, more
+# rows than waves, a wave with one row and none
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N,K,bits,gs", [(1, 5, 32, 4, 32), (1, 4100, 4096, 4, 64), (1, 300, 4160, 4, 32),
+                                           (1, 9000, 1056, 8, 32), (1, 257, 11008, 4, 128), (1, 130, 11008, 8, 64),
+                                           (2, 4099, 2176, 4, 128), (2, 4101, 6144, 4, 64), (2, 513, 2304, 8, 128)])
+def test_group_matmul_rows_in_segments(gpu, M, N, K, bits, gs, half):
+    """One or two rows against the float64 product: within 2^-18 of the terms' absolute sum, 64 float32
+    roundings.  A term meets at most 61: 32 codes of a chunk, two for each of a lane's chunks (11 of
+    16 codes), six between the lanes, or the seven of a group's sum and its product with the bias.
+    A float16 result adds half of its last place."""
+    from lucid_amd import _C
+    from lucid_amd.quantization import _qgemm
+
+    rng = np.random.default_rng(M + N + K + bits)
+    x = rng.standard_normal((M, K)).astype(np.float16 if half else np.float32)
+    packed, scales, biases = _qgemm.quantize(_t(gpu, rng.standard_normal((N, K)).astype(np.float32)), group_size=gs,
+                                             bits=bits)
+    sc, bi = scales.numpy(), biases.numpy()
+    if half:
+        sc, bi = sc.astype(np.float16).astype(np.float64), bi.astype(np.float16).astype(np.float64)
+    g = lambda v: np.repeat(v.astype(np.float64), gs, axis=1)  # noqa: E731
+    codes = O.group_codes(packed.numpy().view(np.uint32), bits).astype(np.float64).reshape(N, K)
+    wd = codes * g(sc) + g(bi)
+    y = _qgemm.quantized_matmul(_t(gpu, x), packed, scales, biases, transpose=True, group_size=gs, bits=bits).numpy()
+    assert _C.last_path() == "wo valu"
+    # codes and group biases are summed apart, so their terms' magnitudes count, not w_hat's
+    mag = np.abs(x.astype(np.float64)) @ (codes * np.abs(g(sc)) + np.abs(g(bi))).T
+    ref = x.astype(np.float64) @ wd.T
+    assert np.all(np.abs(y - ref) <= mag * 2.0**-18 + (np.abs(ref) * 2.0**-11 if half else 0.0))
+
+
+# lq_gemv_w8_packed in one pass: K ranges of one to eight waves, a last block or wave that is partial,
+# more than one K range, fewer columns than a tile and more tiles than CUs
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 7, 64), (3, 17, 512), (16, 4100, 1040), (9, 8200, 2064), (16, 300, 4080),
+                                   (2, 48, 4112), (16, 33, 8208)])
+def test_gemv_w8_packed_one_pass(gpu, M, N, K, half):
+    rng = np.random.default_rng(M * 7 + N + K + half)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[:, ::53] *= 30.0
+    W = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    s = rng.uniform(1e-3, 1e-2 if half else 1e-1, N).astype(np.float32)
+    z = rng.integers(-4, 5, N).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    xr = x.astype(np.float16).astype(np.float32) if half else x
+    got = run_gemv_packed(gpu, x, W, s, z=z, b=b, half=half)
+    _close(got, _gemv_ref(xr, W, s, z=z, b=b), half=half)
