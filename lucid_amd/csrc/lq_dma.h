@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lq_extent.h"
+
 namespace lq {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -42,6 +44,12 @@ __device__ __forceinline__ v4i buffer_rsrc(const void* base, uint32_t bytes) {
     return v4i{__builtin_amdgcn_readfirstlane((int)(uint32_t)b),
                __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)),
                __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000};
+}
+
+// Descriptor of a row-major operand's own bytes (below 2^31).  A copy's address is in range if voff plus the
+// scalar offset is (the hardware compares voff with num_records - soff); anything else reads as 0.
+__device__ __forceinline__ v4i operand_rsrc(const void* base, int64_t rows, int64_t ld, int64_t width) {
+    return buffer_rsrc(base, (uint32_t)operand_bytes(rows, ld, width));
 }
 
 // 16 bytes per lane from rsrc + voff + soff into LDS at lds_addr + 16 * lane.  The LDS

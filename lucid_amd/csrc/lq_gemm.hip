@@ -469,8 +469,10 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N >= 8 ? 2 : 1))) void gemm_i
         }
     }
 
-    const v4i ra = buffer_rsrc(a.A, (uint32_t)((int64_t)a.M * a.lda));
-    const v4i rb = buffer_rsrc(a.B, (uint32_t)((int64_t)a.N * a.ldb));
+    // Rows past M / N lie out of the buffers and read as 0, and so do the chunks past K of the last row
+    // of each (K, lda and ldb are multiples of 16: no chunk straddles the end).
+    const v4i ra = operand_rsrc(a.A, a.M, a.lda, a.K);
+    const v4i rb = operand_rsrc(a.B, a.N, a.ldb, a.K);
     // Lane l of a copy moves chunk slot l % 8 of row l / 8 of its 8-row block: the global
     // chunk (l % 8) ^ dma_swz(row).
     uint32_t a_off[A_I], b_off[B_I];
@@ -489,9 +491,10 @@ __attribute__((amdgpu_waves_per_eu(WAVES_M * WAVES_N >= 8 ? 2 : 1))) void gemm_i
     }
     const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>(lds);
     // RAGGED: K, a multiple of 16, ends inside the last stage.  A's chunks at or past K have bit 31 of
-    // their offset set there, so they lie out of the buffer and read as 0 (B's bytes are multiplied by
-    // 0): one VALU operation per copy.  A variant of its own, because the 256x256 tiles have no register
-    // left: this mask cost whole-stage shapes up to 5%, a branch to it in the loop 20%.
+    // their offset set there, so they lie out of the buffer and read as 0; B's (bytes between its rows, of
+    // its next row, or out of the buffer) are multiplied by 0: one VALU operation per copy.  A variant of
+    // its own, because the 256x256 tiles have no register left: this mask cost whole-stage shapes up to
+    // 5%, a branch to it in the loop 20%.
     uint32_t a_past[RAGGED ? A_I : 1];
     if constexpr (RAGGED) {
 #pragma unroll

@@ -512,3 +512,43 @@ def test_ragged_k(gpu, M, N, K, path):
     ref = O.gemm_w8a8(A, B, sa, sb, za=za, zb=zb, bias=bias, out_kind=O.OUT_QU8S8, out_scale=np.float32(0.05), out_zp=9.0,
                       qmin=0, qmax=255, relu=True)
     np.testing.assert_array_equal(got, ref)
+
+
+def _column_slice(L, rows, ld, off, codes, pad):
+    """`codes` [rows, K] as columns off .. off + K of a matrix of `ld` columns filled with `pad`, whose
+    allocation ends with the last row's last code; (tensor, address of the first code)."""
+    K = codes.shape[1]
+    flat = np.full((rows * ld,), pad, np.int8)
+    flat.reshape(rows, ld)[:, off:off + K] = codes
+    t = _dev(L, flat[:(rows - 1) * ld + off + K])
+    return t, t.data_ptr() + off
+
+
+@pytest.mark.parametrize("M,N,K,lda,ldb,off,path",
+                         [(300, 300, 144, 288, 272, 128, "gemm dma 128x128 ragged k"),
+                          (2100, 4100, 368, 640, 512, 16, "gemm dma 256x128 ragged k"),
+                          (512, 1100, 128, 256, 384, 112, "gemm dma 128x64"),
+                          (300, 300, 143, 288, 272, 128, "gemm dma 128x64"),      # K no multiple of 16: copied
+                          (300, 300, 143, 167, 181, 5, "gemm dma 128x64"),        # and at any alignment
+                          (33, 200, 77, 99, 101, 3, "gemm skinny"),
+                          (140, 130, 144, 160, 176, 1, "gemm generic")])          # misaligned, K a multiple of 16
+def test_column_slices(gpu, M, N, K, lda, ldb, off, path):
+    """Operands that are column slices of wider matrices and end with their last code: int32 sums bit
+    for bit, whatever lies between the rows."""
+    from lucid_amd import _C
+
+    rng = np.random.default_rng(M + K + off)
+    A, B = _codes(rng, (M, K), -128), _codes(rng, (N, K), -128)
+    want = O.gemm_acc(A, B)
+    ws_bytes = _C.lib().lq_gemm_w8a8_workspace_size(M, N, K)
+    ws = gpu.empty((ws_bytes,), np.uint8, "gpu")
+    for pad in (127, -128):
+        ta, pa = _column_slice(gpu, M, lda, off, A, pad)
+        tb, pb = _column_slice(gpu, N, ldb, off, B, pad)
+        C = gpu.empty((M, N), np.int32, "gpu")
+        print(f"column slices M={M} N={N} K={K} lda={lda} ldb={ldb} off={off}", flush=True)
+        _C.call("lq_gemm_w8a8", pa, lda, pb, ldb, C.data_ptr(), N, M, N, K, None, 0, None, 0, None, None, None, None,
+                None, None, -128, 127, O.OUT_I32, 0, ws.data_ptr(), ws_bytes, None)
+        assert _C.last_path() == path
+        np.testing.assert_array_equal(C.numpy(), want)
+        del ta, tb
