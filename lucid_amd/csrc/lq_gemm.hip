@@ -1099,9 +1099,10 @@ __global__ __launch_bounds__(256) void gemm_i8_decode_partial_kernel(GemmArgs a,
     // in issue order, so vmcnt(DEC_MAX_KS) means this wave's A copies have landed while the
     // weights are still streaming, and each k-step below starts as soon as its weight is in.
     // A slice: MT*16 rows x `slots` chunks, copied 64 chunks (1 KB) per wave instruction.
-    // LDS slot g = row * slots + s holds global chunk c = s ^ (row % 16) of the row (rows
-    // past M read as zeros through the buffer bound; chunks past the split's K are never read).
-    const v4i ra = buffer_rsrc(a.A, (uint32_t)((int64_t)a.M * a.lda));
+    // LDS slot g = row * slots + s holds global chunk c = s ^ (row % 16) of the row (rows past M and the
+    // last row's chunks past K read as zeros through the buffer bound; other chunks past K are never
+    // used, or meet the zeros the weight is packed with).
+    const v4i ra = operand_rsrc(a.A, a.M, a.lda, a.K);
     const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>(As);
     const int copies = MT * 16 * slots / 64;
     for (int q = wave; q < copies; q += 4) {

@@ -552,3 +552,22 @@ def test_column_slices(gpu, M, N, K, lda, ldb, off, path):
         assert _C.last_path() == path
         np.testing.assert_array_equal(C.numpy(), want)
         del ta, tb
+
+
+@pytest.mark.parametrize("M,N,K,lda,off", [(48, 512, 1040, 1168, 128), (100, 1030, 144, 400, 256), (128, 64, 4096, 4112, 16)])
+def test_packed_column_slice(gpu, M, N, K, lda, off):
+    """The decode kernel over activations that are a column slice ending with their last code."""
+    from lucid_amd import _C
+
+    rng = np.random.default_rng(M + K)
+    A, B = _codes(rng, (M, K), -128), _codes(rng, (N, K), -128)
+    packed = pack_weights(gpu, B)
+    ws_bytes = _C.lib().lq_gemm_w8a8_workspace_size(M, N, K)
+    ws = gpu.empty((ws_bytes,), np.uint8, "gpu")
+    for pad in (127, -128):
+        ta, pa = _column_slice(gpu, M, lda, off, A, pad)
+        C = gpu.empty((M, N), np.int32, "gpu")
+        _C.call("lq_gemm_w8a8_packed", pa, lda, packed.data_ptr(), C.data_ptr(), N, M, N, K, None, 0, None, 0, None, None,
+                None, None, None, None, -128, 127, O.OUT_I32, 0, ws.data_ptr(), ws_bytes, None)
+        np.testing.assert_array_equal(C.numpy(), O.gemm_acc(A, B))
+        del ta

@@ -25,9 +25,10 @@ def test_copies_stay_in_the_operand(tmp_path):
     assert out.stdout.strip() == "ok"
 
 
-def test_gemm_tiles_bound_their_operands_by_it():
+@pytest.mark.parametrize("kernel,operands", [("gemm_i8_dma_kernel", "AB"), ("gemm_i8_decode_partial_kernel", "A")])
+def test_gemm_kernels_bound_their_operands_by_it(kernel, operands):
     text = open(os.path.join(CSRC, "lq_gemm.hip")).read()
-    kernel = text[text.index("void gemm_i8_dma_kernel"):]
-    kernel = kernel[:kernel.index("__global__")]
-    made = dict(re.findall(r"const v4i (r[ab]) = operand_rsrc\(a\.([AB]), ", kernel))
-    assert made == {"ra": "A", "rb": "B"}
+    body = text[text.index(f"void {kernel}"):]
+    body = body[:body.index("__global__")]
+    made = dict(re.findall(r"const v4i (r[ab]) = operand_rsrc\(a\.([AB]), ", body))
+    assert made == {"r" + o.lower(): o for o in operands}
