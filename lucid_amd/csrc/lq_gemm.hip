@@ -400,11 +400,11 @@ __device__ __forceinline__ void pin_reads_mfmas() {
 
 // --------------------------------------------- LDS-DMA MFMA main loop (large M)
 //
-// The production path for M > 64 when K % 128 == 0.  Global -> LDS copies use the LDS-DMA
+// The production path for M > 64.  Global -> LDS copies use the LDS-DMA
 // form of buffer_load_dwordx4 (data goes straight to LDS, no staging registers): each wave
 // instruction moves 1 KB = 8 rows x 128 K-bytes of A or B into the next stage's buffer.
-// Buffer descriptors bound A and B to M*lda and N*ldb bytes, so rows past M or N read as
-// zero (their outputs are never stored) and no per-row predicates are needed.
+// Buffer descriptors end with the last rows of A and B, so rows past M or N read as zero
+// (their outputs are never stored) and no per-row predicates are needed.
 //
 // A ring of NBUF LDS stages of BK = 128: stage kt+NBUF is issued right after the barrier
 // that retires stage kt, and waited for (vmcnt) NBUF - 1 stages later.  Inside a stage the two 64-byte K steps
@@ -1562,13 +1562,16 @@ struct GemmLaunch {
         // ~15% less time per op than 256x128 tiles (waves of 64x64) but come in half as many
         // workgroups: compare the two in rounds of 256 workgroups (one per CU).
         const int64_t t256 = ((int64_t)(a.M + 255) / 256) * ((a.N + 255) / 256);
-        // Also with fewer tiles than CUs: a tile's chain of stages through LDS (14.6 us at K = 4096) is
-        // shorter than the split-K sums' fills, atomics and last-arriving epilogue: M = 256, N = K = 2048
-        // 62 -> 10.1 us, M = N = 1024, K = 4096 94 -> 14.6 us, M = 300, N = 300, K = 1008 45 -> 11.3 us, and
-        // of the unsplit 128x128 tiles, M = 700, N = 2048, K = 512 22 -> 7.1 us.  At most 16 tiles of a long K
-        // keep the split-K sums, the form that calls without allocation were checked with (M = 256,
-        // N = 1024, K = 4096: 62 us).
-        const bool dma_few = dma_ok && (tiles128 > 16 || a.K < 32 * 128);
+        // Also with fewer tiles than CUs: a tile's chain of stages through LDS (14 us at K = 4096, 2 us per 1024
+        // more) is shorter than the split-K sums' fills, atomics and last-arriving epilogue (36-60 us there):
+        // M = 256, N = K = 2048 62 -> 10.1 us, M = N = 1024, K = 4096 94 -> 14.6 us, M = 256, N = 1024, K = 4096
+        // 56 -> 14 us, M = 300, N = 300, K = 1008 45 -> 11.3 us, and of the unsplit 128x128 tiles, M = 700,
+        // N = 2048, K = 512 22 -> 7.1 us.  Only the longest K give the sums enough to split: at K = 32768 one or
+        // two tiles (M = 129, N = 128: 52 against 68 us; four tiles 70 against 69), from K = 65536 up to 32
+        // (M = 129, N = 2048: 131 against 149; 64 tiles 220 against 191).
+        const bool split_long = workspace_split_bytes > 0 && a.K >= 32768 &&
+                                (tiles128 <= 2 || (a.K >= 65536 && tiles128 <= 32));
+        const bool dma_few = dma_ok && !split_long;
         // K not whole 128-byte stages: two of the tile shapes (the others gain too little over them to
         // be compiled twice).  The register-staged 128x128 tiles below took 115 us at M = N = 4096, K = 4032
         // and 98 us (split-K) at M = 512, N = 4096, K = 1040; these take 75.5 and 9.3 us.

@@ -491,7 +491,10 @@ def test_gemm_dynamic_quantize_equals_calls(gpu, M, N, K, gelu, want):
                                         (4000, 4050, 127, "gemm dma 256x256"), (226, 2111, 620, "gemm dma 128x64"),
                                         (7, 50, 381, "gemm skinny"), (129, 17, 17, "gemm dma 128x64"),
                                         (140, 96, 256, "gemm dma 128x64"), (256, 2048, 4096, "gemm dma 128x64"),
-                                        (200, 1000, 4112, "gemm 128x128 split-k")])
+                                        (200, 1000, 4112, "gemm dma 128x128 ragged k"),
+                                        (256, 1024, 4096, "gemm dma 128x64"), (129, 120, 16384, "gemm dma 128x64"),
+                                        (130, 100, 32784, "gemm 128x128 split-k"), (130, 300, 32768, "gemm dma 128x64"),
+                                        (130, 130, 65552, "gemm 128x128 split-k")])
 def test_ragged_k(gpu, M, N, K, path):
     """int32 sums and a requantized output with both zero points, bit for bit."""
     from lucid_amd import _C

@@ -62,12 +62,14 @@ def _case(rng, M, N, K, with_zb):
 @pytest.mark.parametrize("kind", [O.OUT_Q8, O.OUT_F32])
 def test_noalloc_matches_workspace_entry_point(gpu, kind):
     rng = np.random.default_rng(77 + kind)
-    # 1: split-K 128x128 tiles (few tiles, long K), activation and weight zero points:
-    #    code sums and split partials / counters all in the scratch
+    # 1: split-K 128x128 tiles (two tiles of the longest K: the shapes that kernel is the faster one
+    #    for), activation and weight zero points: code sums and split partials / counters all in
+    #    the scratch
     # 2: a smaller call right after (activation zero point only, skinny kernel)
     # 3: the first shape again after a different-sized use of the scratch
-    shapes = [(200, 1024, 4096, True, "gemm 128x128 split-k"), (48, 520, 1024, False, "gemm skinny"),
-              (200, 1024, 4096, True, "gemm 128x128 split-k")]
+    # 4: the LDS-DMA tiles with both code sums
+    shapes = [(200, 100, 32768, True, "gemm 128x128 split-k"), (48, 520, 1024, False, "gemm skinny"),
+              (200, 100, 32768, True, "gemm 128x128 split-k"), (200, 1024, 4096, True, "gemm dma 128x64")]
     for M, N, K, with_zb, path in shapes:
         A, B, sa, sb, za, zb, bias = _case(rng, M, N, K, with_zb)
         print(f"noalloc M={M} N={N} K={K} kind={kind}", flush=True)
