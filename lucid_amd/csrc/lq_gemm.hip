@@ -1662,6 +1662,13 @@ struct GemmWs {
 // Bytes of a copied row: whole 16-byte chunks, for the tiled kernels' row counts whole 128-byte stages
 // (the zeros cost less there than the masks of a partial stage).
 static int64_t copy_k(int64_t M, int64_t K) { return M > 128 ? (K + 127) / 128 * 128 : (K + 15) / 16 * 16; }
+// Whether rows of a K that is no multiple of 16 are copied.  The kernel that reads them as they are runs
+// one thread per output over bytes: for a short K it ends before the copy's own launch would (N = 64: K = 17
+// 3.3 us against 5.3, K = 30 4.1 against 5.8, K = 65 7.0 against 5.4; above 64 rows 7.2 against 7.8), unless
+// the outputs are many (M = 129, N = 4096, K = 17 9.2 against 8.5; M = 64 5.4 against 6.9).
+static bool copies_pay(int64_t M, int64_t N, int64_t K) {
+    return K % 16 && K >= 16 && (K >= (M > 64 ? 72 : 56) || M * N >= ((int64_t)1 << 23) / K);
+}
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 static GemmWs gemm_ws(int64_t M, int64_t N, int64_t K) {
     GemmWs w;
@@ -1677,7 +1684,7 @@ static GemmWs gemm_ws(int64_t M, int64_t N, int64_t K) {
     const size_t tiles = (size_t)(((M + 127) / 128) * ((N + 127) / 128));
     w.total = w.counters + (may_split ? align256(sizeof(uint32_t) * tiles) : 0);
     // (a call may still find its operands misaligned with K a multiple of 16: it has no copies then)
-    w.copies = K % 16 && K >= 16 ? align256((size_t)(M + N) * (size_t)copy_k(M, K)) : 0;
+    w.copies = copies_pay(M, N, K) ? align256((size_t)(M + N) * (size_t)copy_k(M, K)) : 0;
     return w;
 }
 

@@ -489,7 +489,9 @@ def test_gemm_dynamic_quantize_equals_calls(gpu, M, N, K, gelu, want):
                                         (300, 300, 1008, "gemm dma 128x128 ragged k"),
                                         (1000, 2100, 271, "gemm dma 128x128 3-stage"),
                                         (4000, 4050, 127, "gemm dma 256x256"), (226, 2111, 620, "gemm dma 128x64"),
-                                        (7, 50, 381, "gemm skinny"), (129, 17, 17, "gemm dma 128x64"),
+                                        (7, 50, 381, "gemm skinny"), (129, 17, 17, "gemm generic"),
+                                        (129, 4096, 17, "gemm dma 128x64"), (3, 70, 57, "gemm skinny"), (3, 70, 55, "gemm generic"),
+                                        (65, 70, 71, "gemm generic"), (65, 70, 73, "gemm skinny"),
                                         (140, 96, 256, "gemm dma 128x64"), (256, 2048, 4096, "gemm dma 128x64"),
                                         (200, 1000, 4112, "gemm dma 128x128 ragged k"),
                                         (256, 1024, 4096, "gemm dma 128x64"), (129, 120, 16384, "gemm dma 128x64"),
@@ -534,6 +536,7 @@ def _column_slice(L, rows, ld, off, codes, pad):
                           (300, 300, 143, 288, 272, 128, "gemm dma 128x64"),      # K no multiple of 16: copied
                           (300, 300, 143, 167, 181, 5, "gemm dma 128x64"),        # and at any alignment
                           (33, 200, 77, 99, 101, 3, "gemm skinny"),
+                         (33, 200, 30, 99, 101, 3, "gemm generic"),              # too short to copy
                           (140, 130, 144, 160, 176, 1, "gemm generic")])          # misaligned, K a multiple of 16
 def test_column_slices(gpu, M, N, K, lda, ldb, off, path):
     """Operands that are column slices of wider matrices and end with their last code: int32 sums bit
