@@ -1,31 +1,35 @@
 // lq_wo_nt.hip -- y[m, k] = sum_n x[m, n] w_hat[n, k] for group-wise packed w_hat[N, K] (groups
 // along k): quantized_matmul with transpose=false and the input gradient of the transpose=true
 // product, dX = dY dequant(W) (QuantizedMatmulBackward::apply,
-// lucid/_C/ops/quantized/QuantizedMatmul.cpp:73-90), on v_mfma_f32_16x16x32_f16.
+// lucid/_C/ops/quantized/QuantizedMatmul.cpp:73-90), on the matrix cores.
 //
 // The group scale and bias change along the summed axis, so they cannot be taken out of the sums:
-// w_hat is formed per element, w = fma(c, s, b) in fp32, and both operands enter the MFMA as two
-// fp16 terms hi + lo (~22 significant bits): x w = hi hi + lo hi + hi lo, fp32 accumulation (half x
-// is its own hi term: two products).  Nothing is prepared in memory (the call has no workspace):
-// a workgroup splits its own BM x 32 piece of x and 32 x BN piece of w_hat per step into LDS, in
-// MFMA fragment order, while it multiplies the pieces of the step before; the pieces after come from
-// memory meanwhile.
+// w_hat is formed per element as lq_group_dequantize_f32 writes it, fl32(fl32(c s) + b).  Both operands
+// enter v_mfma_f32_16x16x32_bf16 as sums of bfloat16 terms, which have float32's exponents: a float32
+// value is exactly three of them (8 bits each), a half value two.  x w is the six products of terms
+// that may reach 2^-16 of it (half x: five); what is left out is at most 2^-23 |x| |w|.
+// So each product keeps float32's precision whatever lies beside it in its row, column or tile.  Nothing is
+// prepared in memory (the call has no workspace): a workgroup splits its own BM x 32 piece of x and 32 x BN
+// piece of w_hat per step into LDS, in MFMA fragment order, while it multiplies the pieces of the step
+// before; the pieces after come from memory meanwhile.
 //
-// Exponents.  fp16 terms need values below 2^16 with room for 22 bits under them.  w_hat of a tile
-// is scaled by one power of two from the tile's largest |b| and |s L + b| (first pass over the
-// scales).  A row of x carries a running power of two: set by its first nonzero step (largest value
-// into [2^11, 2^12)), changed only by a step whose largest value leaves [2^-3, 2^15); the sums are
-// then multiplied by the change, exactly.  Infinite inputs would turn into NaN by the split: a tile
-// that meets one is computed again element by element in fp32.
+// The terms of a value must be finite and, since these instructions read subnormal terms as 0, not far
+// below it.  A tile that meets an infinity, a scale that may make one, or eight values or a scale below
+// 2^-100 (but not 0) is computed again with v_mfma_f32_16x16x4_f32 on the float32 values themselves, through the
+// same stages: infinities, NaN and subnormals as a float32 sum has them (M = 2048, N = K = 4096 with an infinity in
+// every tile: 392 us for the terms, 1025 in all).  Beside larger ones of its eight, a smaller value is exact to 2^-126.
 //
-// What bounds it: instruction issue.  Per thread and step 8 values of w_hat (byte load, convert, fma,
-// two roundings) and 8 or 16 of x (two fused multiply-round each) beside 24 or 48 MFMA of a wave, so
-// tiles are as large as the shape allows: 256 x 128 in eight waves of 64 x 64, 128 x 128 in waves of
-// 64 x 32, 32 x 64 with the steps split between four groups of four waves.  Against the float32 VALU
-// kernel this replaced (128 x 128 tiles, 75 of at most 79 TFLOP/s without packed fp32), N = K = 4096,
-// 4 bits, groups of 64: M = 2048 922 -> 300 us, M = 512 881 -> 209, M = 26 880 -> 69; half x, 8 bits,
-// groups of 128: M = 2048 1323 -> 194, M = 26 940 -> 54.  The error against 64 bits fell too
-// (M = 2048: 1.1e-6 -> 7.1e-7): shorter chains of additions.
+// What bounds it: the issue of instructions and the waits around a step's barrier.  Per wave and step of the largest
+// tiles 96 MFMA (half x: 80) and 290 VALU: conversion to terms 11 per pair of values, one addition per
+// sum, three per weight code.  Tiles are as large as the shape allows: 256 x 128 in eight waves of 64 x 64,
+// 128 x 128 in waves of 64 x 32, 32 x 64 with the steps split between four groups of four waves.  N = K = 4096,
+// 4 bits, groups of 64, against the float32 VALU kernel before (128 x 128 tiles, 75 of at most 79
+// TFLOP/s without packed fp32): M = 2048 922 -> 392 us, M = 512 881 -> 229, M = 26 880 -> 64; half x
+// M = 2048 1323 -> 317.  The float32 matrix instructions alone took 595, 335 and 73 us.  Two fp16 terms per value
+// (three products, 312, 211 and 71 us) need a scale per row and tile, and lost values far below it.
+// The error against 64 bits at M = 2048 fell from 1.1e-6 to 2.3e-7: shorter chains of additions.  Ordering the
+// instructions by hand (3 VALU after each MFMA), conversions before the products in half of the waves and after
+// them in the others, or a higher priority for the products measured the same or slower.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,13 +56,36 @@ struct NtArgs {
     int64_t tiles_m, tiles_k;
 };
 
-constexpr int NT_E_UNSET = 1 << 20;
+constexpr float NT_TINY = 0x1p-100f;
+
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
 
 // 16-byte slot of (quarter q, row r) in a fragment's 1 KB: the rotation by 4 q spreads the four
 // quarters of one row (written by neighbouring lanes) over the banks.
 __device__ __forceinline__ int nt_slot(int q, int r) { return q * 16 + ((r + 4 * q) & 15); }
 
-__device__ __forceinline__ float pow2(int e) { return __int_as_float((e + 127) << 23); }  // -126 <= e <= 127
+// Eight values as T bfloat16 terms, each the nearest to what those before it leave: their sum is the
+// value itself, for float32 with T = 3 and for half with T = 2.
+template <int T>
+__device__ __forceinline__ void split_terms(const float (&v)[8], vu4 (&term)[T]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        f2 r = {v[2 * p], v[2 * p + 1]};
+#pragma unroll
+        for (int j = 0; j < T; ++j) {
+            const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, b2));
+            term[j][p] = u;
+            r[0] -= __uint_as_float(u << 16);
+            r[1] -= __uint_as_float(u & 0xFFFF0000u);
+        }
+    }
+}
+
+__device__ __forceinline__ f4 mfma_bf16(vu4 a, vu4 b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
+}
 
 // VEC: rows of x are 16-byte aligned and N a multiple of 8 (an octet past N re-reads the row's last
 // one: its weights are 0).
@@ -66,27 +93,20 @@ __device__ __forceinline__ float pow2(int e) { return __int_as_float((e + 127) <
 template <int BITS, bool XF32, bool VEC, int WM, int WN, int FM, int FN, int GR>
 __global__ __launch_bounds__(64 * WM * WN * GR) void group_matmul_nt_kernel(NtArgs a) {
     constexpr int W = WM * WN, NT = 64 * W, BM = 16 * WM * FM, BN = 16 * WN * FN;
-    constexpr int T = XF32 ? 2 : 1;
+    constexpr int TX = XF32 ? 3 : 2, TW = 3;  // terms of a value of x, of w_hat
     constexpr float L = (float)((1 << BITS) - 1);
     constexpr int XO = (BM * 4 + NT - 1) / NT, WO = BN * 4 / NT;  // octets per thread and step
     static_assert(BN * 4 % NT == 0 && NT % BN == 0 && WO >= 1, "one k per thread");
-    constexpr int X_BYTES = BM * 64 * T, W_BYTES = BN * 64 * 2, STAGE = X_BYTES + W_BYTES;
+    constexpr int X_BYTES = BM * 64 * TX, W_BYTES = BN * 64 * TW, STAGE = X_BYTES + W_BYTES;
     constexpr int SBN = BN / 32 * 32;  // pairs per step: up to BN / 32 groups x 32 rows
     __shared__ __attribute__((aligned(1024))) char lds_[GR][2 * STAGE];
     __shared__ __attribute__((aligned(16))) float2 sbuf_[GR][2][SBN];
-    __shared__ float row_scale_[GR][3][BM];
-    __shared__ int row_e_[GR][BM];
-    __shared__ int changed_[GR][3];
-    __shared__ float wmax[W * GR];
     static_assert(GR == 1 || (GR - 1) * FM * FN * NT * 16 <= GR * 2 * STAGE, "the groups' sums fit the stages");
     const int grp = GR == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
     const int tid = threadIdx.x - grp * NT, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     char* const lds = lds_[grp];
     float2 (*const sbuf)[SBN] = sbuf_[grp];
-    float (*const row_scale)[BM] = row_scale_[grp];
-    int* const row_e = row_e_[grp];
-    int* const changed = changed_[grp];
     const int wm = wave / WN, wn = wave % WN;
     const int steps = ((a.N + 31) / 32 + GR - 1) / GR, s0 = grp * steps;  // steps past N add zeros
     const int64_t row_bytes = (int64_t)a.K * BITS / 8;
@@ -105,37 +125,14 @@ __global__ __launch_bounds__(64 * WM * WN * GR) void group_matmul_nt_kernel(NtAr
         const int m0 = (int)(band * 8 + in % h) * BM, k0 = (int)(in / h) * BN;
         __syncthreads();
 
-        // ---- the tile's weight exponent
-        float wm_ = 0.0f;
-        for (int i = threadIdx.x; i < a.N * ngt; i += NT * GR) {
-            const int n = i / ngt, g = k0 / a.gs + i % ngt;
-            if (g < a.G) {
-                const float s = round_to(a.scales[(int64_t)n * a.G + g], a.hmode);
-                const float b = a.biases ? round_to(a.biases[(int64_t)n * a.G + g], a.hmode) : 0.0f;
-                wm_ = fmaxf(wm_, fmaxf(fabsf(b), fabsf(__builtin_fmaf(s, L, b))));
-            }
-        }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) wm_ = fmaxf(wm_, __shfl_xor(wm_, off, 64));
-        if (lane == 0) wmax[grp * W + wave] = wm_;
-        if (tid < 3) changed[tid] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < W * GR; ++i) wm_ = fmaxf(wm_, wmax[i]);
-        bool bad = !(wm_ <= 3.0e38f);  // an infinity: the fp32 pass below
-        const int ew = wm_ > 0.0f && !bad ? min(max(14 - ilogbf(wm_), -120), 120) : 0;
-
         // ---- this thread's pieces
-        int xr[XO], e[XO];
-        float mx[XO], up[XO];  // the row's largest |x| so far, its 2^e
+        bool bad = false;  // a value whose terms are not finite, or are subnormal
+        int xr[XO];
         const int xq = tid & 3;
         const void* xrow[XO];
 #pragma unroll
         for (int u = 0; u < XO; ++u) {
             xr[u] = (tid + u * NT) >> 2;
-            e[u] = NT_E_UNSET;
-            mx[u] = 0.0f;
-            up[u] = 1.0f;
             xrow[u] = static_cast<const uint8_t*>(a.x) + (int64_t)min(m0 + xr[u], a.M - 1) * a.ldx * (XF32 ? 4 : 2);
         }
         // the weight octets' rows are the same for a wave (BN a multiple of 64): scalar addresses
@@ -186,133 +183,125 @@ __global__ __launch_bounds__(64 * WM * WN * GR) void group_matmul_nt_kernel(NtAr
                 sb.y = a.biases ? a.biases[(int64_t)n * a.G + g] : 0.0f;
             }
         };
-        const float uw = pow2(ew);
         auto store_sb = [&](int t) __attribute__((always_inline)) {
-            if (sb_wave && (tid >> 5) < ngt)
-                sbuf[t & 1][tid] = make_float2(round_to(sb.x, a.hmode) * uw, round_to(sb.y, a.hmode) * uw);
-        };
-        // Step t's rows keep their power of two unless a largest value leaves its range: one branch
-        // for the wave, rarely taken.
-        auto decide = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-            for (int u = 0; u < XO; ++u) {
-                if constexpr (XF32) {
-                    float am = 0.0f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(xv[u][i]));
-                    am = fmaxf(am, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(am), 0xB1, 0xF, 0xF, true)));
-                    am = fmaxf(am, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(am), 0x4E, 0xF, 0xF, true)));
-                    bad |= am > 3.0e38f;
-                    const float at = am * up[u];
-                    mx[u] = fmaxf(mx[u], am);
-                    const bool need = am > 0.0f && (e[u] == NT_E_UNSET || at >= 32768.0f || at < 0.125f);
-                    if (__ballot(need)) {
-                        float by = 1.0f;
-                        if (need) {
-                            // the sums of the steps before stay finite: they are at most 2^75 2^15 N
-                            const int to = min(min(max(11 - ilogbf(am), -120), 120), 75 - ilogbf(mx[u]));
-                            if (e[u] != NT_E_UNSET && to != e[u]) {
-                                by = ldexpf(1.0f, to - e[u]);
-                                changed[t % 3] = 1;
-                            }
-                            e[u] = to;
-                            up[u] = pow2(to);
-                        }
-                        if (xr[u] < BM && xq == 0) row_scale[t % 3][xr[u]] = by;
-                    } else if (xr[u] < BM && xq == 0) {
-                        row_scale[t % 3][xr[u]] = 1.0f;
-                    }
-                } else {
-                    float am = 0.0f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf((float)xh[u][i]));
-                    bad |= am > 65504.0f;
-                }
+            if (sb_wave && (tid >> 5) < ngt) {
+                const float s = round_to(sb.x, a.hmode), b = round_to(sb.y, a.hmode);
+                bad |= !(fabsf(s) * L + fabsf(b) <= 3.0e38f) || (s != 0.0f && fabsf(s) < NT_TINY);
+                sbuf[t & 1][tid] = make_float2(s, b);
             }
         };
-        auto convert = [&](int t) __attribute__((always_inline)) {  // step t into LDS
+        // Step t into LDS: bfloat16 terms, or (EXACT) the float32 values as two pieces of four.
+        auto convert = [&](int t, auto exact) __attribute__((always_inline)) {
+            constexpr bool EXACT = decltype(exact)::value;
             char* base = lds + (t & 1) * STAGE;
+            auto put = [&](vu4* dst, const float (&v)[8], auto terms) __attribute__((always_inline)) {
+                constexpr int T = decltype(terms)::value;
+                if constexpr (EXACT) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        dst[64 * j] = __builtin_bit_cast(vu4, vf4{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]});
+                } else {
+                    vu4 term[T];
+                    split_terms(v, term);
+#pragma unroll
+                    for (int j = 0; j < T; ++j) dst[64 * j] = term[j];
+                }
+            };
 #pragma unroll
             for (int u = 0; u < WO; ++u) {
                 const int oq = oq0 + u * (NT / BN);
                 const float4* p = reinterpret_cast<const float4*>(&sbuf[t & 1][wk / a.gs * 32 + oq * 8]);
-                h8 hi, lo;
+                float v[8];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float4 v = p[i];  // {s, b} of rows 2 i and 2 i + 1
+                    const float4 s = p[i];  // {s, b} of rows 2 i and 2 i + 1
 #pragma unroll
                     for (int j = 0; j < 2; ++j) {
                         const uint32_t c = BITS == 8 ? wv[u][2 * i + j] : (wv[u][2 * i + j] >> (4 * (wk & 1))) & 15u;
-                        const float w = __builtin_fmaf((float)(uint8_t)c, j ? v.z : v.x, j ? v.w : v.y);
-                        const _Float16 hh = (_Float16)w;
-                        hi[2 * i + j] = hh;
-                        lo[2 * i + j] = (_Float16)(w - (float)hh);
+                        v[2 * i + j] = (float)(uint8_t)c * (j ? s.z : s.x) + (j ? s.w : s.y);
                     }
                 }
-                h8* dst = reinterpret_cast<h8*>(base + X_BYTES) + (wk >> 4) * 128 + nt_slot(oq, wk & 15);
-                dst[0] = hi;
-                dst[64] = lo;
+                put(reinterpret_cast<vu4*>(base + X_BYTES) + (wk >> 4) * TW * 64 + nt_slot(oq, wk & 15), v,
+                    std::integral_constant<int, TW>{});
             }
 #pragma unroll
             for (int u = 0; u < XO; ++u) {
-                h8* dst = reinterpret_cast<h8*>(base) + (xr[u] >> 4) * T * 64 + nt_slot(xq, xr[u] & 15);
-                if constexpr (XF32) {
-                    h8 hi, lo;
+                float v[8], am = 0.0f;
+                // (a value past N would meet a zero weight: an infinity there must not)
+                const bool in = !EXACT || (s0 + t) * 32 + xq * 8 < a.N;
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        hi[i] = (_Float16)(xv[u][i] * up[u]);
-                        lo[i] = (_Float16)__builtin_fmaf(xv[u][i], up[u], -(float)hi[i]);
-                    }
-                    if (XO * NT == BM * 4 || xr[u] < BM) {
-                        dst[0] = hi;
-                        dst[64] = lo;
-                    }
-                } else {
-                    if (XO * NT == BM * 4 || xr[u] < BM) dst[0] = xh[u];
+                for (int i = 0; i < 8; ++i) {
+                    if constexpr (XF32) v[i] = in ? xv[u][i] : 0.0f;
+                    else v[i] = in ? (float)xh[u][i] : 0.0f;
+                    am = fmaxf(am, fabsf(v[i]));
                 }
+                bad |= am > (XF32 ? 3.0e38f : 65504.0f) || (XF32 && am != 0.0f && am < NT_TINY);
+                if (XO * NT == BM * 4 || xr[u] < BM)
+                    put(reinterpret_cast<vu4*>(base) + (xr[u] >> 4) * TX * 64 + nt_slot(xq, xr[u] & 15), v,
+                        std::integral_constant<int, TX>{});
             }
         };
 
         f4 acc[FM][FN];
-#pragma unroll
-        for (int m = 0; m < FM; ++m)
-#pragma unroll
-            for (int n = 0; n < FN; ++n) acc[m][n] = f4{0.f, 0.f, 0.f, 0.f};
         const int slot = nt_slot(q, l16);
-        auto multiply = [&](int t, auto between) __attribute__((always_inline)) {
+        auto multiply = [&](int t, auto exact, auto between) __attribute__((always_inline)) {
+            constexpr bool EXACT = decltype(exact)::value;
+            constexpr int NX = EXACT ? 2 : TX, NW = EXACT ? 2 : TW;
             const vu4* X = reinterpret_cast<const vu4*>(lds + (t & 1) * STAGE) + slot;
             const vu4* Wf = reinterpret_cast<const vu4*>(lds + (t & 1) * STAGE + X_BYTES) + slot;
-            h8 xf[FM][T];
+            vu4 xf[FM][NX];
 #pragma unroll
             for (int m = 0; m < FM; ++m)
 #pragma unroll
-                for (int j = 0; j < T; ++j) xf[m][j] = __builtin_bit_cast(h8, X[((wm * FM + m) * T + j) * 64]);
+                for (int j = 0; j < NX; ++j) xf[m][j] = X[((wm * FM + m) * TX + j) * 64];
             between();
 #pragma unroll
             for (int n = 0; n < FN; ++n) {
-                h8 wf[2];
+                vu4 wf[NW];
 #pragma unroll
-                for (int j = 0; j < 2; ++j) wf[j] = __builtin_bit_cast(h8, Wf[((wn * FN + n) * 2 + j) * 64]);
-                // the small terms first
-                if constexpr (XF32) {
+                for (int j = 0; j < NW; ++j) wf[j] = Wf[((wn * FN + n) * TW + j) * 64];
+                if constexpr (EXACT) {
 #pragma unroll
-                    for (int m = 0; m < FM; ++m) acc[m][n] = mfma16(wf[0], xf[m][T - 1], acc[m][n]);
+                    for (int e = 0; e < 8; ++e)
+#pragma unroll
+                        for (int m = 0; m < FM; ++m)
+                            acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(wf[e / 4][e % 4]),
+                                                                             __uint_as_float(xf[m][e / 4][e % 4]), acc[m][n], 0, 0, 0);
+                } else {
+                    // the small products first; one addition to the long sum per step
+                    f4 blk[FM];
+#pragma unroll
+                    for (int m = 0; m < FM; ++m) blk[m] = f4{0.f, 0.f, 0.f, 0.f};
+                    auto add = [&](auto ix, auto iw) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int m = 0; m < FM; ++m) blk[m] = mfma_bf16(wf[decltype(iw)::value], xf[m][decltype(ix)::value], blk[m]);
+                    };
+                    using I0 = std::integral_constant<int, 0>;
+                    using I1 = std::integral_constant<int, 1>;
+                    using I2 = std::integral_constant<int, 2>;
+                    if constexpr (XF32) add(I2{}, I0{});
+                    add(I0{}, I2{});
+                    add(I1{}, I1{});
+                    add(I1{}, I0{});
+                    add(I0{}, I1{});
+                    add(I0{}, I0{});
+#pragma unroll
+                    for (int m = 0; m < FM; ++m) acc[m][n] += blk[m];
                 }
-#pragma unroll
-                for (int m = 0; m < FM; ++m) acc[m][n] = mfma16(wf[1], xf[m][0], acc[m][n]);
-#pragma unroll
-                for (int m = 0; m < FM; ++m) acc[m][n] = mfma16(wf[0], xf[m][0], acc[m][n]);
             }
         };
-
-        if (steps > 0) {
+        auto walk = [&](auto exact) __attribute__((always_inline)) {
+#pragma unroll
+            for (int m = 0; m < FM; ++m)
+#pragma unroll
+                for (int n = 0; n < FN; ++n) acc[m][n] = f4{0.f, 0.f, 0.f, 0.f};
+            if (steps <= 0) return;
             load_sb(0);
             load(0);
             store_sb(0);
             load_sb(1);
             __syncthreads();
-            decide(0);
-            convert(0);
+            convert(0, exact);
             load(min(1, steps - 1));
             store_sb(1);
             load_sb(2);
@@ -320,60 +309,20 @@ __global__ __launch_bounds__(64 * WM * WN * GR) void group_matmul_nt_kernel(NtAr
                 block_barrier();  // step t's pieces and step t + 1's scales are in LDS
                 store_sb(t + 2);
                 load_sb(t + 3);
-                if constexpr (XF32) {
-                    if (__builtin_amdgcn_readfirstlane(changed[t % 3])) {
-#pragma unroll
-                        for (int m = 0; m < FM; ++m) {
-                            const float by = row_scale[t % 3][(wm * FM + m) * 16 + l16];
-#pragma unroll
-                            for (int n = 0; n < FN; ++n) acc[m][n] *= by;
-                        }
-                    }
-                    if (tid == 0) changed[(t + 2) % 3] = 0;  // read by every wave before this barrier
-                }
-                if (t + 1 < steps) decide(t + 1);
                 // the last step converts a step past the end once more: no branch around the products
-                multiply(t, [&]() __attribute__((always_inline)) {
-                    convert(t + 1);
+                multiply(t, exact, [&]() __attribute__((always_inline)) {
+                    convert(t + 1, exact);
                     load(min(t + 2, steps - 1));
                 });
             }
+        };
+        walk(std::false_type{});
+        if (__syncthreads_or(bad)) {
+            walk(std::true_type{});
+            __syncthreads();
         }
 
-        // ---- the outputs
-        if constexpr (XF32) {
-#pragma unroll
-            for (int u = 0; u < XO; ++u)
-                if (xr[u] < BM && xq == 0) row_e[xr[u]] = e[u] == NT_E_UNSET ? 0 : e[u];
-        }
-        if (__syncthreads_or(bad)) {  // element by element in fp32
-            for (int i = threadIdx.x; i < BM * BN; i += NT * GR) {
-                const int row = m0 + i / BN, k = k0 + i % BN;
-                if (row >= a.M || k >= a.K) continue;
-                float v = 0.0f;
-                for (int r = 0; r < a.N; ++r) {
-                    const float xx = XF32 ? static_cast<const float*>(a.x)[(int64_t)row * a.ldx + r]
-                                          : (float)static_cast<const _Float16*>(a.x)[(int64_t)row * a.ldx + r];
-                    const uint32_t byte = a.w[(int64_t)r * row_bytes + (BITS == 8 ? k : k >> 1)];
-                    const float c = (float)(BITS == 8 ? byte : (byte >> (4 * (k & 1))) & 15u);
-                    const int64_t gi = (int64_t)r * a.G + k / a.gs;
-                    const float cs = c * round_to(a.scales[gi], a.hmode);
-                    v = __builtin_fmaf(xx, a.biases ? cs + round_to(a.biases[gi], a.hmode) : cs, v);
-                }
-                v = wo_finish(v, a.bias != nullptr, a.bias ? a.bias[k] : 0.0f, a.relu, a.hmode);
-                if constexpr (XF32) static_cast<float*>(a.y)[(int64_t)row * a.ldy + k] = v;
-                else static_cast<_Float16*>(a.y)[(int64_t)row * a.ldy + k] = (_Float16)v;
-            }
-            continue;
-        }
-        // the rows' powers of two leave the sums, then the groups' sums meet, added in order
-#pragma unroll
-        for (int m = 0; m < FM; ++m) {
-            const int down = -(XF32 ? row_e[(wm * FM + m) * 16 + l16] : 0) - ew;  // -240 .. 240, in two exact steps
-            const float d0 = ldexpf(1.0f, down / 2), d1 = ldexpf(1.0f, down - down / 2);
-#pragma unroll
-            for (int n = 0; n < FN; ++n) acc[m][n] = acc[m][n] * d0 * d1;
-        }
+        // ---- the outputs: the groups' sums meet, added in order
         if constexpr (GR > 1) {
             f4* sums = reinterpret_cast<f4*>(lds_[0]) + tid;
             if (grp > 0) {
@@ -452,10 +401,10 @@ void group_matmul_nt_launch(const WoNtCall& c, hipStream_t st) {
     auto tiles = [&](int bm, int bn) { return (((int64_t)a.M + bm - 1) / bm) * (((int64_t)a.K + bn - 1) / bn); };
     auto pick = [&](auto bits, auto xf) {
         // Rounds of 256 workgroups times a round's time per step, measured at N = 4096 in float32 (us
-        // per step; in half all three take about 0.65 of it): 256 x 128 tiles 2.36, 128 x 128 1.64,
-        // 32 x 64 with the steps split between four wave groups 0.58.
+        // per step; in half all three take about 0.85 of it): 256 x 128 tiles 3.06, 128 x 128 1.94,
+        // 32 x 64 with the steps split between four wave groups 0.56.
         auto cost = [&](int bm, int bn, double step) { return (double)((tiles(bm, bn) + 255) / 256) * step; };
-        const double c256 = cost(256, 128, 2.36), c128 = cost(128, 128, 1.64), c32 = cost(32, 64, 0.58);
+        const double c256 = cost(256, 128, 3.06), c128 = cost(128, 128, 1.94), c32 = cost(32, 64, 0.56);
         if (c256 < c128 && c256 < c32) go(bits, xf, I4{}, I2{}, I4{}, I4{}, I1{}, "wo nt 256x128");
         else if (c128 < c32) go(bits, xf, I2{}, I4{}, I4{}, I2{}, I1{}, "wo nt 128x128");
         else go(bits, xf, I2{}, I2{}, I1{}, I2{}, I4{}, "wo nt 32x64");

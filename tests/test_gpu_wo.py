@@ -709,13 +709,13 @@ NT_CASES = [(33, 40, 64, 8, 64), (1, 8, 32, 4, 32), (70, 333, 288, 4, 32), (129,
 @pytest.mark.parametrize("M,N,K,bits,gs", NT_CASES)
 def test_quantized_matmul_no_transpose_tiles(gpu, M, N, K, bits, gs, half):
     """Every tile size against float64, with rows whose magnitude grows, shrinks or starts at zero
-    along the summed axis (the running power of two of the fp16 split), a row whose large part
-    meets zero weights, and infinities and NaN where float64 has them."""
+    along the summed axis, a row whose large part meets zero weights, and infinities and NaN where
+    float64 has them."""
     from lucid_amd.quantization import _qgemm
 
     rng = np.random.default_rng(M + N + K + bits)
     w = rng.standard_normal((N, K)).astype(np.float32)
-    zero = N // 64 * 32  # whole steps: the split keeps ~22 bits of a row's largest value in its step
+    zero = N // 2
     w[:zero] = 0.0
     x = rng.standard_normal((M, N)).astype(np.float32)
     if M > 8:
@@ -749,6 +749,64 @@ def test_quantized_matmul_no_transpose_tiles(gpu, M, N, K, bits, gs, half):
     y = run(x)
     np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
     np.testing.assert_array_equal(np.isinf(y), np.isinf(ref))
+
+
+# (M, N, K) for each of the three tile sizes, N with a partial step, K with a partial tile
+NT_RANGE_SHAPES = [(40, 200, 320), (1200, 136, 2432), (2300, 104, 2496)]
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("bits,gs", [(4, 32), (8, 64)])
+@pytest.mark.parametrize("M,N,K", NT_RANGE_SHAPES)
+def test_quantized_matmul_no_transpose_range(gpu, M, N, K, bits, gs, half):
+    """Every output against sum |x| |w_hat| of its own: neighbouring groups and rows of the weight
+    whose scales lie up to 1e-10 apart (1e-4 in half), and large activations beside ordinary ones that meet
+    zero weights.  What else lies in a step, a row or a tile must not cost an output its bits.  The
+    bound is a float32 sum's, N roundings of 2^-24, twice for the terms left out."""
+    from lucid_amd.quantization import _qgemm
+
+    rng = np.random.default_rng(M + N + bits)
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    packed, scales, biases = _qgemm.quantize(_t(gpu, w), group_size=gs, bits=bits)
+    lo = 1e-4 if half else 1e-10
+    spread = np.where(np.arange(K // gs) % 2, lo, 1.0)[None, :] * np.where(np.arange(N) % 3 == 1, lo, 1.0)[:, None]
+    sc, bi = (scales.numpy() * spread).astype(np.float32), (biases.numpy() * spread).astype(np.float32)
+    sc[7::32], bi[7::32] = 0.0, 0.0  # one row of every step
+    if half:
+        sc, bi = sc.astype(np.float16).astype(np.float32), bi.astype(np.float16).astype(np.float32)
+    x = rng.standard_normal((M, N)).astype(np.float32)
+    x[::2, 7::32] *= 1e4 if half else 1e12
+    x[1::4] *= 1e-4 if half else 1e-25
+    x = x.astype(np.float16 if half else np.float32)
+    wd = O.group_dequantize(packed.numpy().view(np.uint32), sc, bi, gs, bits).astype(np.float64)
+    y = _qgemm.quantized_matmul(_t(gpu, x), packed, _t(gpu, sc), _t(gpu, bi), transpose=False, group_size=gs,
+                                bits=bits).numpy()
+    x = x.astype(np.float64)
+    bound = (np.abs(x) @ np.abs(wd)) * (2 * N * 2.0 ** -24)
+    if half:
+        bound += np.abs(x @ wd) * 2.0 ** -11 + 2.0 ** -25  # the result's own rounding
+    assert np.all(np.abs(y - x @ wd) <= bound)
+
+
+def test_quantized_matmul_no_transpose_small_values(gpu):
+    """Activations and scales near the smallest float32 numbers, beside ordinary rows: a float32 sum's
+    own accuracy, 2^-149 per product and addition."""
+    from lucid_amd.quantization import _qgemm
+
+    rng = np.random.default_rng(2)
+    M, N, K = 70, 96, 128
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    x = rng.standard_normal((M, N)).astype(np.float32)
+    for i, e in enumerate((-90, -99, -105, -115, -125, -135)):
+        x[i] *= 2.0 ** e
+    packed, scales, biases = _qgemm.quantize(_t(gpu, w), group_size=64, bits=8)
+    for scale in (1.0, 2.0 ** -105):
+        sc, bi = scales.numpy() * np.float32(scale), biases.numpy() * np.float32(scale)
+        wd = O.group_dequantize(packed.numpy().view(np.uint32), sc, bi, 64, 8).astype(np.float64)
+        y = _qgemm.quantized_matmul(_t(gpu, x), packed, _t(gpu, sc), _t(gpu, bi), transpose=False, group_size=64,
+                                    bits=8).numpy()
+        xd = x.astype(np.float64)
+        assert np.all(np.abs(y - xd @ wd) <= (np.abs(xd) @ np.abs(wd)) * (2 * N * 2.0 ** -24) + 2 * N * 2.0 ** -149)
 
 
 def test_group_matmul_no_transpose_empty_reduction(gpu):
