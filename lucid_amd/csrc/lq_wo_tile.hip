@@ -16,11 +16,12 @@
 // 992 -> 205; half x, 4 bits, M = 1024 456 -> 88.  What bounds it now is the issue of instructions:
 // per wave and stage 32 MFMA (16 cycles each), 64 FMA of scales, 32 for unpacking, 26 LDS reads;
 // the matrix cores are busy about a third of the time.
-// Arithmetic per 64-wide block (32 for groups of 32): blk = sum c (hi + lo) in fp32, then
-// acc += s blk + b bsum.  A row's values are scaled by one 2^e for the whole row (its largest
-// value in [2^14, 2^15)); a block whose own maximum lies below 2^-3 of that scale gets an
-// exponent of its own and its sum is multiplied back (factor f, else 1), so every block keeps
-// ~22 significant bits of its own largest value.  2^-e is applied to the finished sum.
+// Arithmetic per 64-wide block (32 for groups of 32), that of the GEMV kernels: the block's values of a
+// row are scaled by 2^e (its largest into [2^14, 2^15)) before the split, blk = sum c (hi + lo) in fp32,
+// then acc += s (blk 2^-e) + b bsum.  2^-e goes to the scale, ahead of the products (after them, 137 us
+// instead of 126 at M = 1024, 8 bits, groups of 64): exact, unless 2^-e is so small that s 2^-e may not
+// be a normal number, so below 2^-90 the rest of it goes to blk.  One scale for the whole row instead took
+// 117 us, and lost bits of values far below the row's largest.
 // Few tiles: K is split into ranges over workgroups, their sums added in range order by
 // wo_tile_reduce_kernel.  Without a workspace the same sums are made by workgroups that split
 // the activations themselves and walk the ranges in order: the same bits, slower.
@@ -44,14 +45,19 @@ struct WtArgs {
     int rs;            // stages per K range
     int ranges;        // K ranges
     const char* xp;    // split activations: [Mp][KB][2 steps][T][4 quarters] of 8 halves
-    const float2* xm;  // [KB][NG][Mp]: block sum (scaled by 2^e), factor f
-    const vf4* xr;     // [Mp]: {2^-e, row sum (scaled), 1 if a block has its own exponent, 0}
+    const float2* xm;  // [KB][NG][Mp]: block sum, 2^-e
+    const float2* xr;  // [Mp]: row sum (per-channel weights), 1 if a block's 2^-e lies below WT_TINY
     const float2* sb;  // [G][Np]: group scale, group bias
     int Np;            // columns padded to 128
     float* part;       // range sums [ranges][tile][frag][thread] f4, or null
 };
 
 constexpr int WT_FLUSH = 8;  // stages per first-level sum
+constexpr float WT_TINY = 0x1p-90f;
+
+// 2^-e as the factor of a group scale and what is left of it for the block's sum (1 above WT_TINY).
+__device__ __forceinline__ float down_scale(float down) { return fmaxf(down, WT_TINY); }
+__device__ __forceinline__ float down_rest(float down) { return fminf(down * (1.0f / WT_TINY), 1.0f); }
 
 // Blocks per stage: groups of 32 make two blocks of 32 k, everything else one of 64.
 template <int S>
@@ -62,13 +68,6 @@ template <int S>
 __device__ __forceinline__ void octet_pos(int o, int& step, int& q) {
     if (S == 2) { step = o & 1; q = o >> 1; }   // a lane quarter holds 16 consecutive k
     else { step = o >> 2; q = o & 3; }          // one block of 32 per step
-}
-
-__device__ __forceinline__ float row_exp2(float amax, int* e_out) {
-    int e = 0;
-    if (amax > 0.0f && amax <= 3.0e38f) e = min(max(14 - ilogbf(amax), -120), 120);
-    *e_out = e;
-    return ldexpf(1.0f, e);
 }
 
 // The 8 values of octet o of one row (0 past K or for rows past M).
@@ -117,62 +116,71 @@ __device__ __forceinline__ float octet_amax(const float (&v)[8]) {
     return a;
 }
 
-// hi / lo terms, block sum and factor of one octet; the 4 S lanes of a block's octets are
-// consecutive lanes of one wave.  up = 2^e of the row.
-template <int BITS, int S, int T>
-__device__ __forceinline__ void split_octet(const float (&v)[8], float up, int e, h8& hi, h8& lo, float& bsum, float& f) {
-    float bs = octet_sum(v), am = octet_amax(v);
-#pragma unroll
-    for (int off = 1; off < 4 * S; off <<= 1) {
-        bs += __shfl_xor(bs, off, 64);
-        am = fmaxf(am, __shfl_xor(am, off, 64));
-    }
-    f = 1.0f;
-    float u = up;
-    if (T == 2 && am > 0.0f && am * up < 0.125f) {
-        int e2;
-        u = row_exp2(am, &e2);
-        f = ldexpf(1.0f, e - e2);
-    }
-    bsum = T == 2 ? bs * up : bs;
+// 2^e and 2^-e of a block from its largest |value|: 14 - exponent, clamped (a subnormal's exponent
+// field is 0: the upper clamp).
+template <int T>
+__device__ __forceinline__ void block_scale(float am, float& up, float& down) {
+    const int e = T == 2 && am > 0.0f && am <= 3.0e38f ? min(max(14 + 127 - (int)(__float_as_uint(am) >> 23), -120), 120) : 0;
+    up = __uint_as_float((uint32_t)(127 + e) << 23);
+    down = __uint_as_float((uint32_t)(127 - e) << 23);
+}
+
+template <int BITS, int T>
+__device__ __forceinline__ void octet_terms(const float (&v)[8], float up, h8 (&x)[T]) {
 #pragma unroll
     for (int h = 0; h < 8; ++h) {
-        const float x = T == 2 ? v[korder<BITS>(h)] * u : v[korder<BITS>(h)];
-        hi[h] = (_Float16)x;
-        lo[h] = T == 2 ? (_Float16)(x - (float)hi[h]) : (_Float16)0.0f;
+        const float f = T == 2 ? v[korder<BITS>(h)] * up : v[korder<BITS>(h)];
+        x[0][h] = (_Float16)f;
+        if constexpr (T == 2) x[1][h] = (_Float16)(f - (float)x[0][h]);
     }
 }
 
-// Quarter w of one row's largest |x| and sum, by one wave: lane l owns octets 64 w + l, + 256, ...
-// The row's sum is its four quarters' sums added in order.
+// Terms, block sum and 2^-e of one octet; the 4 S lanes of a block's octets are consecutive lanes
+// of one wave.
+template <int BITS, int S, int T>
+__device__ __forceinline__ void split_octet(const float (&v)[8], h8 (&x)[T], float& bsum, float& down) {
+    bsum = octet_sum(v);
+    float am = octet_amax(v), up;
+#pragma unroll
+    for (int off = 1; off < 4 * S; off <<= 1) {
+        bsum += __shfl_xor(bsum, off, 64);
+        am = fmaxf(am, __shfl_xor(am, off, 64));
+    }
+    block_scale<T>(am, up, down);
+    octet_terms<BITS, T>(v, up, x);
+}
+
+// The sum over a wave of its lanes' values.
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// One row's sum, by one wave, as the prepare launch adds it: thread t of 256 owns octets t, t + 256, ...,
+// each quarter of the threads is summed over a wave and the four quarters in order.
 template <bool XF32>
-__device__ __forceinline__ void row_scan(const WoTileCall& c, int m, int w, int lane, bool vec, float& amax, float& sum) {
-    amax = 0.0f;
-    sum = 0.0f;
-    const int no = (c.K + 7) / 8;
-    for (int o0 = 64 * w; o0 < no; o0 += 512) {  // two octets in flight
-        float v[2][8];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) load_octet<XF32>(c, m, (o0 + lane + 256 * u) * 8, vec, v[u]);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            amax = fmaxf(amax, octet_amax(v[u]));
-            sum += octet_sum(v[u]);
+__device__ __forceinline__ float row_sum(const WoTileCall& c, int m, int lane, bool vec) {
+    float sum = 0.0f;
+    for (int w = 0; w < 4; ++w) {
+        float s = 0.0f;
+        for (int o = 64 * w + lane; o < (c.K + 7) / 8; o += 256) {
+            float v[8];
+            load_octet<XF32>(c, m, o * 8, vec, v);
+            s += octet_sum(v);
         }
+        s = wave_sum(s);
+        sum = w ? sum + s : s;
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-        sum += __shfl_xor(sum, off, 64);
-    }
+    return sum;
 }
 
 // The operands the tiled kernel wants contiguous.  The first Mp workgroups: one activation row
-// each, as [stage][step][term][lane quarter] 16-byte pieces, with its block sums and factors and
-// its scale.  The others (group-wise): 32 x 32 pieces of the group scales and biases transposed to
+// each, as [stage][step][term][lane quarter] 16-byte pieces, with its blocks' sums and scales and (for
+// per-channel zero points) its sum.  The others (group-wise): 32 x 32 pieces of the group scales and biases transposed to
 // [group][column] pairs, rounded to the activation's type (a missing bias is 0).
 template <int BITS, int S, int T, bool GROUPED, int HM>
-__global__ __launch_bounds__(256) void wo_tile_prep_kernel(WtArgs a, char* xp, float2* xm, vf4* xr, float2* sb) {
+__global__ __launch_bounds__(256) void wo_tile_prep_kernel(WtArgs a, char* xp, float2* xm, float2* xr, float2* sb) {
     constexpr int NG = wt_blocks<S>();
     constexpr bool XF32 = T == 2;
     __shared__ float2 sh[32][33];
@@ -196,32 +204,30 @@ __global__ __launch_bounds__(256) void wo_tile_prep_kernel(WtArgs a, char* xp, f
     }
     const int m = blockIdx.x;
     const bool vec = x_vec<XF32>(a.c);
-    float amax, sum, up = 1.0f;
-    int e = 0;
-    row_scan<XF32>(a.c, m, wave, lane, vec, amax, sum);
-    if (lane == 0) sh[0][wave] = make_float2(amax, sum);
-    __syncthreads();
-    amax = fmaxf(fmaxf(sh[0][0].x, sh[0][1].x), fmaxf(sh[0][2].x, sh[0][3].x));
-    sum = ((sh[0][0].y + sh[0][1].y) + sh[0][2].y) + sh[0][3].y;
-    if (T == 2) up = row_exp2(amax, &e);
-    bool own = false;
+    float sum = 0.0f;
+    bool tiny = false;
     for (int og = tid; og < a.KB * 8; og += 256) {
         const int kb = og >> 3, o = og & 7;
         float v[8];
         load_octet<XF32>(a.c, m, og * 8, vec, v);
-        h8 hi, lo;
-        float bsum, f;
-        split_octet<BITS, S, T>(v, up, e, hi, lo, bsum, f);
+        if (!GROUPED) sum += octet_sum(v);
+        h8 x[T];
+        float bsum, down;
+        split_octet<BITS, S, T>(v, x, bsum, down);
+        tiny |= down < WT_TINY;
         int step, q;
         octet_pos<S>(o, step, q);
         h8* dst = reinterpret_cast<h8*>(xp) + ((int64_t)m * a.KB + kb) * 8 * T + step * T * 4 + q;
-        dst[0] = hi;
-        if (T == 2) dst[4] = lo;
-        if ((o & (4 * S - 1)) == 0) xm[((int64_t)kb * NG + o / (4 * S)) * a.Mp + m] = make_float2(bsum, f);
-        own |= f != 1.0f;
+#pragma unroll
+        for (int t = 0; t < T; ++t) dst[4 * t] = x[t];
+        if ((o & (4 * S - 1)) == 0) xm[((int64_t)kb * NG + o / (4 * S)) * a.Mp + m] = make_float2(bsum, down);
     }
-    own = __syncthreads_or(own);
-    if (tid == 0) xr[m] = vf4{T == 2 ? ldexpf(1.0f, -e) : 1.0f, T == 2 ? sum * up : sum, own ? 1.0f : 0.0f, 0.0f};
+    if (!GROUPED) {
+        sum = wave_sum(sum);
+        if (lane == 0) sh[0][wave].x = sum;
+    }
+    tiny = __syncthreads_or(tiny);
+    if (tid == 0) xr[m] = make_float2(GROUPED ? 0.0f : ((sh[0][0].x + sh[0][1].x) + sh[0][2].x) + sh[0][3].x, tiny ? 1.0f : 0.0f);
 }
 
 // Tile of a workgroup: consecutive tiles (groups of eight tile rows, column by column) on one
@@ -234,9 +240,18 @@ __device__ __forceinline__ void wt_tile_of(int id, int tm, int tn, int& m, int& 
     n = in / h;
 }
 
+// A block's part of an output: acc + s blk + b bsum (group-wise, s with 2^-e in it), acc + blk 2^-e.
+__device__ __forceinline__ float wt_add(float acc, float blk, float s, float b, float bsum) {
+    return __builtin_fmaf(b, bsum, __builtin_fmaf(s, blk, acc));
+}
+template <int T>
+__device__ __forceinline__ float wt_add(float acc, float blk, float down) {
+    return T == 2 ? __builtin_fmaf(blk, down, acc) : acc + blk;
+}
+
 // The finished value of four consecutive columns of one row.
 template <bool GROUPED, bool XF32>
-__device__ __forceinline__ void wt_store(const WoTileCall& c, int m, int n, f4 v, float down, float sum) {
+__device__ __forceinline__ void wt_store(const WoTileCall& c, int m, int n, f4 v, float sum) {
     if (m >= c.M || n >= c.N) return;
     const bool xf = XF32;
     f4 out;
@@ -246,9 +261,7 @@ __device__ __forceinline__ void wt_store(const WoTileCall& c, int m, int n, f4 v
         float t = v[i];
         if constexpr (!GROUPED) {
             if (c.w_zp) t = t - c.w_zp[nn] * sum;
-            t = c.w_scale[nn] * (t * down);
-        } else {
-            t = t * down;
+            t = c.w_scale[nn] * t;
         }
         out[i] = wo_finish(t, c.bias != nullptr, c.bias ? c.bias[nn] : 0.0f, c.relu, c.hmode);
     }
@@ -289,10 +302,9 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
     constexpr int A_I = (A_BYTES + 16 * NT - 1) / (16 * NT), B_I = (B_BYTES + 16 * NT - 1) / (16 * NT);
     constexpr int F_N = (SB_BYTES + XF_BYTES) / 8, F_I = (F_N + NT - 1) / NT;
     constexpr int TOT_BYTES = BM * BN * 4;
-    static_assert(NST * STAGE + TOT_BYTES + (INLINE ? 12 * BM : 0) <= 160 * 1024, "LDS");
+    static_assert(NST * STAGE + TOT_BYTES + (INLINE ? 4 * BM : 0) <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE + TOT_BYTES];
-    __shared__ float2 row_xr[INLINE ? BM : 1];
-    __shared__ int row_e[INLINE ? BM : 1];
+    __shared__ float row_xr[INLINE ? BM : 1];
     const WoTileCall& c = a.c;
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -383,24 +395,13 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
         }
     };
 
-    // ---- the activation rows' scales, where no prepared copy holds them
+    // ---- the activation rows' sums, where no prepared copy holds them
     constexpr bool XF32 = T == 2;
     const bool vec = INLINE && x_vec<XF32>(c);
-    if constexpr (INLINE) {
+    if (INLINE && !GROUPED && c.w_zp) {
         for (int r = wave; r < BM; r += W) {
-            float amax = 0.0f, sum = 0.0f, up = 1.0f;
-            int e = 0;
-            for (int w = 0; w < 4; ++w) {
-                float am, sm;
-                row_scan<XF32>(c, m0 + r, w, lane, vec, am, sm);
-                amax = fmaxf(amax, am);
-                sum = w ? sum + sm : sm;
-            }
-            if (T == 2) up = row_exp2(amax, &e);
-            if (lane == 0) {
-                row_xr[r] = make_float2(T == 2 ? ldexpf(1.0f, -e) : 1.0f, T == 2 ? sum * up : sum);
-                row_e[r] = e;
-            }
+            const float sum = row_sum<XF32>(c, m0 + r, lane, vec);
+            if (lane == 0) row_xr[r] = sum;
         }
         __syncthreads();
     }
@@ -410,16 +411,16 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
             const int r = i >> 3, o = i & 7;
             float v[8];
             load_octet<XF32>(c, m0 + r, kb * 64 + o * 8, vec, v);
-            h8 hi, lo;
-            float bsum, f;
-            split_octet<BITS, S, T>(v, T == 2 ? ldexpf(1.0f, row_e[r]) : 1.0f, row_e[r], hi, lo, bsum, f);
+            h8 x[T];
+            float bsum, down;
+            split_octet<BITS, S, T>(v, x, bsum, down);
             int step, qq;
             octet_pos<S>(o, step, qq);
             h8* dst = reinterpret_cast<h8*>(base) + ((r >> 4) * 2 + step) * T * 64 + qq * 16 + (r & 15);
-            dst[0] = hi;
-            if (T == 2) dst[64] = lo;
+#pragma unroll
+            for (int t = 0; t < T; ++t) dst[64 * t] = x[t];
             if ((o & (4 * S - 1)) == 0) {
-                reinterpret_cast<float2*>(base + A_BYTES + B_BYTES + SB_BYTES)[o / (4 * S) * BM + r] = make_float2(bsum, f);
+                reinterpret_cast<float2*>(base + A_BYTES + B_BYTES + SB_BYTES)[o / (4 * S) * BM + r] = make_float2(bsum, down);
             }
         }
     };
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
         vu4 x[FM][S][T];
         uint32_t w[FN][S * BITS / 4];
         f4 sb[GROUPED ? FN : 1][2];  // scale, bias of four columns, interleaved
-        float2 xf[FM];               // block sum, factor
+        float2 xf[FM];               // block sum, 2^-e
     };
     auto read = [&](Frags& r, const char* base, int b) __attribute__((always_inline)) {
         const vu4* A = reinterpret_cast<const vu4*>(base) + lane;
@@ -492,8 +493,8 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
             }
         }
     };
-    auto products = [&](const Frags& r, auto own) __attribute__((always_inline)) {
-        constexpr bool OWN = decltype(own)::value;  // some row's block has its own exponent
+    auto products = [&](const Frags& r, auto tiny) __attribute__((always_inline)) {
+        constexpr bool TINY = decltype(tiny)::value;  // some block's 2^-e lies below WT_TINY
 #pragma unroll
         for (int n = 0; n < FN; ++n) {
             h8 wa[S];
@@ -510,31 +511,25 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
                     for (int m = 0; m < FM; ++m) blk[m] = mfma16(wa[j], __builtin_bit_cast(h8, r.x[m][j][t]), blk[m]);
 #pragma unroll
             for (int m = 0; m < FM; ++m) {
-                if constexpr (OWN) blk[m] *= r.xf[m].y;
-                if constexpr (GROUPED) {
+                const float down = TINY ? down_scale(r.xf[m].y) : r.xf[m].y;
+                if constexpr (TINY && GROUPED) blk[m] *= down_rest(r.xf[m].y);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        acc[m][n][i] = __builtin_fmaf(r.sb[n][i / 2][i % 2 * 2 + 1], r.xf[m].x,
-                                                      __builtin_fmaf(r.sb[n][i / 2][i % 2 * 2], blk[m][i], acc[m][n][i]));
-                } else {
-                    acc[m][n] += blk[m];
+                for (int i = 0; i < 4; ++i) {
+                    if constexpr (GROUPED) {
+                        const float sc = r.sb[n][i / 2][i % 2 * 2];
+                        acc[m][n][i] = wt_add(acc[m][n][i], blk[m][i], T == 2 ? sc * down : sc, r.sb[n][i / 2][i % 2 * 2 + 1], r.xf[m].x);
+                    } else {
+                        acc[m][n][i] = wt_add<T>(acc[m][n][i], blk[m][i], r.xf[m].y);
+                    }
                 }
             }
         }
     };
     auto finish = [&](int m, int n, f4 v) __attribute__((always_inline)) {
         const int row = m0 + (wm * FM + m) * 16 + l16, col = n0 + (wn * FN + n) * 16 + 4 * q;
-        float down, sum;
-        if constexpr (INLINE) {
-            const float2 r = row_xr[(wm * FM + m) * 16 + l16];
-            down = r.x;
-            sum = r.y;
-        } else {
-            const vf4 r = a.xr[min(row, a.Mp - 1)];
-            down = r.x;
-            sum = r.y;
-        }
-        wt_store<GROUPED, XF32>(c, row, col, v, down, sum);
+        float sum = 0.0f;
+        if (!GROUPED && c.w_zp) sum = INLINE ? row_xr[(wm * FM + m) * 16 + l16] : a.xr[min(row, a.Mp - 1)].x;
+        wt_store<GROUPED, XF32>(c, row, col, v, sum);
     };
 
     if constexpr (INLINE) {
@@ -553,7 +548,7 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
                 for (int b = 0; b < NG; ++b) {
                     Frags r;
                     read(r, lds, b);
-                    products(r, std::integral_constant<bool, T == 2>{});  // factors of 1 change nothing
+                    products(r, std::integral_constant<bool, GROUPED && T == 2>{});  // (the rest of 1 changes nothing)
                 }
                 if (t % WT_FLUSH == WT_FLUSH - 1 || t == n - 1) flush(t < WT_FLUSH);
             }
@@ -578,7 +573,7 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
         load(st, k0);
         store(st, 0);
         load(st, k0 + min(1, n - 1));
-        auto walk = [&](auto own) __attribute__((always_inline)) {
+        auto walk = [&](auto tiny) __attribute__((always_inline)) {
             for (int t = 0; t < n; ++t) {
                 block_barrier();  // stage t is in LDS; the other slot has been read
                 store(st, (t + 1) & 1);
@@ -587,17 +582,16 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
                 for (int b = 0; b < NG; ++b) {
                     Frags r;
                     read(r, lds + (t & 1) * STAGE, b);
-                    products(r, own);
+                    products(r, tiny);
                 }
                 if (t % WT_FLUSH == WT_FLUSH - 1 || t == n - 1) flush(t < WT_FLUSH);
             }
         };
         // one test per workgroup: a test per block would wait for the factors before every product
-        // (141 against 109 us at M = 1024, N = K = 4096, 8 bits)
-        bool own = false;
-        if (T == 2) own = __syncthreads_or(tid < BM && a.xr[min(m0 + tid, a.Mp - 1)].z != 0.0f);
-        if (own) walk(std::integral_constant<bool, T == 2>{});
-        else walk(std::false_type{});
+        if (GROUPED && T == 2 && __syncthreads_or(tid < BM && a.xr[min(m0 + tid, a.Mp - 1)].y != 0.0f))
+            walk(std::integral_constant<bool, GROUPED && T == 2>{});
+        else
+            walk(std::false_type{});
         if (a.part) {
             f4* dst = reinterpret_cast<f4*>(a.part) + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * FM * FN * 64 * W + tid;
 #pragma unroll
@@ -626,7 +620,7 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_reduce_kernel(WtArgs a) 
     const int col = tn * 16 * WN * FN + (wave % WN * FN + n) * 16 + 4 * q;
     const f4* src = reinterpret_cast<const f4*>(a.part) + ((int64_t)blockIdx.x * FM * FN + blockIdx.y) * 64 * W + tid;
     const int64_t stride = (int64_t)gridDim.x * FM * FN * 64 * W;
-    const vf4 xr = a.xr[min(row, a.Mp - 1)];
+    const float sum = !GROUPED && a.c.w_zp ? a.xr[min(row, a.Mp - 1)].x : 0.0f;
     f4 v = src[0];
     int r = 1;
     for (; r + 3 < a.ranges; r += 4) {
@@ -634,7 +628,7 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_reduce_kernel(WtArgs a) 
         v += p0; v += p1; v += p2; v += p3;
     }
     for (; r < a.ranges; ++r) v += src[r * stride];
-    wt_store<GROUPED, XF32>(a.c, row, col, v, xr.x, xr.y);
+    wt_store<GROUPED, XF32>(a.c, row, col, v, sum);
 }
 
 // ------------------------------------------------------------------ host side
@@ -666,7 +660,7 @@ WtPlan wt_plan(int64_t M, int64_t N, int64_t K, bool xf32, int gs) {
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     p.xp = up((size_t)Mp * p.KB * 128 * T);
     p.xm = up((size_t)p.KB * NG * 2 * Mp * 4);
-    p.xr = up((size_t)Mp * 16);
+    p.xr = up((size_t)Mp * 8);
     p.sb = gs ? up((size_t)(K / gs) * 8 * (size_t)(p.tiles_n * p.BN)) : 0;
     p.part = p.ranges > 1 ? up((size_t)p.ranges * t * p.BM * p.BN * 4) : 0;
     return p;
@@ -677,7 +671,7 @@ void wt_go(const WtPlan& p, WtArgs& a, hipStream_t st) {
     const unsigned t = (unsigned)(p.tiles_m * p.tiles_n);
     const unsigned scale_blocks = GROUPED ? (unsigned)((a.G + 31) / 32) * (unsigned)(a.Np / 32) : 0;
     hipLaunchKernelGGL((wo_tile_prep_kernel<BITS, S, T, GROUPED, HM>), dim3((unsigned)a.Mp + scale_blocks), dim3(256), 0, st, a,
-                       const_cast<char*>(a.xp), const_cast<float2*>(a.xm), const_cast<vf4*>(a.xr),
+                       const_cast<char*>(a.xp), const_cast<float2*>(a.xm), const_cast<float2*>(a.xr),
                        const_cast<float2*>(a.sb));
     hipLaunchKernelGGL((wo_tile_kernel<BITS, S, T, GROUPED, HM, WM, WN, FM, FN, false>), dim3(t, (unsigned)p.ranges),
                        dim3(64 * WM * WN), 0, st, a);
@@ -752,7 +746,7 @@ int wo_tile_launch(const WoTileCall& c, void* ws, size_t ws_bytes, hipStream_t s
         char* b = static_cast<char*>(ws);
         a.xp = b;
         a.xm = reinterpret_cast<const float2*>(b + p.xp);
-        a.xr = reinterpret_cast<const vf4*>(b + p.xp + p.xm);
+        a.xr = reinterpret_cast<const float2*>(b + p.xp + p.xm);
         a.sb = reinterpret_cast<const float2*>(b + p.xp + p.xm + p.xr);
         a.part = p.part ? reinterpret_cast<float*>(b + p.xp + p.xm + p.xr + p.sb) : nullptr;
     }

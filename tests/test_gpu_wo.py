@@ -433,6 +433,56 @@ def test_wo_tiles(gpu, bits, gs, M, N, K, half):
         assert abs(outs[0][1, 0] - want) <= 1e-5 * (abs(prod[1, 0]) + abs(b[0]))
 
 
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("bits,gs", [(8, 0), (8, 64), (4, 64), (8, 32), (4, 128)])
+@pytest.mark.parametrize("M,N,K", [(40, 5504, 2048), (200, 2048, 2112)])
+def test_wo_tiles_range(gpu, M, N, K, bits, gs, workspace):
+    """Every output against sum |x| |w| of its own, where a block's largest value and a row's meet zero
+    weights: a value keeps its bits down to 2^-17 of its block's largest (22 of them, so 2^-22 a
+    product, and as much again for the additions), whatever lies in the row's other blocks.  Rows of any
+    magnitude, and blocks whose scale leaves the range of a factor."""
+    from lucid_amd import _C
+
+    if K % max(gs, 1):
+        K = K // gs * gs
+    rng = np.random.default_rng(M + bits + gs)
+    x = (rng.standard_normal((M, K)) * 2.0 ** -12).astype(np.float32)
+    x[:, ::32] = 1.0          # the largest of every block
+    x[:, 64:128] *= 2.0 ** 15  # and of every row
+    x[1] *= np.float32(1e25)
+    x[2] *= np.float32(1e-25)
+    x[3, 256:512] *= np.float32(1e-30)
+    codes = rng.integers(1, 2 ** bits, (N, K))
+    codes[:, ::32] = 0
+    codes[:, 64:128] = 0
+    codes[: N // 2, :256] = 0
+    codes[: N // 2, 512:] = 0  # only the quiet blocks
+    s = rng.uniform(1e-3, 1e-1, (N, K // gs if gs else 1)).astype(np.float32)
+    xd, ds = _t(gpu, x), _t(gpu, s)
+    y = gpu.empty((M, N), np.float32, "gpu")
+    if gs == 0:
+        W = np.where(codes > 127, codes - 256, codes).astype(np.int8)
+        wd = W.astype(np.float64) * s
+        n = _C.lib().lq_gemv_w8_workspace_size(M, N, K) if workspace else 0
+        ws = gpu.empty((max(n, 16),), np.uint8, "gpu")
+        _C.call("lq_gemv_w8", xd.data_ptr(), _C.F32, K, _t(gpu, W).data_ptr(), K, ds.data_ptr(), None, None, y.data_ptr(), N,
+                M, N, K, 0, ws.data_ptr() if n else None, n, None)
+    else:
+        wd = codes * np.repeat(s, gs, 1).astype(np.float64)
+        per = 32 // bits
+        words = (codes.reshape(N, K // per, per).astype(np.uint64) << (np.arange(per, dtype=np.uint64) * bits)).sum(2)
+        packed = _t(gpu, words.astype(np.uint32).view(np.int32))
+        n = _C.lib().lq_group_matmul_workspace_size(M, N, K, gs) if workspace else 0
+        ws = gpu.empty((max(n, 16),), np.uint8, "gpu")
+        _C.call("lq_group_matmul", xd.data_ptr(), _C.F32, K, packed.data_ptr(), ds.data_ptr(), None, None, y.data_ptr(), N, M,
+                N, K, gs, bits, 1, 0, ws.data_ptr() if n else None, n, None)
+    assert _C.last_path().startswith("wo tiles") and (_C.last_path() == "wo tiles inline") == (not workspace)
+    x = x.astype(np.float64)
+    got = y.numpy()
+    assert np.all(np.abs(got - x @ wd.T) <= (np.abs(x) @ np.abs(wd).T) * 2.0 ** -21)
+    assert np.all(got != 0.0)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("gs", [32, 64, 128])
 @pytest.mark.parametrize("M,N,K", [(16, 4096, 4096), (5, 4608, 4096), (12, 1000, 2048)])
