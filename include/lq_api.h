@@ -406,11 +406,13 @@ int lq_row_sums_i8(const int8_t* d_X, int64_t ld, int64_t rows, int64_t K, int32
  * (lucid/nn/quantized/linear.py:206-210 -> lucid/_C/nn/Linear.cpp:199), without forming
  * the float weight.  x / y of x_dtype (LQ_F32 or LQ_F16), W int8 [N, ldw] row-major,
  * d_w_zero_point / d_bias may be NULL.  Float32 accumulation (tolerance parity: the float
- * GEMM's summation order is the reference's own).  Any M; tuned for M <= 16.  With
- * lq_gemv_w8_workspace_size(M, N, K) bytes of device workspace (16-byte aligned; 0 for M <= 2)
- * float32 activations of M > 8 rows are split into fp16 halves once per call instead of once
- * per workgroup (for fewer rows the in-workgroup split is faster and the workspace is not
- * touched); without it (NULL) the call still runs, with identical results. */
+ * GEMM's summation order is the reference's own).  Any M; tuned for M <= 16.
+ * lq_gemv_w8_workspace_size(M, N, K) bytes of device workspace (16-byte aligned; 0 for M <= 2) serve
+ * three forms: 3 to 16 rows whose K ranges are summed by several workgroups; float32 activations of more
+ * than 8 rows split into fp16 halves once per call instead of once per workgroup; and, for more
+ * than 16 rows of a large weight, either type of activations put in the order a tiled kernel reads.  Without
+ * it (NULL, or fewer bytes) the call still runs, slower; above 16 rows with identical results, up to 16 the
+ * order of the additions may differ. */
 size_t lq_gemv_w8_workspace_size(int64_t M, int64_t N, int64_t K);
 int lq_gemv_w8(const void* d_x, int x_dtype, int64_t ldx, const int8_t* d_W, int64_t ldw,
                const float* d_w_scale, const float* d_w_zero_point, const float* d_bias,
@@ -453,12 +455,13 @@ int lq_group_dequantize_f32(const uint32_t* d_packed, const float* d_scales,
  * for bfloat16: a caller with bfloat16 activations widens x to float32 (exact, lq_cast),
  * calls with this flag and narrows y (exact: y is bfloat16-valued).
  * transpose = 0: y[m,k] = sum_n x[m,n] w_hat[n,k] (+ bias[k]) with x [M, N] (ldx >= N) and
- * y [M, K] (ldy >= K), w_hat tiles dequantized as lq_group_dequantize_f32 writes them -- the
- * transpose=false product and the QLoRA input gradient dX = dY dequant(W) of the transpose=1
- * product (QuantizedMatmulBackward::apply, QuantizedMatmul.cpp:73-90); no workspace.
+ * y [M, K] (ldy >= K), w_hat as lq_group_dequantize_f32 writes it, float32 precision per product at
+ * any magnitude -- the transpose=false product and the QLoRA input gradient dX = dY dequant(W) of the
+ * transpose=1 product (QuantizedMatmulBackward::apply, QuantizedMatmul.cpp:73-90); no workspace.
  * d_biases (group offsets) and d_bias (layer bias) may be NULL.
- * lq_group_matmul_workspace_size(M, N, K, group_size) bytes of workspace let float32
- * activations be split once per call for transpose = 1 (as for lq_gemv_w8; NULL still runs). */
+ * lq_group_matmul_workspace_size(M, N, K, group_size) bytes of workspace serve transpose = 1 as
+ * lq_gemv_w8_workspace_size's do there, with the group scales and biases transposed beside the activations;
+ * NULL or fewer bytes still run. */
 size_t lq_group_matmul_workspace_size(int64_t M, int64_t N, int64_t K, int group_size);
 int lq_group_matmul(const void* d_x, int x_dtype, int64_t ldx, const uint32_t* d_packed,
                     const float* d_scales, const float* d_biases, const float* d_bias, void* d_y,

@@ -23,8 +23,7 @@
 // be a normal number, so below 2^-90 the rest of it goes to blk.  One scale for the whole row instead took
 // 117 us, and lost bits of values far below the row's largest.
 // Few tiles: K is split into ranges over workgroups, their sums added in range order by
-// wo_tile_reduce_kernel.  Without a workspace the same sums are made by workgroups that split
-// the activations themselves and walk the ranges in order: the same bits, slower.
+// wo_tile_reduce_kernel.  Without a workspace wo_tile_direct_kernel makes the same sums: the same bits.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -290,21 +289,19 @@ __device__ __forceinline__ void wt_store(const WoTileCall& c, int m, int n, f4 v
     }
 }
 
-// HM: the group scales' rounding (LQ_ROUND_*), a constant so that none costs nothing.
-template <int BITS, int S, int T, bool GROUPED, int HM, int WM, int WN, int FM, int FN, bool INLINE>
+template <int BITS, int S, int T, bool GROUPED, int WM, int WN, int FM, int FN>
 __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
     constexpr int W = WM * WN, BM = 16 * WM * FM, BN = 16 * WN * FN, NG = wt_blocks<S>();
     constexpr int A_BYTES = BM * 128 * T, B_BYTES = BN * 8 * BITS;
     constexpr int SB_BYTES = GROUPED ? NG * 2 * BN * 4 : 0, XF_BYTES = NG * 2 * BM * 4;
     constexpr int STAGE = A_BYTES + B_BYTES + SB_BYTES + XF_BYTES;
-    constexpr int NST = INLINE ? 1 : 2, NT = 64 * W;
+    constexpr int NST = 2, NT = 64 * W;
     // 16-byte pieces per thread and stage, then pairs (scale, bias; block sum, factor)
     constexpr int A_I = (A_BYTES + 16 * NT - 1) / (16 * NT), B_I = (B_BYTES + 16 * NT - 1) / (16 * NT);
     constexpr int F_N = (SB_BYTES + XF_BYTES) / 8, F_I = (F_N + NT - 1) / NT;
     constexpr int TOT_BYTES = BM * BN * 4;
-    static_assert(NST * STAGE + TOT_BYTES + (INLINE ? 4 * BM : 0) <= 160 * 1024, "LDS");
+    static_assert(NST * STAGE + TOT_BYTES <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) char lds[NST * STAGE + TOT_BYTES];
-    __shared__ float row_xr[INLINE ? BM : 1];
     const WoTileCall& c = a.c;
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -316,7 +313,7 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
     // ---- one stage: global memory -> registers -> LDS (LDS-DMA copies, with the scales gathered
     // from their rows, took 178 us where this form took 157, at M = 1024, four waves)
     struct Stage {
-        vu4 x[INLINE ? 1 : A_I];
+        vu4 x[A_I];
         vu4 w[B_I];
         float2 f[F_I];
     };
@@ -331,15 +328,13 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
         b_row[u] = c.w + (int64_t)min(n0 + r, c.N - 1) * c.ldw_bytes;
         b_chunk[u] = (BITS == 8 ? l >> 4 : (l >> 4) & 1) * 16;
     }
-    const char* a_ptr[INLINE ? 1 : A_I];
-    if constexpr (!INLINE) {
+    const char* a_ptr[A_I];
 #pragma unroll
-        for (int u = 0; u < A_I; ++u) {
-            // the piece's place in LDS (fragment order) -> its place in its row
-            const int i = (tid + u * NT) % (A_BYTES / 16), fr = i >> 6, l = i & 63;
-            const int m = min(m0 + fr / (2 * T) * 16 + (l & 15), a.Mp - 1);
-            a_ptr[u] = a.xp + (int64_t)m * a.KB * 128 * T + (fr % (2 * T) * 4 + (l >> 4)) * 16;
-        }
+    for (int u = 0; u < A_I; ++u) {
+        // the piece's place in LDS (fragment order) -> its place in its row
+        const int i = (tid + u * NT) % (A_BYTES / 16), fr = i >> 6, l = i & 63;
+        const int m = min(m0 + fr / (2 * T) * 16 + (l & 15), a.Mp - 1);
+        a_ptr[u] = a.xp + (int64_t)m * a.KB * 128 * T + (fr % (2 * T) * 4 + (l >> 4)) * 16;
     }
     const float2* f_ptr[F_I];  // the first stage's pair and the stages' distance
     int64_t f_step[F_I];
@@ -357,10 +352,8 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
         }
     }
     auto load = [&](Stage& s, int kb) __attribute__((always_inline)) {
-        if constexpr (!INLINE) {
 #pragma unroll
-            for (int u = 0; u < A_I; ++u) s.x[u] = *reinterpret_cast<const vu4*>(a_ptr[u] + (int64_t)kb * 128 * T);
-        }
+        for (int u = 0; u < A_I; ++u) s.x[u] = *reinterpret_cast<const vu4*>(a_ptr[u] + (int64_t)kb * 128 * T);
 #pragma unroll
         for (int u = 0; u < B_I; ++u)
             s.w[u] = *reinterpret_cast<const vu4*>(b_row[u] + min(kb * 8 * BITS + b_chunk[u], row_bytes - 16));
@@ -369,62 +362,25 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
             const int i = pair(u);
             if (GROUPED && i < SB_BYTES / 8) {
                 const int blk = i / BN, g = min((kb * 64 + blk * 32) / c.gs, a.G - 1);
-                if constexpr (INLINE) {
-                    const int64_t at = (int64_t)min(n0 + i % BN, c.N - 1) * a.G + g;
-                    s.f[u] = make_float2(round_to(c.w_scale[at], HM), c.g_bias ? round_to(c.g_bias[at], HM) : 0.0f);
-                } else {
-                    s.f[u] = f_ptr[u][(int64_t)(g - blk) * a.Np];
-                }
-            } else if constexpr (!INLINE) {
+                s.f[u] = f_ptr[u][(int64_t)(g - blk) * a.Np];
+            } else {
                 s.f[u] = f_ptr[u][kb * f_step[u]];
             }
         }
     };
     auto store = [&](const Stage& s, int slot) __attribute__((always_inline)) {
         char* base = lds + slot * STAGE;
-        if constexpr (!INLINE) {
 #pragma unroll
-            for (int u = 0; u < A_I; ++u) *reinterpret_cast<vu4*>(base + (tid + u * NT) % (A_BYTES / 16) * 16) = s.x[u];
-        }
+        for (int u = 0; u < A_I; ++u) *reinterpret_cast<vu4*>(base + (tid + u * NT) % (A_BYTES / 16) * 16) = s.x[u];
 #pragma unroll
         for (int u = 0; u < B_I; ++u) *reinterpret_cast<vu4*>(base + A_BYTES + (tid + u * NT) % (B_BYTES / 16) * 16) = s.w[u];
 #pragma unroll
         for (int u = 0; u < F_I; ++u) {
-            const int i = pair(u);
-            if (!INLINE || i < SB_BYTES / 8) reinterpret_cast<float2*>(base + A_BYTES + B_BYTES)[i] = s.f[u];
+            reinterpret_cast<float2*>(base + A_BYTES + B_BYTES)[pair(u)] = s.f[u];
         }
     };
 
-    // ---- the activation rows' sums, where no prepared copy holds them
     constexpr bool XF32 = T == 2;
-    const bool vec = INLINE && x_vec<XF32>(c);
-    if (INLINE && !GROUPED && c.w_zp) {
-        for (int r = wave; r < BM; r += W) {
-            const float sum = row_sum<XF32>(c, m0 + r, lane, vec);
-            if (lane == 0) row_xr[r] = sum;
-        }
-        __syncthreads();
-    }
-    auto stage_inline = [&](int kb) __attribute__((always_inline)) {
-        char* base = lds;
-        for (int i = tid; i < BM * 8; i += 64 * W) {
-            const int r = i >> 3, o = i & 7;
-            float v[8];
-            load_octet<XF32>(c, m0 + r, kb * 64 + o * 8, vec, v);
-            h8 x[T];
-            float bsum, down;
-            split_octet<BITS, S, T>(v, x, bsum, down);
-            int step, qq;
-            octet_pos<S>(o, step, qq);
-            h8* dst = reinterpret_cast<h8*>(base) + ((r >> 4) * 2 + step) * T * 64 + qq * 16 + (r & 15);
-#pragma unroll
-            for (int t = 0; t < T; ++t) dst[64 * t] = x[t];
-            if ((o & (4 * S - 1)) == 0) {
-                reinterpret_cast<float2*>(base + A_BYTES + B_BYTES + SB_BYTES)[o / (4 * S) * BM + r] = make_float2(bsum, down);
-            }
-        }
-    };
-
     // ---- one stage's products
     // two levels of sums: acc over WT_FLUSH stages, tot over those, in LDS (a chain of all K / 64
     // additions would lose about a bit against the GEMV kernels' sums per wave)
@@ -527,44 +483,11 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
     };
     auto finish = [&](int m, int n, f4 v) __attribute__((always_inline)) {
         const int row = m0 + (wm * FM + m) * 16 + l16, col = n0 + (wn * FN + n) * 16 + 4 * q;
-        float sum = 0.0f;
-        if (!GROUPED && c.w_zp) sum = INLINE ? row_xr[(wm * FM + m) * 16 + l16] : a.xr[min(row, a.Mp - 1)].x;
+        const float sum = !GROUPED && c.w_zp ? a.xr[min(row, a.Mp - 1)].x : 0.0f;
         wt_store<GROUPED, XF32>(c, row, col, v, sum);
     };
 
-    if constexpr (INLINE) {
-        f4 sum[FM][FN];
-        for (int r = 0; r < a.ranges; ++r) {
-            clear();
-            const int k0 = r * a.rs, n = min(a.rs, a.KB - k0);
-            for (int t = 0; t < n; ++t) {
-                __syncthreads();
-                Stage st;
-                load(st, k0 + t);
-                stage_inline(k0 + t);
-                store(st, 0);
-                __syncthreads();
-#pragma unroll
-                for (int b = 0; b < NG; ++b) {
-                    Frags r;
-                    read(r, lds, b);
-                    products(r, std::integral_constant<bool, GROUPED && T == 2>{});  // (the rest of 1 changes nothing)
-                }
-                if (t % WT_FLUSH == WT_FLUSH - 1 || t == n - 1) flush(t < WT_FLUSH);
-            }
-#pragma unroll
-            for (int m = 0; m < FM; ++m)
-#pragma unroll
-                for (int nn = 0; nn < FN; ++nn) {
-                    const f4 v = tot[(m * FN + nn) * NT];
-                    sum[m][nn] = r ? sum[m][nn] + v : v;
-                }
-        }
-#pragma unroll
-        for (int m = 0; m < FM; ++m)
-#pragma unroll
-            for (int nn = 0; nn < FN; ++nn) finish(m, nn, sum[m][nn]);
-    } else {
+    {
         const int k0 = blockIdx.y * a.rs, n = min(a.rs, a.KB - k0);
         clear();
         // stage t + 1 goes from registers to LDS and stage t + 2 from memory to registers while
@@ -604,6 +527,232 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
 #pragma unroll
                 for (int nn = 0; nn < FN; ++nn) finish(m, nn, tot[(m * FN + nn) * NT]);
         }
+    }
+}
+
+// ---- the same sums without a workspace
+//
+// The tiled kernel adds K / 512 or more groups of up to WT_FLUSH stages, first within a range, then the
+// ranges.  Here each wave makes whole groups of 32 rows x 16 FN columns, of activations that it splits itself,
+// straight from memory; GW waves share a row tile's groups, and the sums meet in LDS in that order.  Within a
+// group nothing waits for another wave.  FN = 4 splits x once for 64 columns, FN = 1 fills the chip where tiles are
+// few; GW = 2 keeps the waves busy where a row tile has few groups.
+// N = K = 4096, 8 bits, groups of 64, float32 x (the kernel for few rows, then the tiled kernel in its form that split x
+// in every workgroup, which this replaced): M = 33 40 and 126 -> 27 us, M = 128 106 and 131 -> 34, M = 1024
+// 822 and 285 -> 233; half x M = 33 25 and 117 -> 19; M = 2048, N = K = 1024 98 and 52 -> 35.  Only groups of 32 and per-channel weights at M = 1024 were
+// faster there (235 and 187 against 332 and 212).
+constexpr int WD_WAVES = 8, WD_FM = 2;
+
+template <int BITS, int S, int T, bool GROUPED, int HM, int FN, int GW>
+__global__ __launch_bounds__(64 * WD_WAVES) void wo_tile_direct_kernel(WtArgs a) {
+    constexpr int NG = wt_blocks<S>(), FM = WD_FM, BM = 16 * FM, BN = 16 * FN, SLOTS = FM * FN * 64;
+    constexpr int WB = S * BITS;  // weight bytes of a lane's part of a block
+    constexpr bool XF32 = T == 2;
+    constexpr int RT = WD_WAVES / GW, ST = (SLOTS + 64 * GW - 1) / (64 * GW);  // row tiles, fours of outputs a finishing thread
+    constexpr int GG = WT_FLUSH * (S == 2 ? 1 : 2);  // most group scales of a column in WT_FLUSH stages
+    __shared__ f4 red[WD_WAVES][SLOTS];
+    __shared__ float rows[RT * BM];
+    __shared__ __attribute__((aligned(16))) float2 scales[GROUPED ? WD_WAVES : 1][GROUPED ? GG * BN : 1];  // [group][column]
+    const WoTileCall& c = a.c;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rt = wave / GW, gw = wave % GW;  // this wave's row tile, and which of its waves it is
+    const int m0 = (blockIdx.y * RT + rt) * BM, n0 = blockIdx.x * BN;
+    const bool vec = x_vec<XF32>(c);
+    const int row_bytes = c.K * BITS / 8;
+    if (!GROUPED && c.w_zp) {
+        for (int r = wave; r < RT * BM; r += WD_WAVES) {
+            const float sum = row_sum<XF32>(c, blockIdx.y * RT * BM + r, lane, vec);
+            if (lane == 0) rows[r] = sum;
+        }
+    }
+    // the group scales and biases of stages k0 .. k0 + n of this wave's columns
+    const int sg = GROUPED ? c.gs : 64;
+    auto load_scales = [&](int k0, int n) __attribute__((always_inline)) {
+        const int g0 = k0 * 64 / sg, ng = min((k0 + n) * 64 - 1, c.K - 1) / sg - g0 + 1;
+        for (int i = lane; i < GG * BN; i += 64) {
+            const int g = i % GG, col = i / GG;
+            if (g < ng) {
+                const int64_t at = (int64_t)min(n0 + col, c.N - 1) * a.G + g0 + g;
+                scales[wave][g * BN + col] = make_float2(round_to(c.w_scale[at], HM), c.g_bias ? round_to(c.g_bias[at], HM) : 0.0f);
+            }
+        }
+    };
+    struct Raw {
+        vu4 x[FM][2][T];  // the stage's two octets of a lane's rows
+        uint32_t w[FN][NG][WB / 4];
+    };
+    // octet j of a lane in a stage: of one block of 64 the lane quarter holds 16 consecutive k, of each
+    // block of 32 eight
+    auto octet = [&](int j) __attribute__((always_inline)) { return S == 2 ? 2 * q + j : 4 * j + q; };
+    auto load = [&](Raw& r, int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < FM; ++m) {
+            const int row = min(m0 + 16 * m + l16, c.M - 1);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {  // K is a multiple of 8: whole octets, zeroed past K where they are used
+                const int64_t at = (int64_t)row * c.ldx + min(kb * 64 + octet(j) * 8, c.K - 8);
+                if (vec) {
+                    const vu4* p = reinterpret_cast<const vu4*>(static_cast<const uint8_t*>(c.x) + at * (XF32 ? 4 : 2));
+#pragma unroll
+                    for (int t = 0; t < T; ++t) r.x[m][j][t] = p[t];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4 * T; ++i) {
+                        if constexpr (XF32) {
+                            r.x[m][j][i / 4][i % 4] = static_cast<const uint32_t*>(c.x)[at + i];
+                        } else {
+                            const uint16_t* p = static_cast<const uint16_t*>(c.x) + at + 2 * i;
+                            r.x[m][j][0][i] = p[0] | (uint32_t)p[1] << 16;
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < FN; ++n) {
+            const uint8_t* p = c.w + (int64_t)min(n0 + 16 * n + l16, c.N - 1) * c.ldw_bytes;
+#pragma unroll
+            for (int b = 0; b < NG; ++b) {  // past the row's end: its last bytes, which meet zeros
+                const uint8_t* s = p + min((kb * NG + b) * 4 * WB + q * WB, row_bytes - WB);
+                if constexpr (WB == 16) {
+                    const vu4 v = *reinterpret_cast<const vu4*>(s);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) r.w[n][b][i] = v[i];
+                } else if constexpr (WB == 8) {
+                    const u2v v = *reinterpret_cast<const u2v*>(s);
+                    r.w[n][b][0] = v.x;
+                    r.w[n][b][1] = v.y;
+                } else {
+                    r.w[n][b][0] = *reinterpret_cast<const uint32_t*>(s);
+                }
+            }
+        }
+    };
+    f4 acc[FM][FN];
+    auto add = [&](const Raw& r, int kb, int kg) __attribute__((always_inline)) {  // kg: the group's first stage
+#pragma unroll
+        for (int b = 0; b < NG; ++b) {
+            h8 x[FM][S][T];
+            float bsum[FM], down[FM];
+#pragma unroll
+            for (int m = 0; m < FM; ++m) {
+                const bool row = m0 + 16 * m + l16 < c.M;
+                float v[S][8], am = 0.0f, up;
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    const int o = S == 2 ? j : b;
+                    const bool in = row && kb * 64 + octet(o) * 8 < c.K;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        float f;
+                        if constexpr (XF32) f = __uint_as_float(r.x[m][o][i / 4][i % 4]);
+                        else f = (float)bits_h2(r.x[m][o][0][i / 2])[i % 2];
+                        v[j][i] = in ? f : 0.0f;
+                    }
+                    bsum[m] = j ? bsum[m] + octet_sum(v[j]) : octet_sum(v[j]);
+                    am = fmaxf(am, octet_amax(v[j]));
+                }
+                // the additions of split_octet: octet pairs, then lane quarters 1 and 2 apart
+#pragma unroll
+                for (int off = 16; off < 64; off <<= 1) {
+                    bsum[m] += __shfl_xor(bsum[m], off, 64);
+                    am = fmaxf(am, __shfl_xor(am, off, 64));
+                }
+                block_scale<T>(am, up, down[m]);
+#pragma unroll
+                for (int j = 0; j < S; ++j) octet_terms<BITS, T>(v[j], up, x[m][j]);
+            }
+            const int g = GROUPED ? min(kb * 64 + b * 32, c.K - 1) / sg - kg * 64 / sg : 0;
+#pragma unroll
+            for (int n = 0; n < FN; ++n) {
+                f4 sb[2];  // {scale, bias} of columns 4 q .. 4 q + 3
+                if constexpr (GROUPED) {
+                    const f4* p = reinterpret_cast<const f4*>(&scales[wave][g * BN + 16 * n + 4 * q]);
+                    sb[0] = p[0];
+                    sb[1] = p[1];
+                }
+                h8 wa[S];
+#pragma unroll
+                for (int j = 0; j < S; ++j) wa[j] = unpack_step<BITS, !GROUPED>(&r.w[n][b][j * BITS / 4]);
+                f4 blk[FM];
+#pragma unroll
+                for (int m = 0; m < FM; ++m) blk[m] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < S; ++j)
+#pragma unroll
+                    for (int t = 0; t < T; ++t)
+#pragma unroll
+                        for (int m = 0; m < FM; ++m) blk[m] = mfma16(wa[j], x[m][j][t], blk[m]);
+#pragma unroll
+                for (int m = 0; m < FM; ++m) {
+                    if constexpr (T == 2 && GROUPED) blk[m] *= down_rest(down[m]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if constexpr (GROUPED) {
+                            const float sc = sb[i / 2][i % 2 * 2];
+                            acc[m][n][i] = wt_add(acc[m][n][i], blk[m][i], T == 2 ? sc * down_scale(down[m]) : sc,
+                                                  sb[i / 2][i % 2 * 2 + 1], bsum[m]);
+                        } else {
+                            acc[m][n][i] = wt_add<T>(acc[m][n][i], blk[m][i], down[m]);
+                        }
+                    }
+                }
+            }
+        }
+    };
+    const int per = (a.rs + WT_FLUSH - 1) / WT_FLUSH;  // groups of a range
+    auto first = [&](int g) { return g / per * a.rs + g % per * WT_FLUSH; };
+    auto count = [&](int g) { return min(WT_FLUSH, min((g / per + 1) * a.rs, a.KB) - first(g)); };  // none: <= 0
+    f4 tot[ST], sum[ST];  // of a range, of the ranges before
+    const int groups = a.ranges * per, slot0 = gw * 64 + lane;
+    for (int g0 = 0; g0 < groups; g0 += GW) {
+        const int g = g0 + gw, k0 = first(g), n = g < groups && m0 < c.M ? count(g) : 0;
+        if (n > 0) {
+            if constexpr (GROUPED) load_scales(k0, n);
+#pragma unroll
+            for (int m = 0; m < FM; ++m)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[m][j] = f4{0.f, 0.f, 0.f, 0.f};
+            Raw r[2];
+            load(r[0], k0);
+            for (int t = 0; t < n; t += 2) {
+                load(r[1], k0 + min(t + 1, n - 1));
+                add(r[0], k0 + t, k0);
+                if (t + 1 < n) {
+                    load(r[0], k0 + min(t + 2, n - 1));
+                    add(r[1], k0 + t + 1, k0);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < FM; ++m)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) red[wave][(m * FN + j) * 64 + lane] = acc[m][j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < ST; ++u) {
+            const int slot = slot0 + u * 64 * GW;
+            if (slot < SLOTS)
+                for (int w = 0; w < GW && g0 + w < groups; ++w) {
+                    if (count(g0 + w) <= 0) continue;
+                    const f4 v = red[rt * GW + w][slot];
+                    if ((g0 + w) % per == 0) {
+                        if (g0 + w > 0) sum[u] = g0 + w > per ? sum[u] + tot[u] : tot[u];
+                        tot[u] = v;
+                    } else {
+                        tot[u] += v;
+                    }
+                }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < ST; ++u) {
+        const int slot = slot0 + u * 64 * GW, f = slot >> 6, ml = f / FN * 16 + l16;
+        if (slot < SLOTS)
+            wt_store<GROUPED, XF32>(c, m0 + ml, n0 + f % FN * 16 + 4 * q, groups > per ? sum[u] + tot[u] : tot[u],
+                                    !GROUPED && c.w_zp ? rows[rt * BM + ml] : 0.0f);
     }
 }
 
@@ -673,7 +822,7 @@ void wt_go(const WtPlan& p, WtArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((wo_tile_prep_kernel<BITS, S, T, GROUPED, HM>), dim3((unsigned)a.Mp + scale_blocks), dim3(256), 0, st, a,
                        const_cast<char*>(a.xp), const_cast<float2*>(a.xm), const_cast<float2*>(a.xr),
                        const_cast<float2*>(a.sb));
-    hipLaunchKernelGGL((wo_tile_kernel<BITS, S, T, GROUPED, HM, WM, WN, FM, FN, false>), dim3(t, (unsigned)p.ranges),
+    hipLaunchKernelGGL((wo_tile_kernel<BITS, S, T, GROUPED, WM, WN, FM, FN>), dim3(t, (unsigned)p.ranges),
                        dim3(64 * WM * WN), 0, st, a);
     if (p.ranges > 1)
         hipLaunchKernelGGL((wo_tile_reduce_kernel<GROUPED, T == 2, WM, WN, FM, FN>), dim3(t, FM * FN), dim3(64 * WM * WN), 0, st, a);
@@ -683,10 +832,25 @@ template <int BITS, int S, bool GROUPED>
 void wt_config(const WtPlan& p, WtArgs& a, bool inl, hipStream_t st) {
     auto go = [&](auto t, auto h) {
         constexpr int T = decltype(t)::value, HM = decltype(h)::value;
-        if (inl) {  // one tile size: an output's sums do not depend on it
-            a.tiles_m = (a.c.M + 31) / 32;
-            hipLaunchKernelGGL((wo_tile_kernel<BITS, S, T, GROUPED, HM, 1, 4, 2, 2, true>),
-                               dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(256), 0, st, a);
+        if (inl) {
+            // 64 columns a workgroup where that leaves none of the chip idle, then two waves a row tile where it
+            // has up to four groups
+            auto direct = [&](auto fn, auto gw) {
+                constexpr int FN = decltype(fn)::value, GW = decltype(gw)::value;
+                constexpr int BM = 16 * WD_FM * (WD_WAVES / GW);
+                hipLaunchKernelGGL((wo_tile_direct_kernel<BITS, S, T, GROUPED, HM, FN, GW>),
+                                   dim3((unsigned)((a.c.N + 16 * FN - 1) / (16 * FN)), (unsigned)((a.c.M + BM - 1) / BM)),
+                                   dim3(64 * WD_WAVES), 0, st, a);
+            };
+            using I1 = std::integral_constant<int, 1>;
+            using I2 = std::integral_constant<int, 2>;
+            using I4 = std::integral_constant<int, 4>;
+            using I8 = std::integral_constant<int, 8>;
+            auto groups = [&](int cols) { return (int64_t)((a.c.N + cols - 1) / cols) * ((a.c.M + 31) / 32); };
+            if (groups(32) < 256) direct(I1{}, I8{});
+            else if (groups(64) < 256) direct(I2{}, I8{});
+            else if (groups(64) < 1024) direct(I4{}, I8{});
+            else direct(I4{}, I2{});
         } else if (p.cfg == WT_128) wt_go<BITS, S, T, GROUPED, HM, 2, 4, 4, 2>(p, a, st);
         else if (p.cfg == WT_64) wt_go<BITS, S, T, GROUPED, HM, 2, 4, 2, 2>(p, a, st);
         else wt_go<BITS, S, T, GROUPED, HM, 2, 4, 1, 2>(p, a, st);

@@ -365,7 +365,7 @@ def test_group_matmul_presplit_matches_inline(gpu, bits, gs):
 # and stages, K ranges and none
 WO_TILE_CASES = [(8, 0, 20, 4608, 4096), (8, 0, 64, 4099, 4096), (8, 0, 600, 1000, 1040), (8, 0, 1031, 515, 1040),
                  (8, 0, 2049, 2100, 272), (8, 64, 33, 4096, 4096), (8, 64, 1025, 2050, 512), (8, 128, 129, 2048, 2176),
-                 (8, 32, 300, 1900, 1056), (4, 32, 30, 4200, 4128), (4, 64, 700, 640, 2048), (4, 128, 2200, 2180, 384)]
+                 (8, 64, 1050, 4096, 1088), (8, 32, 300, 1900, 1056), (4, 32, 30, 4200, 4128), (4, 64, 700, 640, 2048), (4, 128, 2200, 2180, 384)]
 
 
 @pytest.mark.parametrize("half", [False, True])
@@ -431,6 +431,38 @@ def test_wo_tiles(gpu, bits, gs, M, N, K, half):
     if not half:  # the small blocks' result, without the large block's products
         want = max(prod[1, 0] + b[0], 0.0)
         assert abs(outs[0][1, 0] - want) <= 1e-5 * (abs(prod[1, 0]) + abs(b[0]))
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("M,N,K,gs", [(130, 2050, 2176, 0), (33, 4099, 4224, 64), (20, 9000, 4128, 32), (1100, 1000, 1152, 128)])
+def test_wo_tiles_unaligned_rows(gpu, M, N, K, gs, half):
+    """Activation rows at no 16-byte alignment, with and without a workspace: the bits of aligned
+    rows."""
+    from lucid_amd import _C
+
+    rng = np.random.default_rng(M + gs)
+    x = rng.standard_normal((M, K)).astype(np.float16 if half else np.float32)
+    W, s = _t(gpu, rng.integers(-128, 128, (N, K)).astype(np.int8)), _t(gpu, rng.uniform(1e-3, 1e-1, (N, K // gs if gs else 1)).astype(np.float32))
+    b = _t(gpu, rng.standard_normal((N, K // gs if gs else 1)).astype(np.float32))
+    size = _C.lib().lq_group_matmul_workspace_size(M, N, K, gs) if gs else _C.lib().lq_gemv_w8_workspace_size(M, N, K)
+    ws = gpu.empty((size,), np.uint8, "gpu")
+    outs = []
+    for ldx in (K, K + 1, K + 5):
+        wide = np.full((M, ldx), 7.0, x.dtype)
+        wide[:, :K] = x
+        xd = _t(gpu, wide)
+        for n in (size, 0):
+            y = gpu.empty((M, N), x.dtype, "gpu")
+            args = (xd.data_ptr(), _C.F16 if half else _C.F32, ldx, W.data_ptr())
+            end = (0, ws.data_ptr() if n else None, n, None)
+            if gs:
+                _C.call("lq_group_matmul", *args, s.data_ptr(), b.data_ptr(), None, y.data_ptr(), N, M, N, K, gs, 8, 1, *end)
+            else:
+                _C.call("lq_gemv_w8", *args, K, s.data_ptr(), b.data_ptr(), None, y.data_ptr(), N, M, N, K, *end)
+            assert _C.last_path().startswith("wo tiles")
+            outs.append(y.numpy())
+    for o in outs[1:]:
+        np.testing.assert_array_equal(o.view(np.uint16 if half else np.uint32), outs[0].view(np.uint16 if half else np.uint32))
 
 
 @pytest.mark.parametrize("workspace", [True, False])
