@@ -277,7 +277,7 @@ void wo_stream_launch(const WoTileCall& c, void* ws, hipStream_t st) {
         a.part_x = reinterpret_cast<float*>(static_cast<char*>(ws) + p.part);
     }
     c.xf32 ? ws_go<true>(a, st) : ws_go<false>(a, st);
-    note_path(p.ranges > 1 ? "wo packed split-k" : "wo packed split-k single range");
+    note_path(p.ranges > 1 ? "wo stream ranges" : "wo stream");
 }
 
 }  // namespace lq

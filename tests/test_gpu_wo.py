@@ -235,11 +235,11 @@ def run_gemv_packed(L, x, W, s, z=None, b=None, relu=False, half=False):
 
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("M,N,K", [(16, 4096, 4096), (1, 11008, 4096), (2, 4096, 11008), (8, 100, 784),
-                                   (3, 1000, 1024), (16, 70, 16), (5, 33, 528)])
+                                   (3, 1000, 1024), (16, 70, 16), (5, 33, 528), (12, 6000, 4096), (14, 500, 1504)])
 def test_gemv_w8_packed(gpu, M, N, K, half):
     """The decode entry over the MFMA-packed weight: against the oracle like lq_gemv_w8, with a
-    zero point, bias and ReLU, and bit for bit lq_gemv_w8 where that takes its split-K route
-    (same kernel, same products and order; only where the weight bytes come from differs)."""
+    zero point, bias and ReLU, and up to K = 4096 bit for bit lq_gemv_w8 where that takes its split-K
+    route (the same products and order, of the split-K pair and of the one pass)."""
     from lucid_amd import _C
 
     print(f"gemv packed M={M} N={N} K={K} half={half}", flush=True)
@@ -251,11 +251,11 @@ def test_gemv_w8_packed(gpu, M, N, K, half):
     z = rng.integers(-4, 5, N).astype(np.float32)
     b = rng.standard_normal(N).astype(np.float32)
     got = run_gemv_packed(gpu, x, W, s, z=z, b=b, relu=True, half=half)
-    assert _C.last_path() in ("wo packed split-k", "wo packed split-k single range")
+    assert _C.last_path() in (ONE, RANGES, SK, SK1)
     xr = x.astype(np.float16).astype(np.float32) if half else x
     _close(got, _gemv_ref(xr, W, s, z=z, b=b, relu=True), half=half)
     rowmajor = run_gemv(gpu, x, W, s, z=z, b=b, relu=True, half=half)
-    if _C.last_path() in ("wo split-k", "wo split-k single range"):
+    if K <= 4096 and _C.last_path() in ("wo split-k", "wo split-k single range"):
         np.testing.assert_array_equal(got.view(np.uint16 if half else np.uint32),
                                       rowmajor.view(np.uint16 if half else np.uint32))
 
@@ -965,12 +965,19 @@ def test_group_matmul_rows_in_segments(gpu, M, N, K, bits, gs, half):
     assert np.all(np.abs(y - ref) <= mag * 2.0**-18 + (np.abs(ref) * 2.0**-11 if half else 0.0))
 
 
-# lq_gemv_w8_packed in one pass: K ranges of one to eight waves, a last block or wave that is partial,
-# more than one K range, fewer columns than a tile and more tiles than CUs
+# lq_gemv_w8_packed, (M, N, K, path of float32 x, of half x): one pass with K ranges of one to eight
+# waves, a last block or wave that is partial, fewer columns than a tile and more tiles than CUs, more than
+# one K range of 4096; and the split-K pair
+ONE, RANGES, SK, SK1 = "wo stream", "wo stream ranges", "wo packed split-k", "wo packed split-k single range"
+
+
 @pytest.mark.parametrize("half", [False, True])
-@pytest.mark.parametrize("M,N,K", [(1, 7, 64), (3, 17, 512), (16, 4100, 1040), (9, 8200, 2064), (16, 300, 4080),
-                                   (2, 48, 4112), (16, 33, 8208)])
-def test_gemv_w8_packed_one_pass(gpu, M, N, K, half):
+@pytest.mark.parametrize("M,N,K,path,half_path", [
+    (1, 7, 64, ONE, ONE), (3, 17, 512, ONE, ONE), (16, 4100, 1040, ONE, ONE), (9, 8200, 2064, ONE, ONE),
+    (16, 300, 4080, SK, ONE), (2, 48, 4112, RANGES, RANGES), (16, 33, 8208, SK, RANGES), (5, 2000, 11008, RANGES, RANGES)])
+def test_gemv_w8_packed_one_pass(gpu, M, N, K, path, half_path, half):
+    from lucid_amd import _C
+
     rng = np.random.default_rng(M * 7 + N + K + half)
     x = rng.standard_normal((M, K)).astype(np.float32)
     x[:, ::53] *= 30.0
@@ -980,4 +987,5 @@ def test_gemv_w8_packed_one_pass(gpu, M, N, K, half):
     b = rng.standard_normal(N).astype(np.float32)
     xr = x.astype(np.float16).astype(np.float32) if half else x
     got = run_gemv_packed(gpu, x, W, s, z=z, b=b, half=half)
+    assert _C.last_path() == (half_path if half else path)
     _close(got, _gemv_ref(xr, W, s, z=z, b=b), half=half)
