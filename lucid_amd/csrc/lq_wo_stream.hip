@@ -248,17 +248,26 @@ void ws_go(const WsArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// Every workgroup reads all of x for its K range, and all of them the same lines: with 128 KB or more
-// of float32 x against a single tile of weights the split-K pair of launches is faster (M = 16,
-// N = K = 4096: 11.7 against 14.5 us; M = 8 10.8 against 11.5; M = 3 10.5 against 10.1), with a second
-// tile, a shorter K or half x this kernel is (N = 8192 17.8 -> 17.3, N = 11008 23.8 -> 19.6; K = 1024
-// 8.3 -> 5.5; half x 10.1 -> 9.0, N = 11008 19.6 -> 13.8, N = K = 1152 7.7 -> 5.2 us; weights from
-// memory).
+// Against wo_gemv_sk_kernel's pair of launches over the same weight (M = 1 to 16, N = 256 to 16384, K = 256 to
+// 14336, 1288 sizes, weights from memory; the rule's choice is within 5% of the faster one at all but 15, within 12%
+// at all):
+//  * K up to 512 is one launch there too: this one's second round of tiles costs more than a second round of
+//    its small workgroups (M = 1, K = 512: N = 4096 4.4 us here, 4.9 there; N = 8192 5.8 and 5.0; N = 16384 7.7 and 5.4).
+//  * Up to 2048 the second launch is what counts (M = 16, N = 4096: K = 1024 5.4 and 8.3; K = 2048 8.5 and 9.1).
+//  * Beyond, every wave reads and splits 512 k of x before its first product, 9 us with one row and 13 with 16,
+//    half x 5 to 8, and the weight has to be worth it (K = 4096: M = 1, N = 2048 8.8 and 8.6, N = 8192 12.4 and 15.6;
+//    M = 16, N = 2048 13.7 and 9.1, N = 6144 15.9 and 15.0, N = 8192 16.8 and 17.7; half x 16 x 512 8.1 and 7.2).
+//  * Ranges of 4096 that are not full leave their workgroups idle, most of all a second one that is all but
+//    empty (N = 8192, K = 4112: M = 1 18.2 and 16.6, M = 16 21.4 and 18.1, half x 15.1 and 15.8, 16.5 and 15.4;
+//    K = 8192, M = 1 23 and 29).
 bool wo_stream_preferred(int64_t M, int64_t N, int64_t K, bool xf32) {
     const WsPlan p = ws_plan(N, K);
-    if (!xf32) return true;
-    return M * std::min<int64_t>(K, 4096) * 4 < 128 * 1024 ||
-           p.tiles * p.ranges > device_cu_count();
+    const int64_t cus = device_cu_count();
+    if (K <= 512) return p.tiles <= (xf32 && M <= 8 ? cus : cus * 3 / 2);
+    if (K <= 2048) return true;
+    if (K > 4096 && (xf32 ? K < 5120 : M > 8 && K < 4608)) return false;
+    const double fill = p.ranges > 1 ? (double)K / (p.ranges * 4096.0) : 1.0;  // of the ranges
+    return 5.0 * N * K * fill > (double)((xf32 ? 68 + 4 * M : 4 * (M - 4)) * (1 << 20));
 }
 
 size_t wo_stream_ws_bytes(int64_t N, int64_t K) { return ws_plan(N, K).bytes; }

@@ -967,14 +967,15 @@ def test_group_matmul_rows_in_segments(gpu, M, N, K, bits, gs, half):
 
 # lq_gemv_w8_packed, (M, N, K, path of float32 x, of half x): one pass with K ranges of one to eight
 # waves, a last block or wave that is partial, fewer columns than a tile and more tiles than CUs, more than
-# one K range of 4096; and the split-K pair
+# one K range of 4096; and either side of each line to the split-K pair
 ONE, RANGES, SK, SK1 = "wo stream", "wo stream ranges", "wo packed split-k", "wo packed split-k single range"
 
 
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("M,N,K,path,half_path", [
-    (1, 7, 64, ONE, ONE), (3, 17, 512, ONE, ONE), (16, 4100, 1040, ONE, ONE), (9, 8200, 2064, ONE, ONE),
-    (16, 300, 4080, SK, ONE), (2, 48, 4112, RANGES, RANGES), (16, 33, 8208, SK, RANGES), (5, 2000, 11008, RANGES, RANGES)])
+    (1, 7, 64, ONE, ONE), (3, 17, 512, ONE, ONE), (8, 4112, 512, SK1, ONE), (16, 4112, 512, ONE, ONE), (3, 6200, 512, SK1, SK1),
+    (16, 4100, 1040, ONE, ONE), (9, 8200, 2064, SK, ONE), (12, 6000, 4096, ONE, ONE), (16, 300, 4080, SK, SK),
+    (2, 48, 4112, SK, RANGES), (9, 8200, 4112, SK, SK), (2, 700, 5120, SK, RANGES), (3, 5400, 5120, RANGES, RANGES), (16, 4096, 8208, SK, RANGES), (16, 33, 8208, SK, SK), (16, 3400, 8192, RANGES, RANGES), (5, 2000, 11008, RANGES, RANGES)])
 def test_gemv_w8_packed_one_pass(gpu, M, N, K, path, half_path, half):
     from lucid_amd import _C
 
