@@ -431,14 +431,19 @@ def test_gemm_gelu_rejects(gpu):
     (100, 512, 512, False, "dynamic quantize two-launch"),
     (4096, 8192, 256, False, "dynamic quantize two-launch"),
     (512, 1024, 192, True, "dynamic quantize two-launch"),
+    (4096, 2048, 400, True, "gemm dma with extrema + dynamic quantize"),   # a partial last stage: 256x128 tiles
+    (1500, 1600, 208, False, "gemm dma with extrema + dynamic quantize"),  # 128x128 tiles
+    (1500, 1600, 203, True, "gemm dma with extrema + dynamic quantize"),   # rows copied first
+    (512, 1024, 203, False, "dynamic quantize two-launch"),
 ])
 def test_gemm_dynamic_quantize_equals_calls(gpu, M, N, K, gelu, want):
     """lq_gemm_w8a8_dynamic_quantize: the float32 product (unsigned activation codes stored as
     c - 128, bias, GELU) and the next Linear's input step -- codes and {min, max, scale, zero
     point} -- bit for bit those of lq_gemm_w8a8 followed by lq_dynamic_quantize_f32.  The DMA
     kernels fold the extrema in their epilogue (256x128, 256x256 and ragged 128x128 tiles,
-    whose rows and columns past the edge must not count); a skinny M, more than 1024 tiles and
-    K % 128 != 0 take the separate calls."""
+    whose rows and columns past the edge must not count, with whole and partial last stages); a skinny
+    M, more than 1024 tiles and fewer than 128 take the separate calls.  Also with the workspace that
+    leaves out the aligned copies of a K that is no multiple of 16."""
     from lucid_amd import _C
 
     print(f"gemm dynamic quantize M={M} N={N} K={K} gelu={gelu}", flush=True)
@@ -466,16 +471,20 @@ def test_gemm_dynamic_quantize_equals_calls(gpu, M, N, K, gelu, want):
     _C.call("lq_dynamic_quantize_f32", y1.data_ptr(), M * N, _C.U8S8, 0, 255, eps, p1.data_ptr(), c1.data_ptr(),
             dws.data_ptr(), d_n, None)
     w_n = _C.lib().lq_gemm_w8a8_dynamic_quantize_workspace_size(M, N, K)
-    ws = gpu.empty((w_n,), np.uint8, "gpu")
-    _C.call("lq_gemm_w8a8_dynamic_quantize", dA.data_ptr(), K, dB.data_ptr(), K, y2.data_ptr(), M, N, K,
-            sa.data_ptr(), 0, sb.data_ptr(), 1, za.data_ptr(), None, sums.data_ptr(), bias.data_ptr(), flags,
-            _C.U8S8, 0, 255, eps, p2.data_ptr(), c2.data_ptr(), ws.data_ptr(), w_n, None)
-    assert _C.last_path() == want  # the separate calls end with lq_dynamic_quantize_f32's own path
-    np.testing.assert_array_equal(y1.numpy().view(np.uint32), y2.numpy().view(np.uint32))
-    np.testing.assert_array_equal(c1.numpy(), c2.numpy())
-    np.testing.assert_array_equal(p1.numpy().view(np.uint32), p2.numpy().view(np.uint32))
-    yv = y2.numpy()
-    np.testing.assert_array_equal(p2.numpy()[:2], np.array([yv.min(), yv.max()], np.float32))
+    sizes = [(w_n, want)]
+    if K % 16:  # less the copies' bytes: the product runs on the rows as they are
+        sizes.append((w_n - g_n + _C.lib().lq_gemm_w8a8_workspace_size(M, N, K // 16 * 16), "dynamic quantize two-launch"))
+    for n, path in sizes:
+        ws = gpu.empty((n,), np.uint8, "gpu")
+        _C.call("lq_gemm_w8a8_dynamic_quantize", dA.data_ptr(), K, dB.data_ptr(), K, y2.data_ptr(), M, N, K,
+                sa.data_ptr(), 0, sb.data_ptr(), 1, za.data_ptr(), None, sums.data_ptr(), bias.data_ptr(), flags,
+                _C.U8S8, 0, 255, eps, p2.data_ptr(), c2.data_ptr(), ws.data_ptr(), n, None)
+        assert _C.last_path() == path  # the separate calls end with lq_dynamic_quantize_f32's own path
+        np.testing.assert_array_equal(y1.numpy().view(np.uint32), y2.numpy().view(np.uint32))
+        np.testing.assert_array_equal(c1.numpy(), c2.numpy())
+        np.testing.assert_array_equal(p1.numpy().view(np.uint32), p2.numpy().view(np.uint32))
+        yv = y2.numpy()
+        np.testing.assert_array_equal(p2.numpy()[:2], np.array([yv.min(), yv.max()], np.float32))
 
 
 # K that is no multiple of 128 (a partial last stage of the LDS-DMA kernels, zeros past K) or of 16

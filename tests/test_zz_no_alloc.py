@@ -82,6 +82,23 @@ def test_noalloc_matches_workspace_entry_point(gpu, kind):
         np.testing.assert_array_equal(got.view(np.uint8), ref.view(np.uint8))
 
 
+def test_noalloc_aligned_copies(gpu):
+    """K no multiple of 16: the aligned copies of the operands lie in the scratch behind the code sums,
+    split partials and counters, where they fit (the second shape's do not: the generic kernel)."""
+    rng = np.random.default_rng(78)
+    for M, N, K, path in ((200, 300, 1001, "gemm dma 128x64"), (129, 9000, 2001, "gemm generic"), (40, 70, 333, "gemm skinny"),
+                          (130, 100, 32777, "gemm 128x128 split-k"), (200, 300, 1001, "gemm dma 128x64")):
+        A, B, sa, sb, za, zb, bias = _case(rng, M, N, K, True)
+        print(f"noalloc M={M} N={N} K={K}", flush=True)
+        want, p_ws = _run(gpu, "ws", A, B, O.OUT_Q8, sa, sb, za, zb, bias, 0.5, -2.0, True)
+        got, p_na = _run(gpu, "noalloc", A, B, O.OUT_Q8, sa, sb, za, zb, bias, 0.5, -2.0, True)
+        assert p_na == path and p_ws == ("gemm dma 128x128 3-stage" if path == "gemm generic" else path)
+        np.testing.assert_array_equal(got, want)
+        ref = O.gemm_w8a8(A, B, sa, sb, za=za, zb=zb, bias=bias, out_scale=0.5, out_zp=-2.0, qmin=-128, qmax=127,
+                          out_kind=O.OUT_Q8, relu=True)
+        np.testing.assert_array_equal(got, ref)
+
+
 def test_noalloc_refuses_shapes_beyond_its_scratch(gpu):
     from lucid_amd import _C
 
