@@ -13,23 +13,26 @@
 // piece of w_hat per step into LDS, in MFMA fragment order, while it multiplies the pieces of the step
 // before; the pieces after come from memory meanwhile.
 //
-// The terms of a value must be finite and, since these instructions read subnormal terms as 0, not far
-// below it.  A tile that meets an infinity, a scale that may make one, or eight values or a scale below
-// 2^-100 (but not 0) is computed again with v_mfma_f32_16x16x4_f32 on the float32 values themselves, through the
-// same stages: infinities, NaN and subnormals as a float32 sum has them (M = 2048, N = K = 4096 with an infinity in
-// every tile: 392 us for the terms, 1025 in all).  Beside larger ones of its eight, a smaller value is exact to 2^-126.
+// The terms of a value must be finite and, since these instructions read subnormal terms as 0, not
+// far below it.  A tile that meets an infinity, a scale that may make one, or eight values or a scale
+// below 2^-100 (but not 0) is computed again with v_mfma_f32_16x16x4_f32 on the float32 values
+// themselves, through the same stages: infinities, NaN and subnormals as a float32 sum has them
+// (M = 2048, N = K = 4096 with an infinity in every tile: 1025 us in all).  Beside larger ones of its
+// eight, a smaller value is exact to 2^-126.
 //
-// What bounds it: the issue of instructions and the waits around a step's barrier.  Per wave and step of the largest
-// tiles 96 MFMA (half x: 80) and 290 VALU: conversion to terms 11 per pair of values, one addition per
-// sum, three per weight code.  Tiles are as large as the shape allows: 256 x 128 in eight waves of 64 x 64,
-// 128 x 128 in waves of 64 x 32, 32 x 64 with the steps split between four groups of four waves.  N = K = 4096,
-// 4 bits, groups of 64, against the float32 VALU kernel before (128 x 128 tiles, 75 of at most 79
-// TFLOP/s without packed fp32): M = 2048 922 -> 392 us, M = 512 881 -> 229, M = 26 880 -> 64; half x
-// M = 2048 1323 -> 317.  The float32 matrix instructions alone took 595, 335 and 73 us.  Two fp16 terms per value
-// (three products, 312, 211 and 71 us) need a scale per row and tile, and lost values far below it.
-// The error against 64 bits at M = 2048 fell from 1.1e-6 to 2.3e-7: shorter chains of additions.  Ordering the
-// instructions by hand (3 VALU after each MFMA), conversions before the products in half of the waves and after
-// them in the others, or a higher priority for the products measured the same or slower.
+// What bounds it: the issue of instructions and the waits around a step's barrier (matrix cores busy
+// 38%, VALU 29% of the time; 1.13 PFLOP/s of bf16 products).  Per wave and step of the largest tiles 96
+// MFMA (half x: 80) and 290 VALU: conversion to terms 11 per pair of values, one addition per sum, three
+// per weight code.  Tiles are as large as the shape allows: 256 x 128 in eight waves of 64 x 64,
+// 128 x 128 in waves of 64 x 32, 32 x 64 with the steps split between four groups of four waves.
+// N = K = 4096, 4 bits, groups of 64, back to back, against the float32 VALU kernel before (128 x 128
+// tiles, 75 of at most 79 TFLOP/s without packed fp32): M = 2048 922 -> 392 us (364 with pauses between
+// calls), M = 512 881 -> 229, M = 26 880 -> 64; half x M = 2048 1323 -> 317.  The float32 matrix
+// instructions alone took 595, 335 and 73 us.  Two fp16 terms per value (three products, 312, 211 and
+// 71 us) need a scale per row and tile, and lost values far below it.  The error against 64 bits at
+// M = 2048 fell from 1.1e-6 to 2.3e-7: shorter chains of additions.  Ordering the instructions by hand
+// (3 VALU after each MFMA), conversions before the products in half of the waves and after them in the
+// others, or a higher priority for the products measured the same or slower.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

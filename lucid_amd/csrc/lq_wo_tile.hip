@@ -12,16 +12,16 @@
 //  * the group scales and biases, transposed by the same prepare launch, and the block sums ride
 //    along.  LDS holds everything in MFMA fragment order: reads and writes without bank conflicts.
 // Measured (float32 x, 8 bits, groups of 64, N = K = 4096; the GEMV kernels before): M = 64 34.5 ->
-// 23 us, M = 256 132 -> 40, M = 1024 504 -> 104 us = 330 TFLOP/s (two fp16 products each), M = 2048
-// 992 -> 205; half x, 4 bits, M = 1024 456 -> 88.  What bounds it now is the issue of instructions:
-// per wave and stage 32 MFMA (16 cycles each), 64 FMA of scales, 32 for unpacking, 26 LDS reads;
-// the matrix cores are busy about a third of the time.
+// 24 us, M = 1024 504 -> 114 us = 301 TFLOP/s (two fp16 products each), M = 2048 992 -> 240;
+// half x, 4 bits, M = 1024 456 -> 92.  What bounds it now is the issue of instructions and the waits around a
+// stage's barrier: per wave and stage 32 MFMA (16 cycles each), 96 multiplications and FMA of scales, 32 VALU for
+// unpacking, 26 LDS reads; the matrix cores are busy 23% of the time (half x 16%), the VALU 29%.
 // Arithmetic per 64-wide block (32 for groups of 32), that of the GEMV kernels: the block's values of a
 // row are scaled by 2^e (its largest into [2^14, 2^15)) before the split, blk = sum c (hi + lo) in fp32,
 // then acc += s (blk 2^-e) + b bsum.  2^-e goes to the scale, ahead of the products (after them, 137 us
-// instead of 126 at M = 1024, 8 bits, groups of 64): exact, unless 2^-e is so small that s 2^-e may not
-// be a normal number, so below 2^-90 the rest of it goes to blk.  One scale for the whole row instead took
-// 117 us, and lost bits of values far below the row's largest.
+// instead of 126 in calls back to back at M = 1024, 8 bits, groups of 64): exact, unless 2^-e is so small
+// that s 2^-e may not be a normal number, so below 2^-90 the rest of it goes to blk.  One scale for the
+// whole row instead took 117 us, and lost bits of values far below the row's largest.
 // Few tiles: K is split into ranges over workgroups, their sums added in range order by
 // wo_tile_reduce_kernel.  Without a workspace wo_tile_direct_kernel makes the same sums: the same bits.
 #include <hip/hip_runtime.h>
@@ -226,7 +226,8 @@ __global__ __launch_bounds__(256) void wo_tile_prep_kernel(WtArgs a, char* xp, f
         if (lane == 0) sh[0][wave].x = sum;
     }
     tiny = __syncthreads_or(tiny);
-    if (tid == 0) xr[m] = make_float2(GROUPED ? 0.0f : ((sh[0][0].x + sh[0][1].x) + sh[0][2].x) + sh[0][3].x, tiny ? 1.0f : 0.0f);
+    if (tid == 0)
+        xr[m] = make_float2(GROUPED ? 0.0f : ((sh[0][0].x + sh[0][1].x) + sh[0][2].x) + sh[0][3].x, tiny ? 1.0f : 0.0f);
 }
 
 // Tile of a workgroup: consecutive tiles (groups of eight tile rows, column by column) on one
@@ -473,7 +474,8 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
                 for (int i = 0; i < 4; ++i) {
                     if constexpr (GROUPED) {
                         const float sc = r.sb[n][i / 2][i % 2 * 2];
-                        acc[m][n][i] = wt_add(acc[m][n][i], blk[m][i], T == 2 ? sc * down : sc, r.sb[n][i / 2][i % 2 * 2 + 1], r.xf[m].x);
+                        acc[m][n][i] = wt_add(acc[m][n][i], blk[m][i], T == 2 ? sc * down : sc,
+                                              r.sb[n][i / 2][i % 2 * 2 + 1], r.xf[m].x);
                     } else {
                         acc[m][n][i] = wt_add<T>(acc[m][n][i], blk[m][i], r.xf[m].y);
                     }
@@ -533,14 +535,15 @@ __global__ __launch_bounds__(64 * WM * WN) void wo_tile_kernel(WtArgs a) {
 // ---- the same sums without a workspace
 //
 // The tiled kernel adds K / 512 or more groups of up to WT_FLUSH stages, first within a range, then the
-// ranges.  Here each wave makes whole groups of 32 rows x 16 FN columns, of activations that it splits itself,
-// straight from memory; GW waves share a row tile's groups, and the sums meet in LDS in that order.  Within a
-// group nothing waits for another wave.  FN = 4 splits x once for 64 columns, FN = 1 fills the chip where tiles are
-// few; GW = 2 keeps the waves busy where a row tile has few groups.
-// N = K = 4096, 8 bits, groups of 64, float32 x (the kernel for few rows, then the tiled kernel in its form that split x
-// in every workgroup, which this replaced): M = 33 40 and 126 -> 27 us, M = 128 106 and 131 -> 34, M = 1024
-// 822 and 285 -> 233; half x M = 33 25 and 117 -> 19; M = 2048, N = K = 1024 98 and 52 -> 35.  Only groups of 32 and per-channel weights at M = 1024 were
-// faster there (235 and 187 against 332 and 212).
+// ranges.  Here each wave makes whole groups of 32 rows x 16 FN columns, of activations that it splits
+// itself, straight from memory; GW waves share a row tile's groups, and the sums meet in LDS in that
+// order.  Within a group nothing waits for another wave.  FN = 4 splits x once for 64 columns, FN = 2 and 1
+// fill the chip where tiles are few; GW = 2 keeps the waves of a workgroup on the same weights, and busy
+// where a row tile has few groups.
+// N = K = 4096, 8 bits, groups of 64, float32 x (the kernel for few rows, and the tiled kernel in a form
+// that split x in every workgroup): M = 33 40 and 126 -> 27 us, M = 128 106 and 131 -> 34, M = 1024 822 and
+// 285 -> 233; half x M = 33 25 and 117 -> 19; M = 2048, N = K = 1024 98 and 52 -> 35.  That form was ahead
+// only for groups of 32 and per-channel weights at M = 1024 (235 against 332 us, 187 against 212).
 constexpr int WD_WAVES = 8, WD_FM = 2;
 
 template <int BITS, int S, int T, bool GROUPED, int HM, int FN, int GW>
@@ -548,7 +551,8 @@ __global__ __launch_bounds__(64 * WD_WAVES) void wo_tile_direct_kernel(WtArgs a)
     constexpr int NG = wt_blocks<S>(), FM = WD_FM, BM = 16 * FM, BN = 16 * FN, SLOTS = FM * FN * 64;
     constexpr int WB = S * BITS;  // weight bytes of a lane's part of a block
     constexpr bool XF32 = T == 2;
-    constexpr int RT = WD_WAVES / GW, ST = (SLOTS + 64 * GW - 1) / (64 * GW);  // row tiles, fours of outputs a finishing thread
+    constexpr int RT = WD_WAVES / GW;                       // row tiles of a workgroup
+    constexpr int ST = (SLOTS + 64 * GW - 1) / (64 * GW);  // fours of outputs that a thread finishes
     constexpr int GG = WT_FLUSH * (S == 2 ? 1 : 2);  // most group scales of a column in WT_FLUSH stages
     __shared__ f4 red[WD_WAVES][SLOTS];
     __shared__ float rows[RT * BM];
@@ -574,7 +578,8 @@ __global__ __launch_bounds__(64 * WD_WAVES) void wo_tile_direct_kernel(WtArgs a)
             const int g = i % GG, col = i / GG;
             if (g < ng) {
                 const int64_t at = (int64_t)min(n0 + col, c.N - 1) * a.G + g0 + g;
-                scales[wave][g * BN + col] = make_float2(round_to(c.w_scale[at], HM), c.g_bias ? round_to(c.g_bias[at], HM) : 0.0f);
+                scales[wave][g * BN + col] =
+                    make_float2(round_to(c.w_scale[at], HM), c.g_bias ? round_to(c.g_bias[at], HM) : 0.0f);
             }
         }
     };

@@ -365,7 +365,8 @@ def test_group_matmul_presplit_matches_inline(gpu, bits, gs):
 # and stages, K ranges and none
 WO_TILE_CASES = [(8, 0, 20, 4608, 4096), (8, 0, 64, 4099, 4096), (8, 0, 600, 1000, 1040), (8, 0, 1031, 515, 1040),
                  (8, 0, 2049, 2100, 272), (8, 64, 33, 4096, 4096), (8, 64, 1025, 2050, 512), (8, 128, 129, 2048, 2176),
-                 (8, 64, 1050, 4096, 1088), (8, 32, 300, 1900, 1056), (4, 32, 30, 4200, 4128), (4, 64, 700, 640, 2048), (4, 128, 2200, 2180, 384)]
+                 (8, 64, 1050, 4096, 1088), (8, 32, 300, 1900, 1056), (4, 32, 30, 4200, 4128),
+                 (4, 64, 700, 640, 2048), (4, 128, 2200, 2180, 384)]
 
 
 @pytest.mark.parametrize("half", [False, True])
@@ -442,8 +443,9 @@ def test_wo_tiles_unaligned_rows(gpu, M, N, K, gs, half):
 
     rng = np.random.default_rng(M + gs)
     x = rng.standard_normal((M, K)).astype(np.float16 if half else np.float32)
-    W, s = _t(gpu, rng.integers(-128, 128, (N, K)).astype(np.int8)), _t(gpu, rng.uniform(1e-3, 1e-1, (N, K // gs if gs else 1)).astype(np.float32))
-    b = _t(gpu, rng.standard_normal((N, K // gs if gs else 1)).astype(np.float32))
+    W, G = _t(gpu, rng.integers(-128, 128, (N, K)).astype(np.int8)), K // gs if gs else 1
+    s = _t(gpu, rng.uniform(1e-3, 1e-1, (N, G)).astype(np.float32))
+    b = _t(gpu, rng.standard_normal((N, G)).astype(np.float32))
     size = _C.lib().lq_group_matmul_workspace_size(M, N, K, gs) if gs else _C.lib().lq_gemv_w8_workspace_size(M, N, K)
     ws = gpu.empty((size,), np.uint8, "gpu")
     outs = []
@@ -461,8 +463,9 @@ def test_wo_tiles_unaligned_rows(gpu, M, N, K, gs, half):
                 _C.call("lq_gemv_w8", *args, K, s.data_ptr(), b.data_ptr(), None, y.data_ptr(), N, M, N, K, *end)
             assert _C.last_path().startswith("wo tiles")
             outs.append(y.numpy())
+    bits = np.uint16 if half else np.uint32
     for o in outs[1:]:
-        np.testing.assert_array_equal(o.view(np.uint16 if half else np.uint32), outs[0].view(np.uint16 if half else np.uint32))
+        np.testing.assert_array_equal(o.view(bits), outs[0].view(bits))
 
 
 @pytest.mark.parametrize("workspace", [True, False])
@@ -975,7 +978,8 @@ ONE, RANGES, SK, SK1 = "wo stream", "wo stream ranges", "wo packed split-k", "wo
 @pytest.mark.parametrize("M,N,K,path,half_path", [
     (1, 7, 64, ONE, ONE), (3, 17, 512, ONE, ONE), (8, 4112, 512, SK1, ONE), (16, 4112, 512, ONE, ONE), (3, 6200, 512, SK1, SK1),
     (16, 4100, 1040, ONE, ONE), (9, 8200, 2064, SK, ONE), (12, 6000, 4096, ONE, ONE), (16, 300, 4080, SK, SK),
-    (2, 48, 4112, SK, RANGES), (9, 8200, 4112, SK, SK), (2, 700, 5120, SK, RANGES), (3, 5400, 5120, RANGES, RANGES), (16, 4096, 8208, SK, RANGES), (16, 33, 8208, SK, SK), (16, 3400, 8192, RANGES, RANGES), (5, 2000, 11008, RANGES, RANGES)])
+    (2, 48, 4112, SK, RANGES), (9, 8200, 4112, SK, SK), (2, 700, 5120, SK, RANGES), (3, 5400, 5120, RANGES, RANGES),
+    (16, 4096, 8208, SK, RANGES), (16, 33, 8208, SK, SK), (16, 3400, 8192, RANGES, RANGES), (5, 2000, 11008, RANGES, RANGES)])
 def test_gemv_w8_packed_one_pass(gpu, M, N, K, path, half_path, half):
     from lucid_amd import _C
 
