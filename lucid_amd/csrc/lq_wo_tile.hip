@@ -561,12 +561,13 @@ __global__ __launch_bounds__(64 * WD_WAVES) void wo_tile_direct_kernel(WtArgs a)
     const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, l16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rt = wave / GW, gw = wave % GW;  // this wave's row tile, and which of its waves it is
-    const int m0 = (blockIdx.y * RT + rt) * BM, n0 = blockIdx.x * BN;
+    const int cols = (c.N + BN - 1) / BN, row0 = blockIdx.x / cols * RT * BM;  // consecutive workgroups share rows of x
+    const int m0 = row0 + rt * BM, n0 = blockIdx.x % cols * BN;
     const bool vec = x_vec<XF32>(c);
     const int row_bytes = c.K * BITS / 8;
     if (!GROUPED && c.w_zp) {
         for (int r = wave; r < RT * BM; r += WD_WAVES) {
-            const float sum = row_sum<XF32>(c, blockIdx.y * RT * BM + r, lane, vec);
+            const float sum = row_sum<XF32>(c, row0 + r, lane, vec);
             if (lane == 0) rows[r] = sum;
         }
     }
@@ -842,9 +843,9 @@ void wt_config(const WtPlan& p, WtArgs& a, bool inl, hipStream_t st) {
             // has up to four groups
             auto direct = [&](auto fn, auto gw) {
                 constexpr int FN = decltype(fn)::value, GW = decltype(gw)::value;
-                constexpr int BM = 16 * WD_FM * (WD_WAVES / GW);
-                hipLaunchKernelGGL((wo_tile_direct_kernel<BITS, S, T, GROUPED, HM, FN, GW>),
-                                   dim3((unsigned)((a.c.N + 16 * FN - 1) / (16 * FN)), (unsigned)((a.c.M + BM - 1) / BM)),
+                constexpr int BM = 16 * WD_FM * (WD_WAVES / GW), BN = 16 * FN;
+                const unsigned grid = (unsigned)((a.c.N + BN - 1) / BN) * (unsigned)((a.c.M + BM - 1) / BM);
+                hipLaunchKernelGGL((wo_tile_direct_kernel<BITS, S, T, GROUPED, HM, FN, GW>), dim3(grid),
                                    dim3(64 * WD_WAVES), 0, st, a);
             };
             using I1 = std::integral_constant<int, 1>;

@@ -468,6 +468,31 @@ def test_wo_tiles_unaligned_rows(gpu, M, N, K, gs, half):
         np.testing.assert_array_equal(o.view(bits), outs[0].view(bits))
 
 
+def test_wo_tiles_many_rows(gpu):
+    """More row tiles than a grid's second dimension holds, without a workspace and with one: the same
+    bits, and the first and last rows against float64."""
+    from lucid_amd import _C
+
+    rng = np.random.default_rng(9)
+    M, N, K = 65536 * 32 + 70, 8, 64
+    x = np.tile(rng.standard_normal((M // 64 + 1, K)).astype(np.float16), (64, 1))[:M]
+    W = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    s = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    xd, wd, sd = _t(gpu, x), _t(gpu, W), _t(gpu, s)
+    size = _C.lib().lq_gemv_w8_workspace_size(M, N, K)
+    ws = gpu.empty((size,), np.uint8, "gpu")
+    outs = []
+    for n, path in ((size, "wo tiles"), (0, "wo tiles inline")):
+        y = gpu.empty((M, N), np.float16, "gpu")
+        _C.call("lq_gemv_w8", xd.data_ptr(), _C.F16, K, wd.data_ptr(), K, sd.data_ptr(), None, None, y.data_ptr(), N, M, N, K,
+                0, ws.data_ptr() if n else None, n, None)
+        assert _C.last_path() == path
+        outs.append(y.numpy())
+    np.testing.assert_array_equal(outs[0], outs[1])
+    rows = np.r_[0:100, M - 100:M]
+    _close(outs[1][rows], _gemv_ref(x[rows].astype(np.float32), W, s), half=True)
+
+
 @pytest.mark.parametrize("workspace", [True, False])
 @pytest.mark.parametrize("bits,gs", [(8, 0), (8, 64), (4, 64), (8, 32), (4, 128)])
 @pytest.mark.parametrize("M,N,K", [(40, 5504, 2048), (200, 2048, 2112)])
