@@ -1,8 +1,9 @@
 """GPU parity of the W8A8 int8 MFMA GEMM (lq_gemm_w8a8) through the C ABI.
 
 * int32 accumulators: bit-exact against the oracle's int64 brute force on every kernel
-  path (skinny M <= 64; LDS-DMA 256x256, 256x128 and 128x128 tiles; register-staged 128x128 tiles
-  with and without split-K; generic);
+  path (skinny M <= 128; LDS-DMA 256x256, 256x128, 128x128 and 128x64 tiles with whole and partial
+  last stages; register-staged 128x128 tiles with and without split-K; operands copied to aligned
+  rows; generic);
 * every epilogue kind (f32, f16, requantized int8 / uint8 / int16 / uint8-as-int8,
   fake-quantized f32) with activation and weight zero points, bias and ReLU: bit-exact
   against the oracle's epilogue (same op order, no FMA);
@@ -113,9 +114,9 @@ def _codes(rng, shape, lo=-127, hi=127):
 
 
 # Shapes chosen to hit every dispatch path of the kernel selector:
-#   M <= 16 / 32 / 64 -> skinny (1, 2, 4 m-tiles); K % 128 == 0 with enough tiles -> LDS-DMA
-#   256x256 / 256x128 / 128x128; otherwise register-staged 128x128 (split-K when tiles are few);
-#   K % 16 != 0 or unaligned -> generic.
+#   M <= 16 / 32 / 64 / 128 -> skinny (1, 2, 4, 8 m-tiles); more rows -> LDS-DMA 256x256 / 256x128 /
+#   128x128 / 128x64, with a partial last stage where K % 128 != 0; a K no multiple of 16 -> copied to
+#   aligned rows first, or, where it is short, generic.
 ACC_SHAPES = [
     (1, 64, 64), (1, 1000, 784), (3, 4096, 512), (16, 256, 4096), (17, 100, 256),
     (32, 48, 1024), (33, 160, 640), (64, 10, 256), (64, 256, 784), (65, 130, 96),
@@ -136,7 +137,7 @@ def test_int32_accumulator_exact(gpu, M, N, K):
 
 
 def test_int32_accumulator_staged_many_tiles(gpu):
-    """Many tiles with K % 128 != 0 (register-staged path) and ragged M, N and K."""
+    """Many tiles with K % 128 != 0 (a partial last stage) and ragged M, N and K."""
     rng = np.random.default_rng(5)
     M, N, K = 2000, 6400, 400
     A = _codes(rng, (M, K))
@@ -273,6 +274,41 @@ def test_epilogue_kinds_exact(gpu, M, N, K, kind):
             np.testing.assert_array_equal(got.view(np.uint16), want.view(np.uint16))
         else:
             np.testing.assert_array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("K,path", [(208, "gemm 128x128"), (2064, "gemm 128x128 split-k")])
+def test_epilogue_kinds_register_staged(gpu, K, path):
+    """The register-staged 128x128 tiles, without and with K splits, every output kind: rows so far
+    apart that the LDS-DMA copies' 32-bit offsets cannot span them (64-bit addresses here)."""
+    from lucid_amd import _C
+
+    rng = np.random.default_rng(K)
+    M, N, lda = 200, 300, 4_750_000
+    A, B = _codes(rng, (M, K), -128, 127), _codes(rng, (N, K), -127, 127)
+    dA = gpu.empty(((M - 1) * lda + K,), np.int8, "gpu")
+    for r in range(M):
+        row = np.ascontiguousarray(A[r])
+        _C.call("lq_memcpy_h2d", dA.data_ptr() + r * lda, row.ctypes.data, K, None)
+        gpu.synchronize()
+    dB = _dev(gpu, B)
+    sa, sb = rng.uniform(1e-3, 1e-1, M).astype(np.float32), rng.uniform(1e-3, 1e-1, N).astype(np.float32)
+    zb, bias = rng.integers(-4, 5, N).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    dev = [_dev(gpu, np.atleast_1d(np.asarray(v, np.float32))) for v in (sa, sb, 3.0, zb, bias, 0.37)]
+    n = _C.lib().lq_gemm_w8a8_workspace_size(M, N, K)
+    ws = gpu.empty((n,), np.uint8, "gpu")
+    for kind in KINDS:
+        qmin, qmax = GRID.get(kind, (-128, 127))
+        out_zp = 128.0 if qmin == 0 else -3.0
+        zp = _dev(gpu, np.array([out_zp], np.float32))
+        C = gpu.empty((M, N), _OUT_DT[kind], "gpu")
+        print(f"gemm register-staged K={K} kind={kind}", flush=True)
+        _C.call("lq_gemm_w8a8", dA.data_ptr(), lda, dB.data_ptr(), K, C.data_ptr(), N, M, N, K, dev[0].data_ptr(), 1,
+                dev[1].data_ptr(), 1, dev[2].data_ptr(), dev[3].data_ptr(), None, dev[4].data_ptr(), dev[5].data_ptr(),
+                zp.data_ptr(), qmin, qmax, kind, _C.EPI_RELU, ws.data_ptr(), n, None)
+        assert _C.last_path() == path
+        want = O.gemm_w8a8(A, B, sa, sb, za=3.0, zb=zb, bias=bias, out_scale=0.37, out_zp=out_zp, qmin=qmin, qmax=qmax,
+                           out_kind=kind, relu=True)
+        np.testing.assert_array_equal(C.numpy().view(np.uint8), want.view(np.uint8))
 
 
 def test_cached_weight_sums_and_scalar_scales(gpu):
